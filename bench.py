@@ -548,12 +548,15 @@ def main():
     value = samples / dt / 1e6
     segs = totals["segments"]
     paths = totals["paths"]
-    # the bounce-loop kernels' share: the last paths of each pass are traced and
-    # shaded by the fused tail launch (k_tail), timed apart
+    # the bounce-loop kernels' share: what the fused launches trace and shade is timed apart
     loop_segs = segs - totals["tail_segments"]
     trace_bytes = TRACE_BYTES_PER_SEGMENT * loop_segs
     shade_bytes = SHADE_BYTES_PER_SEGMENT * loop_segs + ACCUM_BYTES_PER_PATH * paths
-    if totals["trace_ms"] >= totals["shade_ms"]:
+    if totals["tail_ms"] >= max(totals["trace_ms"], totals["shade_ms"]):
+        # the whole render in fused path launches: 12 B written per sample, and
+        # read and summed once per pass
+        kname, kbytes, kms, nl = "k_paths", 12 * paths, totals["tail_ms"], totals["tail_launches"]
+    elif totals["trace_ms"] >= totals["shade_ms"]:
         kname, kbytes, kms, nl = "k_trace", trace_bytes, totals["trace_ms"], totals["trace_launches"]
     else:
         kname, kbytes, kms, nl = "k_shade", shade_bytes, totals["shade_ms"], totals["shade_launches"]

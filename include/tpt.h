@@ -345,11 +345,13 @@ typedef struct tpt_render_desc {
  * override material::scatter (headers/material.h:74-80), so a path that the
  * medium stops ends there, black. */
 #define TPT_RENDER_MEDIA_SCATTER 2u
-/* flags: drain every pass with trace / shade launches only.  By default, once
- * a pass has handed out all its work and few paths are left, one fused launch
- * (k_tail) carries those paths through their remaining bounces (scenes with
+/* flags: render with trace / shade launches only.  By default, for scenes with
  * constant textures, at most one rect light, no motion or media, on the
- * small-scene or sphere-only walk); every sample is the same bit for bit. */
+ * small-scene or sphere-only walk, fused launches carry paths through their
+ * bounces: a plain render takes one launch per pass for all of them (k_paths;
+ * it keeps no path queues, so queue_capacity, blocks_per_cu and graph_iters
+ * have no effect on it), a guided one ends each pass with one (k_tail).  Every
+ * sample is the same bit for bit. */
 #define TPT_RENDER_NO_TAIL 4u
 /* flags: count the closest-hit walk's operations by kind (box_tests,
  * sphere_tests, rect_tests, xforms of tpt_render_stats), for the counted VALU
@@ -366,8 +368,8 @@ typedef struct tpt_render_stats {
   uint64_t nodes_visited;  /* pre-order slots visited by closest-hit queries */
   double trace_ms, shade_ms;          /* with TPT_RENDER_PROFILE */
   uint64_t trace_launches, shade_launches;
-  uint64_t tail_segments;  /* segments traced by the fused tail launches (included in segments) */
-  double tail_ms;          /* with TPT_RENDER_PROFILE: time of the fused tail launches */
+  uint64_t tail_segments;  /* segments traced by the fused launches (included in segments) */
+  double tail_ms;          /* with TPT_RENDER_PROFILE: time of the fused launches */
   uint64_t tail_launches;
   /* with TPT_RENDER_COUNT_OPS (else 0): slab tests, sphere tests, rect tests
    * and wrapper chains (translate / rotate_y) applied by the closest-hit walks */

@@ -1,0 +1,68 @@
+"""Plain renders in one path launch per pass (k_paths) against the bounce loop.
+
+By default a plain render of a scene with constant textures and at most one
+rect light carries every path through all its bounces in one launch; with
+tail=False (TPT_RENDER_NO_TAIL) the bounce loop renders it.  Same functions,
+same Philox streams, samples summed in the same order: the sums must be equal
+bit for bit and the counts the same, at sizes around a wave's 64 rays, the 64
+work shards and a block's 256 threads.
+"""
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+COUNTS = ("paths", "segments", "light_queries", "nodes_visited", "nan_samples")
+
+
+@pytest.mark.parametrize("name", ["cornell555", "random_spheres", "random_spheres_n3000"])
+@pytest.mark.parametrize("w,h,spp,depth,offset", [
+    (1, 1, 1, 50, 0),        # one path
+    (9, 7, 1, 50, 3),        # 63 items: one short run of rays
+    (13, 5, 1, 1, 0),        # 65 items, paths cut at depth 1
+    (257, 1, 3, 0, 0),       # depth 0: every hit ends its path
+    (61, 67, 5, 50, 2),      # ragged: 20435 items over 64 shards
+    (320, 200, 9, 50, 1000),  # more items than lanes in flight
+])
+def test_paths_equal_bounce_loop(tpt, device, name, w, h, spp, depth, offset):
+    import torch
+
+    sc = tpt.Scene.named(name)
+    i = sc.host.info
+    cam = tpt.camera_make(tuple(i.lookfrom), tuple(i.lookat), (0.0, 1.0, 0.0), i.vfov, w / h, i.aperture, i.focus)
+    kw = dict(width=w, height=h, spp=spp, seed=5, sample_offset=offset, max_depth=depth, camera=cam)
+    a, qa, sa = sc.render(**kw)
+    b, qb, sb = sc.render(tail=False, **kw)
+    assert torch.equal(a, b) and torch.equal(qa, qb)
+    for k in COUNTS:
+        assert sa[k] == sb[k], k
+    assert sa["paths"] == w * h * spp
+    assert sa["tail_launches"] == 1 and sa["tail_segments"] == sa["segments"]
+    assert sb["tail_launches"] == 0
+
+
+def test_paths_pooled_jobs_equal_bounce_loop(tpt, device):
+    """Jobs of several scenes and sizes in one launch, sums without squares among them."""
+    import torch
+
+    hosts = [tpt.HostScene(f"random_spheres_n{n}", seed=k + 1) for k, n in enumerate((60, 900, 90, 2500, 300))]
+    pool = tpt.Scene.pool(hosts)
+
+    def run(flags):
+        jobs, bufs = [], []
+        for k, (w, h, spp) in enumerate(((3, 1, 1), (64, 48, 5), (17, 33, 2), (80, 31, 3), (1, 65, 7))):
+            j, s, q = pool.job(scene=k, width=w, height=h, spp=spp, seed=40 + k, max_depth=50,
+                               sumsq_buf=False if k == 2 else None)
+            jobs.append(j)
+            bufs.append(s)
+            if k != 2:
+                bufs.append(q)
+        L = tpt.Launch()
+        L.flags = flags
+        return bufs, pool.render_jobs(jobs, launch=L)
+
+    (ba, sa), (bb, sb) = run(0), run(4)
+    for x, y in zip(ba, bb):
+        assert torch.equal(x, y)
+    for k in COUNTS:
+        assert sa[k] == sb[k], k
+    assert sa["tail_launches"] == 1 and sb["tail_launches"] == 0

@@ -12,6 +12,7 @@
 
 #include "../host/errors.h"
 #include "guide_train.h"
+#include "paths.h"
 #include "render.h"
 
 #include <random>
@@ -134,6 +135,10 @@ struct tpt_scene {
   pass_hdr *d_hdr = nullptr, *h_hdr = nullptr;
   pass_ent *d_pass = nullptr, *h_pass = nullptr;
   uint32_t pass_cap = 0;
+  // render in one launch per pass (k_paths): its tables and counters
+  char *tables = nullptr, *h_tables = nullptr;  // device, pinned
+  size_t tables_bytes = 0;
+  hipEvent_t ev_begin = nullptr, ev_end = nullptr;
   // captured bounce loop (hipGraph), replayed in every pass of a render call
   hipStream_t gstream = nullptr;
   hipEvent_t ev_in = nullptr, ev_out = nullptr;
@@ -192,6 +197,10 @@ void free_scene(tpt_scene *s) {
   (void)hipFree(s->d_jobs);
   (void)hipFree(s->d_hdr);
   (void)hipFree(s->d_pass);
+  (void)hipFree(s->tables);
+  if (s->h_tables) (void)hipHostFree(s->h_tables);
+  if (s->ev_begin) (void)hipEventDestroy(s->ev_begin);
+  if (s->ev_end) (void)hipEventDestroy(s->ev_end);
   if (s->h_hdr) (void)hipHostFree(s->h_hdr);
   if (s->h_pass) (void)hipHostFree(s->h_pass);
   for (auto e : s->events) (void)hipEventDestroy(e);
@@ -211,6 +220,7 @@ void free_scene(tpt_scene *s) {
 // up to at most `capacity`.  G2 = 0: no guided shading (plain renders), only
 // G1 kernels append.
 size_t region_size(uint32_t capacity, uint32_t g1, uint32_t g2) {
+  if (!capacity) return 0;  // no queues (k_paths)
   const size_t r1 = (g1 + NSUB - 1) / NSUB, r2 = (g2 + NSUB - 1) / NSUB;
   return capacity / NSUB + capacity / g1 + (g2 ? capacity / g2 : 0) + r1 * 256 + r2 * 512 + 256;
 }
@@ -765,6 +775,19 @@ void launch_tail(const bounce_launch &B, hipStream_t st, uint32_t parity, uint32
   }
 }
 
+// Blocks per CU of k_paths (its occupancy target is in waves per SIMD, one block of 4 waves each).
+uint32_t path_blocks_per_cu(const bounce_launch &) { return 4; }
+
+void launch_paths(const bounce_launch &B, hipStream_t st, uint32_t grid) {
+  const dim3 g(grid), b(PATH_THREADS);
+  if (B.sweep)
+    hipLaunchKernelGGL((k_paths<true, false>), g, b, 0, st, B.S, B.S.slots, B.S.entries, B.P, B.Q);
+  else if (B.multi)
+    hipLaunchKernelGGL((k_paths<false, true>), g, b, 0, st, B.S, B.S.slots, B.S.entries, B.P, B.Q);
+  else
+    hipLaunchKernelGGL((k_paths<false, false>), g, b, 0, st, B.S, B.S.slots, B.S.entries, B.P, B.Q);
+}
+
 template <bool COUNT>
 void launch_trace_t(const bounce_launch &B, hipStream_t st, uint32_t parity) {
   const dim3 g(B.grid), b(TRACE_THREADS);
@@ -826,6 +849,124 @@ void launch_shade(const bounce_launch &B, hipStream_t st, uint32_t parity) {
   }
 }
 
+// Column sums of `rows` per-block statistics rows into out[0..ST_COUNT).
+__global__ void __launch_bounds__(256) k_stats_total(const unsigned long long *stats, uint32_t rows,
+                                                       unsigned long long *out) {
+  __shared__ unsigned long long part[256];
+  constexpr uint32_t kLanes = 256 / ST_COUNT;  // partial sums per counter
+  const uint32_t k = threadIdx.x % ST_COUNT, lane = threadIdx.x / ST_COUNT;
+  unsigned long long v = 0;
+  for (uint32_t r = lane; r < rows; r += kLanes) v += stats[static_cast<size_t>(r) * ST_COUNT + k];
+  part[threadIdx.x] = v;
+  __syncthreads();
+  if (threadIdx.x < ST_COUNT) {
+    unsigned long long t = 0;
+    for (uint32_t l = 0; l < kLanes; ++l) t += part[l * ST_COUNT + threadIdx.x];
+    out[threadIdx.x] = t;
+  }
+}
+
+// Items of a pass of k_paths.  Its drain costs about a path's longest chain of
+// bounces (0.1-0.2 ms); 2^28 items take about 30 ms or more and hold 3.2 GB of results.
+constexpr uint64_t kPassItemsPaths = 1ull << 28;
+
+// The plain render of scenes that k_paths takes, `plan` in passes of at most
+// kPassItemsPaths items: one path launch and one accumulation per pass, and no
+// host synchronisation before the end.
+int render_paths(tpt_scene *s, const std::vector<job_dev> &jd, const std::vector<pass_plan> &plan, bounce_launch B,
+                 bool profile, tpt_render_stats *stats, hipStream_t ws) {
+  const uint32_t n_jobs = static_cast<uint32_t>(jd.size());
+  uint32_t max_items = 0;
+  size_t n_ent = 0;
+  for (const auto &pp : plan) {
+    max_items = std::max(max_items, pp.n_items);
+    n_ent += pp.ents.size();
+  }
+  const uint32_t full = static_cast<uint32_t>(s->n_cu) * path_blocks_per_cu(B);
+  const uint32_t grid = std::min<uint32_t>(full, (max_items + PATH_THREADS - 1) / PATH_THREADS);
+  int rc = ensure_state(s, 0, max_items, full, 0);
+  if (rc != TPT_OK) return rc;
+  B.Q = s->Q;
+  // one blob: jobs, pass headers, pass tables, then (device only) the stats totals
+  const auto up = [](size_t n) { return (n + 255) & ~size_t(255); };
+  const size_t at_hdr = up(n_jobs * sizeof(job_dev)), at_ent = at_hdr + up(plan.size() * sizeof(pass_hdr)),
+               at_tot = at_ent + up(n_ent * sizeof(pass_ent)), bytes = at_tot + 256;
+  static_assert(ST_COUNT * sizeof(unsigned long long) <= 256, "totals");
+  if (bytes > s->tables_bytes) {
+    (void)hipFree(s->tables);
+    if (s->h_tables) (void)hipHostFree(s->h_tables);
+    s->tables = s->h_tables = nullptr;
+    s->tables_bytes = 0;
+    HIP_TRY(hipMalloc(&s->tables, bytes));
+    HIP_TRY(hipHostMalloc(reinterpret_cast<void **>(&s->h_tables), bytes, hipHostMallocDefault));
+    s->tables_bytes = bytes;
+  }
+  if (!s->ev_begin) HIP_TRY(hipEventCreate(&s->ev_begin));
+  if (!s->ev_end) HIP_TRY(hipEventCreate(&s->ev_end));
+  std::memcpy(s->h_tables, jd.data(), n_jobs * sizeof(job_dev));
+  size_t e0 = 0;
+  for (size_t k = 0; k < plan.size(); ++k) {
+    const pass_hdr h{plan[k].n_items, 0, static_cast<uint32_t>(plan[k].ents.size()), plan[k].n_acc};
+    std::memcpy(s->h_tables + at_hdr + k * sizeof(pass_hdr), &h, sizeof(h));
+    std::memcpy(s->h_tables + at_ent + e0 * sizeof(pass_ent), plan[k].ents.data(), plan[k].ents.size() * sizeof(pass_ent));
+    e0 += plan[k].ents.size();
+  }
+  HIP_TRY(hipEventRecord(s->ev_begin, ws));
+  HIP_TRY(hipMemcpyAsync(s->tables, s->h_tables, at_tot, hipMemcpyHostToDevice, ws));
+  hipLaunchKernelGGL(k_zero_stats, dim3(64), dim3(256), 0, ws, s->Q.stats, grid * ST_COUNT);
+  B.P.jobs = reinterpret_cast<const job_dev *>(s->tables);
+  double path_ms = 0.0;
+  e0 = 0;
+  for (size_t k = 0; k < plan.size(); ++k) {
+    B.P.hdr = reinterpret_cast<const pass_hdr *>(s->tables + at_hdr) + k;
+    B.P.pass = reinterpret_cast<const pass_ent *>(s->tables + at_ent) + e0;
+    e0 += plan[k].ents.size();
+    hipLaunchKernelGGL(k_init, dim3((COUNTER_WORDS / CSTRIDE + 255) / 256), dim3(256), 0, ws, B.P, B.Q);
+    if (profile) {
+      while (s->events.size() < 2) {
+        hipEvent_t e;
+        HIP_TRY(hipEventCreate(&e));
+        s->events.push_back(e);
+      }
+      HIP_TRY(hipEventRecord(s->events[0], ws));
+    }
+    launch_paths(B, ws, grid);
+    if (profile) {
+      HIP_TRY(hipEventRecord(s->events[1], ws));
+      HIP_TRY(hipEventSynchronize(s->events[1]));
+      float a = 0.0f;
+      if (hipEventElapsedTime(&a, s->events[0], s->events[1]) == hipSuccess) path_ms += a;
+    }
+    const dim3 ag(std::min<uint32_t>((plan[k].n_acc + 255) / 256, static_cast<uint32_t>(s->n_cu) * 64u));
+    if (B.multi)
+      hipLaunchKernelGGL(k_accumulate<true>, ag, dim3(256), 0, ws, B.P, static_cast<const float *>(s->Q.res));
+    else
+      hipLaunchKernelGGL(k_accumulate<false>, ag, dim3(256), 0, ws, B.P, static_cast<const float *>(s->Q.res));
+  }
+  unsigned long long *tot = reinterpret_cast<unsigned long long *>(s->tables + at_tot);
+  hipLaunchKernelGGL(k_stats_total, dim3(1), dim3(256), 0, ws, static_cast<const unsigned long long *>(s->Q.stats),
+                     grid, tot);
+  HIP_TRY(hipGetLastError());
+  HIP_TRY(hipEventRecord(s->ev_end, ws));
+  HIP_TRY(hipMemcpyAsync(s->h_tables + at_tot, tot, ST_COUNT * sizeof(*tot), hipMemcpyDeviceToHost, ws));
+  HIP_TRY(hipStreamSynchronize(ws));
+  if (stats) {
+    unsigned long long t[ST_COUNT];
+    std::memcpy(t, s->h_tables + at_tot, sizeof(t));
+    float ms = 0.0f;
+    (void)hipEventElapsedTime(&ms, s->ev_begin, s->ev_end);
+    stats->paths = t[ST_PATHS];
+    stats->segments = stats->tail_segments = t[ST_SEGMENTS];
+    stats->light_queries = t[ST_LIGHT];
+    stats->nan_samples = t[ST_NAN];
+    stats->nodes_visited = t[ST_NODES];
+    stats->kernel_ms = ms;
+    stats->tail_ms = path_ms;
+    stats->tail_launches = plan.size();
+  }
+  return TPT_OK;
+}
+
 // Renders every job; the render loop described in render.h.
 int render_core(tpt_scene *s, const tpt_job *jobs, uint32_t n_jobs, const tpt_launch &L, tpt_guide *guide,
                 tpt_render_stats *stats, void *stream_ptr) {
@@ -875,6 +1016,27 @@ int render_core(tpt_scene *s, const tpt_job *jobs, uint32_t n_jobs, const tpt_la
     d.sum = J.d_sum;
     d.sumsq = J.d_sumsq;
   }
+  bounce_launch B;
+  std::memset(&B, 0, sizeof(B));  // the captured-graph key compares its bytes
+  B.S = multi ? s->pool_view() : s->view(jobs[0].scene);
+  B.sweep = !multi && s->sweep[jobs[0].scene];
+  B.sph = true;
+  B.simple = true;
+  for (uint32_t j = 0; j < n_jobs; ++j) {
+    B.sph = B.sph && s->sph[jobs[j].scene];
+    B.simple = B.simple && s->simple[jobs[j].scene];
+    if (s->motion[jobs[j].scene]) B.P.motion = 1;
+    if (s->media[jobs[j].scene]) B.P.media = 1;
+  }
+  B.multi = multi;
+  B.guided = guide != nullptr;
+  B.count = (L.flags & TPT_RENDER_COUNT_OPS) != 0;
+  B.tail = !(L.flags & TPT_RENDER_NO_TAIL) && !B.count && B.simple && (B.sweep || B.sph);
+  B.P.scenes = s->d_scenes;
+  B.P.guide_verts = ~0u;
+  B.P.media_scatter = (L.flags & TPT_RENDER_MEDIA_SCATTER) ? 1u : 0u;
+  if (B.tail && !guide)
+    return render_paths(s, jd, plan_passes(jobs, n_jobs, kPassItemsPaths), B, profile, stats, cs);
   const std::vector<pass_plan> plan =
       plan_passes(jobs, n_jobs, guide && L.guiding ? kPassItemsRecording : kPassItems);
   uint32_t max_items = 0, max_ent = 0;
@@ -930,14 +1092,13 @@ int render_core(tpt_scene *s, const tpt_job *jobs, uint32_t n_jobs, const tpt_la
   // (passes of 2^30 items) 3538 / 3613 / 3667, its guided frame (one pass of
   // 368M items) 2669 / 2689 / 2718, the textured spheres' 1600^2 frame (one
   // pass of 768M items, per-lane walks) 1736 / 1724 / 1672.
-  const bool sweep_scene = !multi && s->sweep[jobs[0].scene];
-  uint32_t cap = L.queue_capacity;
+    uint32_t cap = L.queue_capacity;
   if (!cap) {
     size_t free_b = 0, total_b = 0;
     if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) free_b = 0;
     const size_t budget = (free_b + s->state_bytes) / 10 * 7;
     cap = 1u << 29;
-    while (!sweep_scene && cap > (1u << 27) && static_cast<uint64_t>(cap) * 2 > max_items) cap >>= 1;
+    while (!B.sweep && cap > (1u << 27) && static_cast<uint64_t>(cap) * 2 > max_items) cap >>= 1;
     while (cap > (1u << 20) &&
            state_bytes_for(std::min(cap, max_items), max_items, grid, state_guide_grid) > budget)
       cap >>= 1;
@@ -945,32 +1106,13 @@ int render_core(tpt_scene *s, const tpt_job *jobs, uint32_t n_jobs, const tpt_la
   cap = std::min(cap, max_items);
   if ((rc = ensure_state(s, cap, max_items, grid, state_guide_grid)) != TPT_OK) return rc;
 
-  bounce_launch B;
-  std::memset(&B, 0, sizeof(B));  // the captured-graph key compares its bytes
-  B.S = multi ? s->pool_view() : s->view(jobs[0].scene);
   B.Q = s->Q;
   B.grid = grid;
   B.guide_grid = guide_grid;
-  B.sweep = sweep_scene;
-  B.sph = true;
-  B.simple = true;
-  for (uint32_t j = 0; j < n_jobs; ++j) {
-    B.sph = B.sph && s->sph[jobs[j].scene];
-    B.simple = B.simple && s->simple[jobs[j].scene];
-    if (s->motion[jobs[j].scene]) B.P.motion = 1;
-    if (s->media[jobs[j].scene]) B.P.media = 1;
-  }
-  B.multi = multi;
-  B.guided = guide != nullptr;
-  B.count = (L.flags & TPT_RENDER_COUNT_OPS) != 0;
-  B.tail = !(L.flags & TPT_RENDER_NO_TAIL) && !B.count && B.simple && (B.sweep || B.sph);
   render_params &P = B.P;
   P.jobs = s->d_jobs;
-  P.scenes = s->d_scenes;
   P.hdr = s->d_hdr;
   P.pass = s->d_pass;
-  P.guide_verts = ~0u;
-  P.media_scatter = (L.flags & TPT_RENDER_MEDIA_SCATTER) ? 1u : 0u;
   if (guide) {
     P.g_tiles = guide->xtiles;
     P.g_params = guide->params;
@@ -1279,23 +1421,6 @@ __global__ void k_noalloc_pass(job_dev *jobs, job_dev job, pass_hdr *hdr, pass_h
   }
 }
 
-// Column sums of `rows` per-block statistics rows into out[0..ST_COUNT).
-__global__ void __launch_bounds__(256) k_noalloc_stats(const unsigned long long *stats, uint32_t rows,
-                                                       unsigned long long *out) {
-  __shared__ unsigned long long part[256];
-  constexpr uint32_t kLanes = 256 / ST_COUNT;  // partial sums per counter
-  const uint32_t k = threadIdx.x % ST_COUNT, lane = threadIdx.x / ST_COUNT;
-  unsigned long long v = 0;
-  for (uint32_t r = lane; r < rows; r += kLanes) v += stats[static_cast<size_t>(r) * ST_COUNT + k];
-  part[threadIdx.x] = v;
-  __syncthreads();
-  if (threadIdx.x < ST_COUNT) {
-    unsigned long long t = 0;
-    for (uint32_t l = 0; l < kLanes; ++l) t += part[l * ST_COUNT + threadIdx.x];
-    out[threadIdx.x] = t;
-  }
-}
-
 // Grid of the no-allocation render: 4 blocks of 256 per CU, at most 1024
 // blocks (the statistics rows and the region bound are sized for that), at
 // least NSUB (the fused tail launches at least NSUB blocks).
@@ -1485,7 +1610,7 @@ int render_noalloc(tpt_scene *s, const tpt_camera *camera, const tpt_render_desc
                        P, static_cast<const float *>(Q.res));
     s0 += take;
   }
-  hipLaunchKernelGGL(k_noalloc_stats, dim3(1), dim3(256), 0, ws, static_cast<const unsigned long long *>(Q.stats),
+  hipLaunchKernelGGL(k_stats_total, dim3(1), dim3(256), 0, ws, static_cast<const unsigned long long *>(Q.stats),
                      grid, d_totals);
   HIP_TRY(hipGetLastError());
   // the totals come back through the scene's pinned count buffer (8 KB)
