@@ -345,12 +345,12 @@ typedef struct tpt_render_desc {
  * override material::scatter (headers/material.h:74-80), so a path that the
  * medium stops ends there, black. */
 #define TPT_RENDER_MEDIA_SCATTER 2u
-/* flags: render with trace / shade launches only.  By default, for scenes with
+/* flags: render with trace / shade launches only.  By default a plain render
+ * takes one launch per pass that carries every path through all its bounces
+ * (k_paths; it keeps no path queues, so queue_capacity, blocks_per_cu and
+ * graph_iters have no effect on it), and a guided render of a scene with
  * constant textures, at most one rect light, no motion or media, on the
- * small-scene or sphere-only walk, fused launches carry paths through their
- * bounces: a plain render takes one launch per pass for all of them (k_paths;
- * it keeps no path queues, so queue_capacity, blocks_per_cu and graph_iters
- * have no effect on it), a guided one ends each pass with one (k_tail).  Every
+ * small-scene or sphere-only walk, ends each pass with one (k_tail).  Every
  * sample is the same bit for bit. */
 #define TPT_RENDER_NO_TAIL 4u
 /* flags: count the closest-hit walk's operations by kind (box_tests,
@@ -368,8 +368,12 @@ typedef struct tpt_render_stats {
   uint64_t nodes_visited;  /* pre-order slots visited by closest-hit queries */
   double trace_ms, shade_ms;          /* with TPT_RENDER_PROFILE */
   uint64_t trace_launches, shade_launches;
-  uint64_t tail_segments;  /* segments traced by the fused launches (included in segments) */
-  double tail_ms;          /* with TPT_RENDER_PROFILE: time of the fused launches */
+  /* the fused launches of the scenes that k_tail takes (k_tail and, for plain
+     renders, k_paths): their segments (included in segments), time (with
+     TPT_RENDER_PROFILE) and number; other scenes' path launches are counted in
+     trace_ms and trace_launches */
+  uint64_t tail_segments;
+  double tail_ms;
   uint64_t tail_launches;
   /* with TPT_RENDER_COUNT_OPS (else 0): slab tests, sphere tests, rect tests
    * and wrapper chains (translate / rotate_y) applied by the closest-hit walks */

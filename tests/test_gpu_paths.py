@@ -1,8 +1,9 @@
 """Plain renders in one path launch per pass (k_paths) against the bounce loop.
 
-By default a plain render of a scene with constant textures and at most one
-rect light carries every path through all its bounces in one launch; with
-tail=False (TPT_RENDER_NO_TAIL) the bounce loop renders it.  Same functions,
+By default a plain render carries every path through all its bounces in one
+launch; with tail=False (TPT_RENDER_NO_TAIL) the bounce loop renders it.  The
+scenes cover every variant of the kernel: each walk (small scenes, sphere-only,
+general, media) with simple and with general shading, alone and pooled.  Same functions,
 same Philox streams, samples summed in the same order: the sums must be equal
 bit for bit and the counts the same, at sizes around a wave's 64 rays, the 64
 work shards and a block's 256 threads.
@@ -14,7 +15,8 @@ pytestmark = pytest.mark.gpu
 COUNTS = ("paths", "segments", "light_queries", "nodes_visited", "nan_samples")
 
 
-@pytest.mark.parametrize("name", ["cornell555", "random_spheres", "random_spheres_n3000"])
+@pytest.mark.parametrize("name", ["cornell555", "random_spheres", "random_spheres_n3000", "ref_cornell_box",
+                                  "random_spheres_textured", "box_list", "cornell_smoke", "ref_random_scene"])
 @pytest.mark.parametrize("w,h,spp,depth,offset", [
     (1, 1, 1, 50, 0),        # one path
     (9, 7, 1, 50, 3),        # 63 items: one short run of rays
@@ -36,15 +38,27 @@ def test_paths_equal_bounce_loop(tpt, device, name, w, h, spp, depth, offset):
     for k in COUNTS:
         assert sa[k] == sb[k], k
     assert sa["paths"] == w * h * spp
-    assert sa["tail_launches"] == 1 and sa["tail_segments"] == sa["segments"]
+    if name in ("cornell555", "random_spheres", "random_spheres_n3000"):  # the scenes that tail_* counts
+        assert sa["tail_launches"] == 1 and sa["tail_segments"] == sa["segments"]
     assert sb["tail_launches"] == 0
 
 
-def test_paths_pooled_jobs_equal_bounce_loop(tpt, device):
+POOLS = {
+    "spheres": [f"random_spheres_n{n}" for n in (60, 900, 90, 2500, 300)],
+    "textured spheres": ["random_spheres_textured", "random_spheres_n70", "random_spheres", "random_spheres_n400",
+                         "random_spheres_textured"],
+    "simple": ["cornell555", "random_spheres", "box_list", "cornell555", "random_spheres_n60"],
+    "general": ["ref_cornell_box", "ref_random_scene", "ref_two_perlin_spheres", "box_list", "random_spheres"],
+    "media": ["cornell_smoke", "ref_random_scene", "cornell555", "cornell_smoke", "random_spheres"],
+}
+
+
+@pytest.mark.parametrize("which", list(POOLS))
+def test_paths_pooled_jobs_equal_bounce_loop(tpt, device, which):
     """Jobs of several scenes and sizes in one launch, sums without squares among them."""
     import torch
 
-    hosts = [tpt.HostScene(f"random_spheres_n{n}", seed=k + 1) for k, n in enumerate((60, 900, 90, 2500, 300))]
+    hosts = [tpt.HostScene(n, seed=k + 1) for k, n in enumerate(POOLS[which])]
     pool = tpt.Scene.pool(hosts)
 
     def run(flags):
@@ -65,4 +79,4 @@ def test_paths_pooled_jobs_equal_bounce_loop(tpt, device):
         assert torch.equal(x, y)
     for k in COUNTS:
         assert sa[k] == sb[k], k
-    assert sa["tail_launches"] == 1 and sb["tail_launches"] == 0
+    assert sa["tail_launches"] == (1 if which == "spheres" else 0) and sb["tail_launches"] == 0

@@ -13,7 +13,9 @@
 // (two Philox blocks and three double divisions) never runs for a few lanes.
 // Measured, bounce loop -> this kernel: Cornell 1200x1200 128 spp 48.8 -> 41.4
 // ms, random spheres 400x400 16 spp 3.39 -> 2.51 ms, 16 pooled renders of up
-// to 8000 spheres 14.3 -> 11.2 ms.
+// to 8000 spheres 14.3 -> 11.2 ms; with textures (1600x1600 12 spp) 23.4 ->
+// 18.5 ms, media (smoke box 400x400 64 spp) 7.8 -> 6.0 ms, a 160x120 4 spp
+// preview 1.14 -> 0.67 ms.
 //
 // The grid is what stays resident (4 waves per SIMD); a wave leaves its loop
 // when the shards are empty and its lanes' paths have ended, at most max_depth
@@ -47,8 +49,15 @@ __device__ __forceinline__ uint32_t claim_run(const pass_hdr &H, uint32_t *count
   return 0;
 }
 
-template <bool SWEEP, bool MULTI>
-__global__ void __launch_bounds__(PATH_THREADS) __attribute__((amdgpu_waves_per_eu(4)))
+// SWEEP, SPH, MEDIA: the walk, as for k_trace; SIMPLE: the shading, as for k_shade.
+// Waves per SIMD: 4 fit 128 VGPRs without spilling where one walk is compiled;
+// the general walk needs 3 waves' registers, the media walk 2.
+__host__ __device__ constexpr uint32_t path_waves(bool sweep, bool sph, bool simple, bool media) {
+  return media ? 2u : (sweep || sph || simple ? 4u : 3u);
+}
+
+template <bool SWEEP, bool MULTI, bool SPH, bool SIMPLE, bool MEDIA = false>
+__global__ void __launch_bounds__(PATH_THREADS) __attribute__((amdgpu_waves_per_eu(path_waves(SWEEP, SPH, SIMPLE, MEDIA))))
 k_paths(scene_view S, const tpt_slot *__restrict__ slots, const tpt_entry *__restrict__ entries, render_params P,
         render_state Q) {
   S.slots = slots;
@@ -112,9 +121,10 @@ k_paths(scene_view S, const tpt_slot *__restrict__ slots, const tpt_entry *__res
     const item_ctx c{p.ent, job, px, smp};
     const scene_view Sj = view_of<MULTI>(S, P, job);
     hit_t h{0.0f, kNone, kNone, 0};
-    const ray_ctx rc{0.0f, 0u, 0u, 0u, 0u, 0u};
+    const ray_ctx rc = !SIMPLE && !SWEEP && !SPH && (P.motion | P.media) && live ? make_ray_ctx(P, c, p.depth)
+                                                                                 : ray_ctx{0.0f, 0u, 0u, 0u, 0u, 0u};
     const bool got =
-        trace_world<SWEEP, !SWEEP, false>(Sj, p.o, p.d, rc, 0.001f, kFltMax, &h, &st[ST_NODES], live);
+        trace_world<SWEEP, SPH, MEDIA>(Sj, p.o, p.d, rc, 0.001f, kFltMax, &h, &st[ST_NODES], live);
     if (live) {
       ++st[ST_SEGMENTS];
       uint32_t cls = Q_TERMINAL;
@@ -124,7 +134,7 @@ k_paths(scene_view S, const tpt_slot *__restrict__ slots, const tpt_entry *__res
       } else {
         h.slot = kNone;
       }
-      if (!shade_hit<true>(S, Sj, P, P.jobs[job], c, p, h, cls, st)) {
+      if (!shade_hit<SIMPLE>(S, Sj, P, P.jobs[job], c, p, h, cls, st)) {
         const pass_ent E = P.pass[MULTI ? p.ent : 0u];
         p.item = E.item_begin + (smp - E.s_begin) * P.jobs[job].n_pix + px;
         finish_sample<false>(P, Q, p, st);

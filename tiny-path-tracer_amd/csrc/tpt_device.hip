@@ -775,17 +775,28 @@ void launch_tail(const bounce_launch &B, hipStream_t st, uint32_t parity, uint32
   }
 }
 
-// Blocks per CU of k_paths (its occupancy target is in waves per SIMD, one block of 4 waves each).
-uint32_t path_blocks_per_cu(const bounce_launch &) { return 4; }
+// Blocks per CU of k_paths: its occupancy target, in waves per SIMD, one block of 4 waves each.
+uint32_t path_blocks_per_cu(const bounce_launch &B) { return path_waves(B.sweep, B.sph, B.simple, B.P.media != 0); }
+
+template <bool SWEEP, bool MULTI, bool SPH, bool SIMPLE, bool MEDIA>
+void launch_paths_t(const bounce_launch &B, hipStream_t st, uint32_t grid) {
+  hipLaunchKernelGGL((k_paths<SWEEP, MULTI, SPH, SIMPLE, MEDIA>), dim3(grid), dim3(PATH_THREADS), 0, st, B.S,
+                     B.S.slots, B.S.entries, B.P, B.Q);
+}
 
 void launch_paths(const bounce_launch &B, hipStream_t st, uint32_t grid) {
-  const dim3 g(grid), b(PATH_THREADS);
-  if (B.sweep)
-    hipLaunchKernelGGL((k_paths<true, false>), g, b, 0, st, B.S, B.S.slots, B.S.entries, B.P, B.Q);
-  else if (B.multi)
-    hipLaunchKernelGGL((k_paths<false, true>), g, b, 0, st, B.S, B.S.slots, B.S.entries, B.P, B.Q);
-  else
-    hipLaunchKernelGGL((k_paths<false, false>), g, b, 0, st, B.S, B.S.slots, B.S.entries, B.P, B.Q);
+  if (B.P.media) return B.multi ? launch_paths_t<false, true, false, false, true>(B, st, grid)
+                                : launch_paths_t<false, false, false, false, true>(B, st, grid);
+  if (B.sweep) return B.simple ? launch_paths_t<true, false, false, true, false>(B, st, grid)
+                               : launch_paths_t<true, false, false, false, false>(B, st, grid);
+  if (B.sph && B.simple) return B.multi ? launch_paths_t<false, true, true, true, false>(B, st, grid)
+                                        : launch_paths_t<false, false, true, true, false>(B, st, grid);
+  if (B.sph) return B.multi ? launch_paths_t<false, true, true, false, false>(B, st, grid)
+                            : launch_paths_t<false, false, true, false, false>(B, st, grid);
+  if (B.simple) return B.multi ? launch_paths_t<false, true, false, true, false>(B, st, grid)
+                               : launch_paths_t<false, false, false, true, false>(B, st, grid);
+  B.multi ? launch_paths_t<false, true, false, false, false>(B, st, grid)
+          : launch_paths_t<false, false, false, false, false>(B, st, grid);
 }
 
 template <bool COUNT>
@@ -956,13 +967,19 @@ int render_paths(tpt_scene *s, const std::vector<job_dev> &jd, const std::vector
     float ms = 0.0f;
     (void)hipEventElapsedTime(&ms, s->ev_begin, s->ev_end);
     stats->paths = t[ST_PATHS];
-    stats->segments = stats->tail_segments = t[ST_SEGMENTS];
+    stats->segments = t[ST_SEGMENTS];
     stats->light_queries = t[ST_LIGHT];
     stats->nan_samples = t[ST_NAN];
     stats->nodes_visited = t[ST_NODES];
     stats->kernel_ms = ms;
-    stats->tail_ms = path_ms;
-    stats->tail_launches = plan.size();
+    if (B.tail) {
+      stats->tail_segments = t[ST_SEGMENTS];
+      stats->tail_ms = path_ms;
+      stats->tail_launches = plan.size();
+    } else {
+      stats->trace_ms = path_ms;
+      stats->trace_launches = profile ? plan.size() : 0;
+    }
   }
   return TPT_OK;
 }
@@ -1035,7 +1052,7 @@ int render_core(tpt_scene *s, const tpt_job *jobs, uint32_t n_jobs, const tpt_la
   B.P.scenes = s->d_scenes;
   B.P.guide_verts = ~0u;
   B.P.media_scatter = (L.flags & TPT_RENDER_MEDIA_SCATTER) ? 1u : 0u;
-  if (B.tail && !guide)
+  if (!guide && !B.count && !(L.flags & TPT_RENDER_NO_TAIL))
     return render_paths(s, jd, plan_passes(jobs, n_jobs, kPassItemsPaths), B, profile, stats, cs);
   const std::vector<pass_plan> plan =
       plan_passes(jobs, n_jobs, guide && L.guiding ? kPassItemsRecording : kPassItems);
