@@ -365,7 +365,8 @@ typedef struct tpt_render_stats {
   uint64_t light_queries;  /* light-pdf intersections */
   uint64_t nan_samples;    /* samples with a NaN channel zeroed by de_nan */
   double kernel_ms;        /* GPU time of the whole pass (events around it) */
-  uint64_t nodes_visited;  /* pre-order slots visited by closest-hit queries */
+  uint64_t nodes_visited;  /* pre-order slots visited by closest-hit queries (small scenes, which are traced
+                              without a walk: the primitives, a closed box of six rects counting once) */
   double trace_ms, shade_ms;          /* with TPT_RENDER_PROFILE */
   uint64_t trace_launches, shade_launches;
   /* the fused launches of the scenes that k_tail takes (k_tail and, for plain

@@ -35,6 +35,33 @@ __device__ __forceinline__ float len(v3 a) { return sqrtf(dot(a, a)); }
 __device__ __forceinline__ v3 unit(v3 a) { return a / len(a); }
 __device__ __forceinline__ float comp(v3 a, uint32_t i) { return i == 0 ? a.x : (i == 1 ? a.y : a.z); }
 
+// What the uniform pass of walk_flat.h reads of a small scene's primitives, 32
+// bytes each, through scalar loads.  rect: plane k, in-plane centres c0, c1
+// and half-extents h0, h1.  sphere: centre (k, c0, c1), radius h0.  box (six
+// rects of one list that close a box): low corner (k, c0, c1), high corner
+// (h0, h1, x).  win: its record in flat_wins (a box: of its low x face, then
+// high x, low y, high y, low z, high z).
+struct flat_scan {
+  float k, c0, c1, h0, h1, x;
+  uint32_t win, pad;
+};
+// What its winner needs, 80 bytes.
+struct flat_win {
+  float f[5];                 // primitive parameters as in tpt_slot
+  uint32_t slot, entry, mat;  // as in hit_t
+  float box[6];               // the innermost box around it
+  uint32_t boxed;             // 0: there is none, or it is passed whenever the winner is certain
+  uint32_t xform, kind, leaf;  // wrapper chain or ~0u; TPT_SLOT_RECT or TPT_SLOT_SPHERE; leaf id
+  uint32_t order, pad;         // its place in the order of segments, slots and entries
+};
+// Primitives seen through one wrapper chain, in this order: rects by normal
+// axis (counts in bits 0-7, 8-15, 16-23 of n), spheres (24-31), boxes (n_box);
+// and the chain itself (nops 0: none), so that one load fetches all of it.
+struct flat_group {
+  uint32_t n, n_box, nops, kinds;
+  float p[TPT_XFORM_MAX_OPS][3];
+};
+
 // Read-only scene arrays on the device (all in HBM; the hot ones are small
 // enough to stay L2-resident for the benchmark scenes).
 struct scene_view {
@@ -49,6 +76,12 @@ struct scene_view {
   const tpt_light *lights;
   const tpt_motion *motions;
   const uint32_t *seg_xf;  // per segment: xform | flip<<31 (TPT_SEGMENT_PLAIN), or null: none wrapped
+  const flat_scan *flat;  // small scenes: every primitive, by group
+  const flat_win *fwins;
+  const flat_group *fgroups;
+  uint32_t n_fgroups, n_flat;  // 0: no uniform pass
+  uint32_t flat_nan;   // record of the last rect in the reference's order, or ~0u
+  float flat_mag;      // largest coordinate magnitude of its primitives and wrappers
   uint32_t n_slots, n_segments, n_lights, light_mode;
   float walk_ulp;  // 2^-22 x the largest coordinate magnitude of the scene (sphere-only walk bound)
 };

@@ -123,8 +123,8 @@ k_paths(scene_view S, const tpt_slot *__restrict__ slots, const tpt_entry *__res
     hit_t h{0.0f, kNone, kNone, 0};
     const ray_ctx rc = !SIMPLE && !SWEEP && !SPH && (P.motion | P.media) && live ? make_ray_ctx(P, c, p.depth)
                                                                                  : ray_ctx{0.0f, 0u, 0u, 0u, 0u, 0u};
-    const bool got =
-        trace_world<SWEEP, SPH, MEDIA>(Sj, p.o, p.d, rc, 0.001f, kFltMax, &h, &st[ST_NODES], live);
+    const bool got = SWEEP ? small_world(Sj, p.o, p.d, rc, 0.001f, kFltMax, &h, &st[ST_NODES], live)
+                           : trace_world<false, SPH, MEDIA>(Sj, p.o, p.d, rc, 0.001f, kFltMax, &h, &st[ST_NODES], live);
     if (live) {
       ++st[ST_SEGMENTS];
       uint32_t cls = Q_TERMINAL;

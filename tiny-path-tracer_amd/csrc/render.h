@@ -30,6 +30,7 @@
 
 #include "guide.h"
 #include "shade.h"
+#include "walk_flat.h"
 
 #pragma clang fp contract(off)
 
@@ -428,16 +429,15 @@ __global__ void __launch_bounds__(256) k_init(render_params P, render_state Q) {
   }
 }
 
-// SWEEP: wave-uniform traversal for small scenes (see segment_sweep).  SPH:
+// SWEEP: the uniform pass of small scenes (walk_flat.h).  SPH:
 // every leaf of the scene (or pool) is a sphere; without the rect and list
 // code the kernel fits 64 registers, 8 waves per SIMD.  MEDIA: the scenes hold
 // constant_media (their code costs registers, so only this variant has it).  The slot/entry arrays come
 // in as separate restrict arguments so that wave-uniform loads from them can
 // use the scalar data path.  COUNT: also counts the walk's operations by kind
 // (TPT_RENDER_COUNT_OPS; the other variants are built without that code).
-// The sweep variant parks its path record in LDS during the walk (see below)
-// and targets 6 waves per SIMD (80 VGPRs, 4 spilled): 4% faster on the Cornell
-// frame than 5 waves with the record in registers, 2% faster than 7 waves.
+// The path record is parked in LDS during the walk (see below); the uniform
+// pass then fits 71 VGPRs.
 constexpr uint32_t TRACE_THREADS = 256;  // k_trace's block size (its record stash holds one record per thread)
 template <bool SWEEP, bool MULTI, bool SPH = false, bool MEDIA = false, bool COUNT = false>
 __global__ void __launch_bounds__(TRACE_THREADS) __attribute__((amdgpu_waves_per_eu(SPH ? 8 : (MEDIA ? 1 : (SWEEP ? 6 : 5))))) k_trace(scene_view S, const tpt_slot *__restrict__ slots,
@@ -445,6 +445,7 @@ __global__ void __launch_bounds__(TRACE_THREADS) __attribute__((amdgpu_waves_per
                                                render_state Q, uint32_t parity) {
   static_assert(!(SWEEP && MULTI), "the wave-uniform sweep needs one scene");
   static_assert(!(SWEEP && SPH), "the sweep takes every leaf kind");
+  static_assert(!(COUNT && SWEEP), "operations are counted in the walks of each lane");
   static_assert(!(MEDIA && (SWEEP || SPH)), "media go through the general walk");
   S.slots = slots;
   S.entries = entries;
@@ -465,8 +466,7 @@ __global__ void __launch_bounds__(TRACE_THREADS) __attribute__((amdgpu_waves_per
   // The record read before the walk is stored here and read back after it:
   // only the ray stays in registers across the walk.  The compiler barrier
   // before the read-back keeps the compiler from forwarding the stored values
-  // in registers.  Measured: Cornell +4% with the sweep at 6 waves;
-  // sphere-only walk at 8 waves, 19 instead of 23 spilled VGPRs, batch64 +3%;
+  // in registers.  Measured: sphere-only walk at 8 waves, 19 instead of 23 spilled VGPRs, batch64 +3%;
   // the general walk spills 2-11 instead of 6-13 VGPRs (no change in time on
   // box_list).
   __shared__ float4 stash[3 * TRACE_THREADS];
@@ -476,8 +476,8 @@ __global__ void __launch_bounds__(TRACE_THREADS) __attribute__((amdgpu_waves_per
     uint32_t cls = 3;
     // Without SWEEP only the ray and the (depth, entry) word stay live across
     // the traversal (fewer registers, more waves); the third plane is read
-    // after it.  The sweep's waves are few and short of latency cover, so it
-    // reads the whole record first (and parks it in LDS during the walk).
+    // after it.  The uniform pass is short of latency cover, so it reads the
+    // whole record first (and parks it in LDS meanwhile).
     uint32_t src = 0;
     float4 a{}, b{}, c0{};
     hit_t h{0.0f, kNone, kNone, 0};
@@ -523,8 +523,10 @@ __global__ void __launch_bounds__(TRACE_THREADS) __attribute__((amdgpu_waves_per
       else
         got = trace_world<false, SPH, MEDIA>(Sj, v3{a.x, a.y, a.z}, v3{b.x, b.y, b.z}, rc, 0.001f, kFltMax, &h,
                                              &st[ST_NODES], valid, COUNT ? &oc : nullptr);
+    } else if (SWEEP) {
+      got = small_world(Sj, v3{a.x, a.y, a.z}, v3{b.x, b.y, b.z}, rc, 0.001f, kFltMax, &h, &st[ST_NODES], valid);
     } else {
-      got = trace_world<SWEEP, SPH, MEDIA>(Sj, v3{a.x, a.y, a.z}, v3{b.x, b.y, b.z}, rc, 0.001f, kFltMax, &h,
+      got = trace_world<false, SPH, MEDIA>(Sj, v3{a.x, a.y, a.z}, v3{b.x, b.y, b.z}, rc, 0.001f, kFltMax, &h,
                                            &st[ST_NODES], valid, COUNT ? &oc : nullptr);
     }
     {
@@ -1042,8 +1044,9 @@ __global__ void __launch_bounds__(256) k_tail(scene_view S, const tpt_slot *__re
       const item_ctx c = live ? item_in_entry(P, MULTI ? p.ent : 0u, p.item) : item_ctx{0u, 0u, 0u, 0u};
       const scene_view Sj = view_of<MULTI>(S, P, c.job);
       hit_t h{0.0f, kNone, kNone, 0};
-      const bool got = trace_world<SWEEP, SPH, false>(Sj, p.o, p.d, ray_ctx{0.0f, 0u, 0u, 0u, 0u, 0u}, 0.001f,
-                                                      kFltMax, &h, &st[ST_NODES], live);
+      const ray_ctx rc{0.0f, 0u, 0u, 0u, 0u, 0u};
+      const bool got = SWEEP ? small_world(Sj, p.o, p.d, rc, 0.001f, kFltMax, &h, &st[ST_NODES], live)
+                             : trace_world<false, SPH, false>(Sj, p.o, p.d, rc, 0.001f, kFltMax, &h, &st[ST_NODES], live);
       uint32_t cls = Q_TERMINAL;
       if (live) {
         ++st[ST_SEGMENTS];

@@ -33,6 +33,7 @@ __global__ void __launch_bounds__(256) k_trace_closest(scene_view S, const tpt_s
                                                        int32_t *__restrict__ mat) {
   S.slots = slots;
   S.entries = entries;
+  if (SWEEP) flat_touch(S);
   const uint64_t i = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   const bool live = i < n;
   v3 o{0.0f, 0.0f, 0.0f}, d{0.0f, 0.0f, 0.0f};
@@ -44,11 +45,12 @@ __global__ void __launch_bounds__(256) k_trace_closest(scene_view S, const tpt_s
     if (times) rc.time = times[i];
   }
   hit_t h;
-  uint32_t nodes = 0;
-  const bool got = trace_world<SWEEP, SPH, MEDIA>(S, o, d, rc, tmin, tmax, &h, &nodes, live);
+  uint32_t nodes = 0, id = 0;
+  const bool got = SWEEP ? small_world<true>(S, o, d, rc, tmin, tmax, &h, &nodes, live, &id)
+                         : trace_world<false, SPH, MEDIA>(S, o, d, rc, tmin, tmax, &h, &nodes, live);
   if (!live) return;
   if (got) {
-    leaf[i] = static_cast<int32_t>(leaf_id(S, h));
+    leaf[i] = static_cast<int32_t>(SWEEP ? id : leaf_id(S, h));
     tout[i] = h.t;
     if (rec) {
       v3 p, nn;
@@ -93,6 +95,13 @@ bool is_gfx950(int dev) {
 
 }  // namespace
 
+// A scene's part of the uniform pass's arrays (n_groups 0: it has none).
+struct flat_range {
+  uint32_t scan0 = 0, win0 = 0, group0 = 0, n_groups = 0, n_scans = 0;
+  uint32_t nan_win = 0xFFFFFFFFu;
+  float mag = 0.0f;
+};
+
 // A scene handle: one or more flattened scenes packed into one pool (indices
 // rebased), plus the render state grown on demand.
 struct tpt_scene {
@@ -109,6 +118,9 @@ struct tpt_scene {
   tpt_light *lights = nullptr;
   tpt_motion *motions = nullptr;
   uint32_t *seg_xf = nullptr;  // per pooled segment; null when no scene has a wrapped segment
+  flat_scan *flat = nullptr;   // records of the uniform pass (walk_flat.h) of the small scenes
+  flat_win *fwins = nullptr;
+  flat_group *fgroups = nullptr;
   uint32_t n_slots = 0, n_segments = 0, n_lights = 0;
   // the pool's scenes
   std::vector<scene_dev> scn;
@@ -117,6 +129,7 @@ struct tpt_scene {
   std::vector<uint8_t> simple;    // per scene: constant textures, no light or one xz_rect light
   std::vector<uint8_t> motion;    // per scene: has moving spheres (rays need their time)
   std::vector<uint8_t> media;     // per scene: has constant_medium (queries need media draws)
+  std::vector<flat_range> flat_of;  // per scene: its part of flat and fgroups
   std::vector<uint32_t> n_slots_of;
   std::vector<uint32_t> n_leaves_of;
   scene_dev *d_scenes = nullptr;
@@ -159,6 +172,13 @@ struct tpt_scene {
     v.lights = lights + scn[k].light_begin;
     v.motions = motions;
     v.seg_xf = seg_xf ? seg_xf + scn[k].seg_begin : nullptr;
+    v.flat = flat ? flat + flat_of[k].scan0 : nullptr;
+    v.fwins = fwins ? fwins + flat_of[k].win0 : nullptr;
+    v.fgroups = fgroups ? fgroups + flat_of[k].group0 : nullptr;
+    v.n_fgroups = flat_of[k].n_groups;
+    v.n_flat = flat_of[k].n_scans;
+    v.flat_nan = flat_of[k].nan_win;
+    v.flat_mag = flat_of[k].mag;
     v.n_slots = n_slots;
     v.n_segments = scn[k].n_seg;
     v.n_lights = scn[k].n_lights;
@@ -192,6 +212,9 @@ void free_scene(tpt_scene *s) {
   (void)hipFree(s->lights);
   (void)hipFree(s->motions);
   (void)hipFree(s->seg_xf);
+  (void)hipFree(s->flat);
+  (void)hipFree(s->fwins);
+  (void)hipFree(s->fgroups);
   (void)hipFree(s->d_scenes);
   (void)hipFree(s->state);
   (void)hipFree(s->d_jobs);
@@ -389,6 +412,173 @@ float rebase_bits(float f, uint32_t base) {
   return f;
 }
 
+// Records of the uniform pass (walk_flat.h) for a scene that is walked by the
+// wave together, appended to scans / wins / groups: every sphere and rect of
+// its slots and lists, grouped by wrapper chain; six rects in a row of one
+// list that close a box become one record.  sb, eb, xb, mb: the scene's first
+// slot, entry, transform and material in the pool.
+constexpr uint32_t kFlatMax = 64;  // most primitives of the pass
+enum { FLAT_SPHERE = 3, FLAT_BOX = 4 };
+struct flat_item {
+  flat_scan scan;
+  flat_win win[6];  // one, or a box's faces
+  uint32_t cls;     // 0..2 rect by axis, FLAT_SPHERE, FLAT_BOX
+};
+
+// The closed box of six rects (k, a0, a1, b0, b1 with axes), if they are one:
+// lo / hi corners and which of them is each face (low x, high x, low y, ...).
+bool closed_box(const flat_item *r, float lo[3], float hi[3], int face[6]) {
+  for (int a = 0; a < 3; ++a) {
+    int at[2], n = 0;
+    for (int i = 0; i < 6; ++i)
+      if (r[i].cls == static_cast<uint32_t>(a)) {
+        if (n == 2) return false;
+        at[n++] = i;
+      }
+    if (n != 2) return false;
+    const float k0 = r[at[0]].win[0].f[0], k1 = r[at[1]].win[0].f[0];
+    if (!(k0 != k1)) return false;
+    const int l = k0 < k1 ? 0 : 1;
+    lo[a] = std::fmin(k0, k1), hi[a] = std::fmax(k0, k1);
+    face[2 * a] = at[l], face[2 * a + 1] = at[1 - l];
+  }
+  for (int i = 0; i < 6; ++i) {
+    const uint32_t a = r[i].cls, u = a == 0 ? 1 : 0, v = a == 2 ? 1 : 2;  // in-plane axes
+    const float *f = r[i].win[0].f;
+    if (f[1] != lo[u] || f[2] != hi[u] || f[3] != lo[v] || f[4] != hi[v]) return false;
+    if (r[i].win[0].xform != r[0].win[0].xform || r[i].win[0].slot != r[0].win[0].slot) return false;
+  }
+  return true;
+}
+
+flat_range flat_records(const tpt_flat_scene &f, uint32_t sb, uint32_t eb, uint32_t xb, uint32_t mb,
+                        std::vector<flat_scan> *scans, std::vector<flat_win> *wins, std::vector<flat_group> *groups) {
+  std::vector<flat_item> items;
+  float mag = 0.0f;
+  bool ok = true;
+  auto add = [&](const float *w, uint32_t kind, uint32_t word, uint32_t xform, uint32_t slot, uint32_t entry,
+                 uint32_t leaf, uint32_t parent) {
+    flat_item it{};
+    flat_win &q = it.win[0];
+    const int nf = kind == TPT_SLOT_RECT ? 5 : 4;
+    for (int k = 0; k < nf; ++k) q.f[k] = w[k], ok = ok && std::fabs(w[k]) < 1e18f;
+    flat_scan &p = it.scan;
+    p.k = w[0];
+    if (kind == TPT_SLOT_RECT) {
+      it.cls = (word >> 28) & 3u;
+      p.c0 = 0.5f * (w[1] + w[2]), p.c1 = 0.5f * (w[3] + w[4]);
+      p.h0 = 0.5f * (w[2] - w[1]), p.h1 = 0.5f * (w[4] - w[3]);
+      for (int k = 0; k < 5; ++k) mag = std::fmax(mag, std::fabs(w[k]));
+      ok = ok && it.cls < 3;
+      if (ok && parent != kNone && xform == 0xFFFFFFFFu) {
+        // inside its parent box: the box needs no test of its own
+        const float *b = f.slots[parent].f;
+        const uint32_t a = it.cls, u = a == 0 ? 1 : 0, v = a == 2 ? 1 : 2;
+        if (b[a] <= w[0] && w[0] <= b[3 + a] && b[u] <= w[1] && w[2] <= b[3 + u] && b[v] <= w[3] && w[4] <= b[3 + v])
+          parent = kNone;
+      }
+    } else if (kind == TPT_SLOT_SPHERE) {
+      it.cls = FLAT_SPHERE;
+      p.c0 = w[1], p.c1 = w[2], p.h0 = w[3];
+      for (int k = 0; k < 3; ++k) mag = std::fmax(mag, std::fabs(w[k]) + std::fabs(w[3]));
+    } else {
+      ok = false;
+    }
+    q.slot = slot + sb, q.entry = entry == kNone ? kNone : entry + eb, q.kind = kind;
+    q.leaf = leaf;
+    q.order = static_cast<uint32_t>(items.size());
+    q.boxed = parent != kNone;
+    if (q.boxed) std::memcpy(q.box, f.slots[parent].f, sizeof(q.box));
+    q.mat = rebase_word(word, mb);
+    q.xform = xform == 0xFFFFFFFFu ? kNone : xform + xb;
+    items.push_back(it);
+  };
+  for (uint32_t g = 0; g < f.n_segments; ++g) {
+    std::vector<uint32_t> open;  // boxes around slot i
+    for (uint32_t i = f.segments[2 * g]; i < f.segments[2 * g + 1]; ++i) {
+      const tpt_slot &s = f.slots[i];
+      while (!open.empty() && f.slots[open.back()].a <= i) open.pop_back();
+      const uint32_t kind = s.b >> 28, parent = open.empty() ? kNone : open.back();
+      if (kind == TPT_SLOT_BOX) {
+        open.push_back(i);
+      } else if (kind == TPT_SLOT_LIST) {
+        uint32_t cnt, leaf0;
+        std::memcpy(&leaf0, &s.f[0], 4);
+        std::memcpy(&cnt, &s.f[1], 4);
+        for (uint32_t e = s.a; e < s.a + cnt; ++e)
+          add(f.entries[e].f, f.entries[e].b, f.entries[e].a, f.entries[e].xform, i, e, leaf0 + (e - s.a), parent);
+      } else {
+        add(s.f, kind, s.a, 0xFFFFFFFFu, i, kNone, s.b & TPT_PAYLOAD_MASK, parent);
+      }
+    }
+  }
+  // a chain's offsets reach the local coordinates (1.5: its rotations)
+  float reach = 0.0f;
+  for (uint32_t x = 0; x < f.n_xforms; ++x) {
+    float off = 0.0f;
+    for (uint32_t i = 0; i < f.xforms[x].nops; ++i)
+      for (int k = 0; k < 3; ++k) {
+        ok = ok && std::fabs(f.xforms[x].p[i][k]) < 1e18f;
+        if (((f.xforms[x].kinds >> (2 * i)) & 3u) == TPT_XFORM_TRANSLATE) off += std::fabs(f.xforms[x].p[i][k]);
+      }
+    reach = std::fmax(reach, 1.5f * off);
+  }
+  flat_range r;
+  if (!ok || items.empty() || items.size() > kFlatMax) return r;
+  // the last rect in the order of slots and entries
+  uint32_t nan_slot = kNone, nan_entry = kNone;
+  for (const flat_item &it : items)
+    if (it.win[0].kind == TPT_SLOT_RECT) nan_slot = it.win[0].slot, nan_entry = it.win[0].entry;
+  std::vector<flat_item> merged;
+  for (size_t i = 0; i < items.size();) {
+    float lo[3], hi[3];
+    int face[6];
+    if (i + 6 <= items.size() && items[i].win[0].entry != kNone && closed_box(&items[i], lo, hi, face)) {
+      flat_item b{};
+      b.cls = FLAT_BOX;
+      b.scan.k = lo[0], b.scan.c0 = lo[1], b.scan.c1 = lo[2];
+      b.scan.h0 = hi[0], b.scan.h1 = hi[1], b.scan.x = hi[2];
+      for (int k = 0; k < 6; ++k) b.win[k] = items[i + face[k]].win[0];
+      merged.push_back(b);
+      i += 6;
+    } else {
+      merged.push_back(items[i++]);
+    }
+  }
+  r.scan0 = static_cast<uint32_t>(scans->size());
+  r.win0 = static_cast<uint32_t>(wins->size());
+  r.group0 = static_cast<uint32_t>(groups->size());
+  r.mag = mag + reach;
+  std::vector<uint32_t> chains;
+  for (const flat_item &it : merged)
+    if (std::find(chains.begin(), chains.end(), it.win[0].xform) == chains.end()) chains.push_back(it.win[0].xform);
+  for (uint32_t xf : chains) {
+    flat_group fg{};
+    if (xf != kNone) {
+      const tpt_xform &x = f.xforms[xf - xb];
+      fg.nops = x.nops, fg.kinds = x.kinds;
+      std::memcpy(fg.p, x.p, sizeof(fg.p));
+    }
+    for (uint32_t c = 0; c <= FLAT_BOX; ++c)
+      for (flat_item &it : merged)
+        if (it.win[0].xform == xf && it.cls == c) {
+          it.scan.win = static_cast<uint32_t>(wins->size()) - r.win0;
+          scans->push_back(it.scan);
+          wins->insert(wins->end(), it.win, it.win + (c == FLAT_BOX ? 6 : 1));
+          if (c == FLAT_BOX)
+            ++fg.n_box;
+          else
+            fg.n += 1u << (8 * c);
+        }
+    groups->push_back(fg);
+  }
+  r.n_groups = static_cast<uint32_t>(chains.size());
+  r.n_scans = static_cast<uint32_t>(merged.size());
+  for (uint32_t w = r.win0; nan_slot != kNone && w < wins->size(); ++w)
+    if ((*wins)[w].slot == nan_slot && (*wins)[w].entry == nan_entry) r.nan_win = w - r.win0;
+  return r;
+}
+
 int create_pool(const tpt_flat_scene *scenes, uint32_t n, tpt_scene **out) {
   if (!scenes || !out || n == 0) return tpt::fail(TPT_ERR_INVALID, "tpt_scene_create: no scenes");
   *out = nullptr;
@@ -411,6 +601,10 @@ int create_pool(const tpt_flat_scene *scenes, uint32_t n, tpt_scene **out) {
   std::vector<scene_dev> scn(n);
   std::vector<uint8_t> sweep(n), sph(n), simple(n), motion(n), media(n);
   std::vector<uint32_t> nslots(n), nleaves(n);
+  std::vector<flat_scan> flat;
+  std::vector<flat_win> fwins;
+  std::vector<flat_group> fgroups;
+  std::vector<flat_range> flat_of(n);
   for (uint32_t k = 0; k < n; ++k) {
     const tpt_flat_scene &f = scenes[k];
     const uint64_t sb = slots.size(), eb = entries.size(), xb = xforms.size(), mb = materials.size(),
@@ -507,6 +701,11 @@ int create_pool(const tpt_flat_scene *scenes, uint32_t n, tpt_scene **out) {
     bool wrapped = false;
     for (uint32_t g = 0; f.segment_xforms && g < f.n_segments; ++g) wrapped |= f.segment_xforms[g] != TPT_SEGMENT_PLAIN;
     sweep[k] = f.n_slots <= 64 && !motion[k] && !media[k] && !wrapped;
+    if (sweep[k]) {
+      flat_of[k] = flat_records(f, static_cast<uint32_t>(sb), static_cast<uint32_t>(eb), static_cast<uint32_t>(xb),
+                                static_cast<uint32_t>(mb), &flat, &fwins, &fgroups);
+      sweep[k] = flat_of[k].n_groups > 0;
+    }
     if (wrapped) sph[k] = 0;  // the sphere-only walk is built without segment transforms
     simple[k] = !motion[k] && !media[k] &&
                 (f.n_lights == 0 || (f.light_mode == 0 && f.lights[0].kind == TPT_LIGHT_XZ_RECT));
@@ -531,6 +730,9 @@ int create_pool(const tpt_flat_scene *scenes, uint32_t n, tpt_scene **out) {
       (rc = upload(&s->lights, lights.data(), lights.size())) ||
       (rc = upload(&s->motions, motions.data(), motions.size())) ||
       (rc = upload(&s->seg_xf, seg_xf.data(), any_wrapped ? seg_xf.size() : 0)) ||
+      (rc = upload(&s->flat, flat.data(), flat.size())) ||
+      (rc = upload(&s->fwins, fwins.data(), fwins.size())) ||
+      (rc = upload(&s->fgroups, fgroups.data(), fgroups.size())) ||
       (rc = upload(&s->d_scenes, scn.data(), scn.size()))) {
     free_scene(s);
     delete s;
@@ -545,6 +747,7 @@ int create_pool(const tpt_flat_scene *scenes, uint32_t n, tpt_scene **out) {
   s->simple = simple;
   s->motion = motion;
   s->media = media;
+  s->flat_of = flat_of;
   s->n_slots_of = nslots;
   s->n_leaves_of = nleaves;
   if (hipHostMalloc(reinterpret_cast<void **>(&s->host_count), NSUB * CSTRIDE * sizeof(uint32_t), hipHostMallocDefault) !=
@@ -802,8 +1005,8 @@ void launch_paths(const bounce_launch &B, hipStream_t st, uint32_t grid) {
 template <bool COUNT>
 void launch_trace_t(const bounce_launch &B, hipStream_t st, uint32_t parity) {
   const dim3 g(B.grid), b(TRACE_THREADS);
-  if (B.sweep)
-    hipLaunchKernelGGL((k_trace<true, false, false, false, COUNT>), g, b, 0, st, B.S, B.S.slots, B.S.entries, B.P,
+  if (B.sweep && !COUNT)
+    hipLaunchKernelGGL((k_trace<true, false, false, false, false>), g, b, 0, st, B.S, B.S.slots, B.S.entries, B.P,
                        B.Q, parity);
   else if (B.multi && B.P.media)
     hipLaunchKernelGGL((k_trace<false, true, false, true, COUNT>), g, b, 0, st, B.S, B.S.slots, B.S.entries, B.P,
