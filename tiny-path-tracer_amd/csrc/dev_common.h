@@ -62,6 +62,29 @@ struct flat_group {
   float p[TPT_XFORM_MAX_OPS][3];
 };
 
+// The tree of a sphere-only scene (walk_bvh.h).  A node holds both children's
+// boxes, b[axis] = (low, high of child 0, low, high of child 1), and their
+// references: a node, or kBvhLeaf | leaf.  A leaf: the sphere, its parent box
+// in the reference's tree (infinite: none), its slot, and its rank among equal t.
+constexpr uint32_t kBvhLeaf = 0x80000000u, kBvhNone = 0xFFFFFFFFu;
+constexpr uint32_t kBvhDepth = 24;  // most levels of nodes (2^24 spheres fit a balanced one)
+constexpr float kWalkBigRadius = 2.0f;  // spheres above it are tested by every ray
+constexpr float kBvhPad = 5.6e-7f;  // 1.25 * 7.5 u
+struct bvh_node {
+  float b[3][4];
+  uint32_t ref[2], pad[2];
+};
+struct bvh_leaf {
+  float c[3], r, lo[3], hi[3];
+  uint32_t slot, rank;
+};
+struct bvh_scene {
+  float lo[3], hi[3];  // bounds of the spheres in the tree
+  float pad, mag;      // kBvhPad over their smallest radius; the largest coordinate magnitude
+  uint32_t root, big0, n_big;  // big spheres: leaves [big0, big0 + n_big)
+  uint32_t multi, ready, unused[3];  // more than one segment; a tree was built
+};
+
 // Read-only scene arrays on the device (all in HBM; the hot ones are small
 // enough to stay L2-resident for the benchmark scenes).
 struct scene_view {
@@ -82,6 +105,9 @@ struct scene_view {
   uint32_t n_fgroups, n_flat;  // 0: no uniform pass
   uint32_t flat_nan;   // record of the last rect in the reference's order, or ~0u
   float flat_mag;      // largest coordinate magnitude of its primitives and wrappers
+  const bvh_node *bvh_nodes;  // sphere-only scenes
+  const bvh_leaf *bvh_leaves;
+  const bvh_scene *bvh;  // this scene's
   uint32_t n_slots, n_segments, n_lights, light_mode;
   float walk_ulp;  // 2^-22 x the largest coordinate magnitude of the scene (sphere-only walk bound)
 };

@@ -65,6 +65,7 @@ k_paths(scene_view S, const tpt_slot *__restrict__ slots, const tpt_entry *__res
   const pass_hdr H = *P.hdr;
   // the wave's generated camera rays that no lane has taken yet: o, d, pixel, sample, entry
   __shared__ float pool[PATH_WAVES][9][64];
+  __shared__ uint32_t bstack[SPH ? kBvhDepth * PATH_THREADS : 1];  // sphere_world's
   const uint32_t wave = threadIdx.x / 64, lane = __lane_id();
   float(*mine)[64] = pool[wave];
   uint32_t pool_at = 0, pool_n = 0;  // wave-uniform
@@ -123,8 +124,14 @@ k_paths(scene_view S, const tpt_slot *__restrict__ slots, const tpt_entry *__res
     hit_t h{0.0f, kNone, kNone, 0};
     const ray_ctx rc = !SIMPLE && !SWEEP && !SPH && (P.motion | P.media) && live ? make_ray_ctx(P, c, p.depth)
                                                                                  : ray_ctx{0.0f, 0u, 0u, 0u, 0u, 0u};
-    const bool got = SWEEP ? small_world(Sj, p.o, p.d, rc, 0.001f, kFltMax, &h, &st[ST_NODES], live)
-                           : trace_world<false, SPH, MEDIA>(Sj, p.o, p.d, rc, 0.001f, kFltMax, &h, &st[ST_NODES], live);
+    bool got;
+    if (SWEEP)
+      got = small_world(Sj, p.o, p.d, rc, 0.001f, kFltMax, &h, &st[ST_NODES], live);
+    else if (SPH)
+      got = sphere_world<!MULTI, PATH_THREADS>(Sj, p.o, p.d, rc, 0.001f, kFltMax, live, bstack + threadIdx.x, &h,
+                                               &st[ST_NODES]);
+    else
+      got = trace_world<false, MEDIA>(Sj, p.o, p.d, rc, 0.001f, kFltMax, &h, &st[ST_NODES], live);
     if (live) {
       ++st[ST_SEGMENTS];
       uint32_t cls = Q_TERMINAL;

@@ -30,6 +30,7 @@
 
 #include "guide.h"
 #include "shade.h"
+#include "walk_bvh.h"
 #include "walk_flat.h"
 
 #pragma clang fp contract(off)
@@ -169,6 +170,7 @@ __device__ __forceinline__ scene_view view_of(const scene_view &S, const render_
   v.n_lights = sc.n_lights;
   v.light_mode = sc.light_mode;
   v.walk_ulp = sc.walk_ulp;
+  v.bvh = S.bvh + P.jobs[job].scene;
   return v;
 }
 
@@ -470,6 +472,7 @@ __global__ void __launch_bounds__(TRACE_THREADS) __attribute__((amdgpu_waves_per
   // the general walk spills 2-11 instead of 6-13 VGPRs (no change in time on
   // box_list).
   __shared__ float4 stash[3 * TRACE_THREADS];
+  __shared__ uint32_t bstack[SPH && !COUNT ? kBvhDepth * TRACE_THREADS : 1];  // sphere_world's
   for (uint32_t base = blockIdx.x * blockDim.x; base < count; base += stride) {
     const uint32_t qi = base + threadIdx.x;
     const bool valid = qi < count;
@@ -509,24 +512,13 @@ __global__ void __launch_bounds__(TRACE_THREADS) __attribute__((amdgpu_waves_per
                            : ray_ctx{0.0f, 0u, 0u, 0u, 0u, 0u};
     op_counts oc;
     bool got;
-    if (SPH) {
-      // A wave of camera rays of one job walks nearly the same slots (about
-      // the longest lane's walk in all): it sweeps the tree together, with
-      // scalar slot loads and no divergence on the slot kind.
-      const unsigned long long vm = __ballot(valid);
-      const int first = vm ? __ffsll(static_cast<long long>(vm)) - 1 : 0;
-      const uint32_t job_u = __builtin_amdgcn_readlane(job, first);
-      const bool same = !valid || (depth == 0 && job == job_u);
-      if (vm != 0ull && __ballot(!same) == 0ull)
-        got = trace_world<true, SPH, false>(view_of<MULTI>(S, P, job_u), v3{a.x, a.y, a.z}, v3{b.x, b.y, b.z}, rc,
-                                            0.001f, kFltMax, &h, &st[ST_NODES], valid, COUNT ? &oc : nullptr);
-      else
-        got = trace_world<false, SPH, MEDIA>(Sj, v3{a.x, a.y, a.z}, v3{b.x, b.y, b.z}, rc, 0.001f, kFltMax, &h,
-                                             &st[ST_NODES], valid, COUNT ? &oc : nullptr);
+    if (SPH && !COUNT) {
+      got = sphere_world<!MULTI, TRACE_THREADS>(Sj, v3{a.x, a.y, a.z}, v3{b.x, b.y, b.z}, rc, 0.001f, kFltMax, valid,
+                                                bstack + threadIdx.x, &h, &st[ST_NODES]);
     } else if (SWEEP) {
       got = small_world(Sj, v3{a.x, a.y, a.z}, v3{b.x, b.y, b.z}, rc, 0.001f, kFltMax, &h, &st[ST_NODES], valid);
     } else {
-      got = trace_world<false, SPH, MEDIA>(Sj, v3{a.x, a.y, a.z}, v3{b.x, b.y, b.z}, rc, 0.001f, kFltMax, &h,
+      got = trace_world<SPH, MEDIA>(Sj, v3{a.x, a.y, a.z}, v3{b.x, b.y, b.z}, rc, 0.001f, kFltMax, &h,
                                            &st[ST_NODES], valid, COUNT ? &oc : nullptr);
     }
     {
@@ -1017,11 +1009,12 @@ __global__ void __launch_bounds__(256) k_tail(scene_view S, const tpt_slot *__re
                                               const tpt_entry *__restrict__ entries, render_params P,
                                               render_state Q, uint32_t parity) {
   static_assert(!(SWEEP && MULTI), "the wave-uniform sweep needs one scene");
-  static_assert(!(SWEEP && SPH), "the sweep takes every leaf kind");
+  static_assert(SWEEP != SPH, "small scenes or sphere-only ones");
   S.slots = slots;
   S.entries = entries;
   __shared__ uint32_t offs[NSUB];
   __shared__ uint32_t pre[NSUB + 1];
+  __shared__ uint32_t bstack[SPH ? kBvhDepth * 256 : 1];  // sphere_world's
   if (threadIdx.x < NSUB) offs[threadIdx.x] = rc_at(parity, threadIdx.x);
   __syncthreads();
   region_prefix(Q.counters, offs, NSUB, pre);
@@ -1046,7 +1039,8 @@ __global__ void __launch_bounds__(256) k_tail(scene_view S, const tpt_slot *__re
       hit_t h{0.0f, kNone, kNone, 0};
       const ray_ctx rc{0.0f, 0u, 0u, 0u, 0u, 0u};
       const bool got = SWEEP ? small_world(Sj, p.o, p.d, rc, 0.001f, kFltMax, &h, &st[ST_NODES], live)
-                             : trace_world<false, SPH, false>(Sj, p.o, p.d, rc, 0.001f, kFltMax, &h, &st[ST_NODES], live);
+                             : sphere_world<!MULTI, 256>(Sj, p.o, p.d, rc, 0.001f, kFltMax, live, bstack + threadIdx.x,
+                                                         &h, &st[ST_NODES]);
       uint32_t cls = Q_TERMINAL;
       if (live) {
         ++st[ST_SEGMENTS];

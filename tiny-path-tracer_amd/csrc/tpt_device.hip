@@ -11,6 +11,7 @@
 #include <vector>
 
 #include "../host/errors.h"
+#include "bvh_build.h"
 #include "guide_train.h"
 #include "paths.h"
 #include "render.h"
@@ -46,8 +47,14 @@ __global__ void __launch_bounds__(256) k_trace_closest(scene_view S, const tpt_s
   }
   hit_t h;
   uint32_t nodes = 0, id = 0;
-  const bool got = SWEEP ? small_world<true>(S, o, d, rc, tmin, tmax, &h, &nodes, live, &id)
-                         : trace_world<false, SPH, MEDIA>(S, o, d, rc, tmin, tmax, &h, &nodes, live);
+  __shared__ uint32_t bstack[SPH ? kBvhDepth * 256 : 1];  // sphere_world's
+  bool got;
+  if (SWEEP)
+    got = small_world<true>(S, o, d, rc, tmin, tmax, &h, &nodes, live, &id);
+  else if (SPH)
+    got = sphere_world<true, 256>(S, o, d, rc, tmin, tmax, live, bstack + threadIdx.x, &h, &nodes);
+  else
+    got = trace_world<false, MEDIA>(S, o, d, rc, tmin, tmax, &h, &nodes, live);
   if (!live) return;
   if (got) {
     leaf[i] = static_cast<int32_t>(SWEEP ? id : leaf_id(S, h));
@@ -121,6 +128,9 @@ struct tpt_scene {
   flat_scan *flat = nullptr;   // records of the uniform pass (walk_flat.h) of the small scenes
   flat_win *fwins = nullptr;
   flat_group *fgroups = nullptr;
+  bvh_node *bvh_nodes = nullptr;  // trees of the sphere-only scenes (walk_bvh.h)
+  bvh_leaf *bvh_leaves = nullptr;
+  bvh_scene *bvh = nullptr;  // per scene
   uint32_t n_slots = 0, n_segments = 0, n_lights = 0;
   // the pool's scenes
   std::vector<scene_dev> scn;
@@ -179,6 +189,9 @@ struct tpt_scene {
     v.n_flat = flat_of[k].n_scans;
     v.flat_nan = flat_of[k].nan_win;
     v.flat_mag = flat_of[k].mag;
+    v.bvh_nodes = bvh_nodes;
+    v.bvh_leaves = bvh_leaves;
+    v.bvh = bvh + k;
     v.n_slots = n_slots;
     v.n_segments = scn[k].n_seg;
     v.n_lights = scn[k].n_lights;
@@ -215,6 +228,9 @@ void free_scene(tpt_scene *s) {
   (void)hipFree(s->flat);
   (void)hipFree(s->fwins);
   (void)hipFree(s->fgroups);
+  (void)hipFree(s->bvh_nodes);
+  (void)hipFree(s->bvh_leaves);
+  (void)hipFree(s->bvh);
   (void)hipFree(s->d_scenes);
   (void)hipFree(s->state);
   (void)hipFree(s->d_jobs);
@@ -605,6 +621,9 @@ int create_pool(const tpt_flat_scene *scenes, uint32_t n, tpt_scene **out) {
   std::vector<flat_win> fwins;
   std::vector<flat_group> fgroups;
   std::vector<flat_range> flat_of(n);
+  std::vector<bvh_node> bnodes;
+  std::vector<bvh_leaf> bleaves;
+  std::vector<bvh_scene> bscn(n);
   for (uint32_t k = 0; k < n; ++k) {
     const tpt_flat_scene &f = scenes[k];
     const uint64_t sb = slots.size(), eb = entries.size(), xb = xforms.size(), mb = materials.size(),
@@ -707,6 +726,8 @@ int create_pool(const tpt_flat_scene *scenes, uint32_t n, tpt_scene **out) {
       sweep[k] = flat_of[k].n_groups > 0;
     }
     if (wrapped) sph[k] = 0;  // the sphere-only walk is built without segment transforms
+    std::memset(&bscn[k], 0, sizeof(bscn[k]));
+    if (sph[k]) bscn[k] = build_bvh(f, static_cast<uint32_t>(sb), &bnodes, &bleaves);
     simple[k] = !motion[k] && !media[k] &&
                 (f.n_lights == 0 || (f.light_mode == 0 && f.lights[0].kind == TPT_LIGHT_XZ_RECT));
     for (uint32_t t = 0; t < f.n_textures; ++t) simple[k] = simple[k] && f.textures[t].kind == TPT_TEX_CONSTANT;
@@ -733,6 +754,9 @@ int create_pool(const tpt_flat_scene *scenes, uint32_t n, tpt_scene **out) {
       (rc = upload(&s->flat, flat.data(), flat.size())) ||
       (rc = upload(&s->fwins, fwins.data(), fwins.size())) ||
       (rc = upload(&s->fgroups, fgroups.data(), fgroups.size())) ||
+      (rc = upload(&s->bvh_nodes, bnodes.data(), bnodes.size())) ||
+      (rc = upload(&s->bvh_leaves, bleaves.data(), bleaves.size())) ||
+      (rc = upload(&s->bvh, bscn.data(), bscn.size())) ||
       (rc = upload(&s->d_scenes, scn.data(), scn.size()))) {
     free_scene(s);
     delete s;

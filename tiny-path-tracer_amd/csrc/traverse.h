@@ -36,9 +36,8 @@ namespace tptd {
 constexpr uint32_t kNone = 0xFFFFFFFFu;
 constexpr float kFltMaxT = 3.402823466e38f;  // std::numeric_limits<float>::max()
 // Sphere-only walk: a box whose subtree holds a sphere of radius above
-// kWalkBigRadius has kBoxUnbounded set in its skip word (device copy only;
+// kWalkBigRadius (dev_common.h) has kBoxUnbounded set in its skip word (device copy only;
 // skip links are below 2^28) and is always tested against t_max.
-constexpr float kWalkBigRadius = 2.0f;
 constexpr uint32_t kBoxUnbounded = 0x80000000u;
 
 struct hit_t {
@@ -466,75 +465,11 @@ __device__ __forceinline__ bool segment_fast(const scene_view &S, uint32_t start
   return have;
 }
 
-// Smallest value over the active lanes of the wave (the device library's
-// wavefront reduction, DPP moves instead of LDS permutes).
-__device__ __forceinline__ uint32_t wave_min(uint32_t v) { return __ockl_wfred_min_u32(v); }
-
-// Wave-uniform sweep of one segment, for small scenes: the wave steps through
-// the slots together, always at the smallest slot some lane still has to
-// visit; a lane acts only on the slot equal to its own next pre-order slot.
-// Each lane therefore evaluates exactly the slots of its own pre-order walk,
-// in the same order (same results as segment_fast), while the slot index is
-// wave-uniform: slot data comes through scalar loads and the branch on the
-// slot kind does not diverge.  Lanes with `live` false take no part.
-// Must be called by all lanes of the wave together.  SPH: a sphere-only
-// scene, each lane's boxes bounded by its own held hit as in segment_fast
-// (the sweep then serves large trees for rays whose walks mostly coincide,
-// such as one wave's camera rays).
-template <bool SPH = false>
-__device__ __forceinline__ bool segment_sweep(const scene_view &S, uint32_t start, uint32_t end, bool live, v3 o, v3 d,
-                                              v3 inv, const ray_ctx &rc, float tmin, float tmax, hit_t *out,
-                                              bool *saw_nan, uint32_t *nodes, op_counts *oc = nullptr) {
-  bool have = false;
-  hit_t best{0.0f, kNone, kNone, 0};
-  uint32_t next = live ? start : end;
-  uint32_t visited = 0;
-  float bound = tmax;
-  float reach = 0.0f;
-  if (SPH)
-    reach = 0.015625f * kWalkBigRadius * rsqrtf(d.x * d.x + d.y * d.y + d.z * d.z) +
-            S.walk_ulp * fmaxf(fmaxf(fabsf(inv.x), fabsf(inv.y)), fabsf(inv.z));
-  uint32_t i = __builtin_amdgcn_readfirstlane(wave_min(next));
-  while (i < end) {
-    const slot_t s = load_slot(&S.slots[i]);
-    const uint32_t kind = s.b >> 28;
-    const bool mine = next == i;
-    if (mine) {
-      ++visited;
-      if (kind == TPT_SLOT_BOX) {
-        if (oc) ++oc->box;
-        const bool unbounded = !SPH || (s.a & kBoxUnbounded);
-        next = slab_nn(s, o, inv, tmin, unbounded ? tmax : bound) ? i + 1 : (s.a & TPT_PAYLOAD_MASK);
-      } else {
-        float t;
-        uint32_t entry, mat;
-        if (leaf_t<SPH>(S, s, kind, o, d, rc, tmin, tmax, &t, &entry, &mat, oc)) {
-          if (t != t) *saw_nan = true;
-          if (!have || t <= best.t) {
-            best = hit_t{t, i, entry, mat};
-            have = true;
-            if (SPH) bound = sphere_walk_bound(t, tmin, tmax, reach);
-          }
-        }
-        next = i + 1;
-      }
-    }
-    // Next slot: i + 1 when any lane goes there (the common case), else the
-    // smallest pending skip target.
-    const bool step = __ballot(next == i + 1) != 0ull;
-    i = step ? i + 1 : __builtin_amdgcn_readfirstlane(wave_min(next));
-  }
-  *nodes += visited;
-  if (have) *out = best;
-  return have;
-}
-
 // World = segments evaluated like a hitable_list (t_max shrinks between them).
-// SWEEP selects segment_sweep (all lanes of the wave must call together).  A
-// NaN bound (a caller's t_min, or t_max after a segment whose winner had a
+// A NaN bound (a caller's t_min, or t_max after a segment whose winner had a
 // NaN t) sends the segment to segment_exact, which keeps the reference's slab
 // updates verbatim.
-template <bool SWEEP = false, bool SPH = false, bool MEDIA = false>
+template <bool SPH = false, bool MEDIA = false>
 __device__ __forceinline__ bool trace_world(const scene_view &S, v3 o, v3 d, const ray_ctx &rc, float tmin, float tmax,
                                             hit_t *out, uint32_t *nodes, bool live = true, op_counts *oc = nullptr) {
   const v3 inv0{1.0f / d.x, 1.0f / d.y, 1.0f / d.z};
@@ -548,10 +483,10 @@ __device__ __forceinline__ bool trace_world(const scene_view &S, v3 o, v3 d, con
     if (start >= end) continue;
     // a bvh_node seen through translate / rotate_y: its walk takes the ray
     // those wrappers hand down (headers/rect_box.h:87-95, src/rect_box.cc:171-180);
-    // scenes with such segments use neither the sweep nor the sphere-only walk
+    // scenes with such segments do not use the sphere-only walk
     o = o0, d = d0;
     v3 inv = inv0;
-    const uint32_t sx = !SWEEP && !SPH && S.seg_xf ? S.seg_xf[g] : TPT_SEGMENT_PLAIN;
+    const uint32_t sx = !SPH && S.seg_xf ? S.seg_xf[g] : TPT_SEGMENT_PLAIN;
     if ((sx & TPT_SEGMENT_PLAIN) != TPT_SEGMENT_PLAIN) {
       to_local(S.xforms[sx & TPT_SEGMENT_PLAIN], &o, &d);
       if (oc) ++oc->xform;
@@ -559,13 +494,9 @@ __device__ __forceinline__ bool trace_world(const scene_view &S, v3 o, v3 d, con
     }
     const bool bounded = tmin == tmin && cur == cur;
     bool got = false;
-    if (SWEEP) {
-      got = segment_sweep<SPH>(S, start, end, live && bounded, o, d, inv, rc, tmin, cur, &h, &saw_nan, nodes, oc);
-    } else {
-      if (!live) continue;
-      if (bounded) got = segment_fast<SPH, MEDIA>(S, start, end, o, d, inv, rc, tmin, cur, &h, &saw_nan, nodes, oc);
-    }
-    if (live && (saw_nan || !bounded)) got = segment_exact<SPH, MEDIA>(S, start, o, d, inv, rc, tmin, cur, &h);
+    if (!live) continue;
+    if (bounded) got = segment_fast<SPH, MEDIA>(S, start, end, o, d, inv, rc, tmin, cur, &h, &saw_nan, nodes, oc);
+    if (saw_nan || !bounded) got = segment_exact<SPH, MEDIA>(S, start, o, d, inv, rc, tmin, cur, &h);
     if (got) {
       *out = h;
       cur = h.t;
