@@ -85,19 +85,54 @@ __global__ void __launch_bounds__(256) k_trace_closest(scene_view S, const tpt_s
     if (e_ != hipSuccess) return tpt::fail(TPT_ERR_HIP, std::string(#expr) + ": " + hipGetErrorString(e_)); \
   } while (0)
 
-template <class T>
-int upload(T **dst, const T *src, size_t n) {
-  *dst = nullptr;
-  if (n == 0) return TPT_OK;
-  HIP_TRY(hipMalloc(reinterpret_cast<void **>(dst), n * sizeof(T)));
-  HIP_TRY(hipMemcpy(*dst, src, n * sizeof(T), hipMemcpyHostToDevice));
-  return TPT_OK;
-}
+// Host arrays gathered into one device allocation and one copy.
+struct gather {
+  std::vector<char> bytes;
+  struct part {
+    void **dst;
+    size_t at;
+  };
+  std::vector<part> parts;
+  template <class T>
+  void add(T **dst, const std::vector<T> &v, bool used = true) {
+    *dst = nullptr;
+    if (v.empty() || !used) return;
+    const size_t at = (bytes.size() + 255) & ~size_t(255), n = v.size() * sizeof(T);
+    bytes.resize(at + n);
+    std::memcpy(bytes.data() + at, v.data(), n);
+    parts.push_back(part{reinterpret_cast<void **>(dst), at});
+  }
+  int upload(char **blob) {
+    *blob = nullptr;
+    if (bytes.empty()) return TPT_OK;
+    HIP_TRY(hipMalloc(reinterpret_cast<void **>(blob), bytes.size()));
+    HIP_TRY(hipMemcpy(*blob, bytes.data(), bytes.size(), hipMemcpyHostToDevice));
+    for (const part &p : parts) *p.dst = *blob + p.at;
+    return TPT_OK;
+  }
+};
 
-bool is_gfx950(int dev) {
-  hipDeviceProp_t prop;
-  if (hipGetDeviceProperties(&prop, dev) != hipSuccess) return false;
-  return std::strncmp(prop.gcnArchName, "gfx950", 6) == 0;
+// What does not change about a device, asked once (the query takes longer than
+// a small scene's upload).
+struct device_info {
+  bool known = false, gfx950 = false;
+  int n_cu = 256;
+};
+device_info info_of(int dev) {
+  static std::mutex mu;
+  static std::vector<device_info> seen;
+  std::lock_guard<std::mutex> lock(mu);
+  if (dev < 0) return device_info();
+  if (seen.size() <= static_cast<size_t>(dev)) seen.resize(dev + 1);
+  device_info &d = seen[dev];
+  if (!d.known) {
+    hipDeviceProp_t prop;
+    if (hipGetDeviceProperties(&prop, dev) != hipSuccess) return device_info();
+    d.gfx950 = std::strncmp(prop.gcnArchName, "gfx950", 6) == 0;
+    d.n_cu = prop.multiProcessorCount;
+    d.known = true;
+  }
+  return d;
 }
 
 }  // namespace
@@ -114,6 +149,7 @@ struct flat_range {
 struct tpt_scene {
   int device = 0;
   int n_cu = 256;
+  char *arrays = nullptr;  // one allocation for every scene array below
   tpt_slot *slots = nullptr;
   uint32_t *segments = nullptr;
   tpt_entry *entries = nullptr;
@@ -214,24 +250,7 @@ struct tpt_scene {
 namespace {
 
 void free_scene(tpt_scene *s) {
-  (void)hipFree(s->slots);
-  (void)hipFree(s->segments);
-  (void)hipFree(s->entries);
-  (void)hipFree(s->xforms);
-  (void)hipFree(s->materials);
-  (void)hipFree(s->textures);
-  (void)hipFree(s->texels);
-  (void)hipFree(s->perlin);
-  (void)hipFree(s->lights);
-  (void)hipFree(s->motions);
-  (void)hipFree(s->seg_xf);
-  (void)hipFree(s->flat);
-  (void)hipFree(s->fwins);
-  (void)hipFree(s->fgroups);
-  (void)hipFree(s->bvh_nodes);
-  (void)hipFree(s->bvh_leaves);
-  (void)hipFree(s->bvh);
-  (void)hipFree(s->d_scenes);
+  (void)hipFree(s->arrays);
   (void)hipFree(s->state);
   (void)hipFree(s->d_jobs);
   (void)hipFree(s->d_hdr);
@@ -633,6 +652,7 @@ int create_pool(const tpt_flat_scene *scenes, uint32_t n, tpt_scene **out) {
         eb + f.n_entries > 0xFFFFFFF0ull)
       return tpt::fail(TPT_ERR_INVALID, "tpt_scene_create: pool too large for 32-bit indices");
     sph[k] = 1;
+    slots.reserve(sb + f.n_slots);
     for (uint32_t i = 0; i < f.n_slots; ++i) {
       tpt_slot s = f.slots[i];
       const uint32_t kind = s.b >> 28;
@@ -735,29 +755,31 @@ int create_pool(const tpt_flat_scene *scenes, uint32_t n, tpt_scene **out) {
     nleaves[k] = f.n_leaves;
   }
   if (tpt_device_count() < 1) return tpt::fail(TPT_ERR_NODEVICE, "tpt_scene_create: no gfx950 device");
+  int dev = 0, rc = TPT_OK;
+  HIP_TRY(hipGetDevice(&dev));
   auto *s = new tpt_scene();
-  int rc = TPT_OK;
-  HIP_TRY(hipGetDevice(&s->device));
-  hipDeviceProp_t prop;
-  if (hipGetDeviceProperties(&prop, s->device) == hipSuccess) s->n_cu = prop.multiProcessorCount;
-  if ((rc = upload(&s->slots, slots.data(), slots.size())) ||
-      (rc = upload(&s->segments, segments.data(), segments.size())) ||
-      (rc = upload(&s->entries, entries.data(), entries.size())) ||
-      (rc = upload(&s->xforms, xforms.data(), xforms.size())) ||
-      (rc = upload(&s->materials, materials.data(), materials.size())) ||
-      (rc = upload(&s->textures, textures.data(), textures.size())) ||
-      (rc = upload(&s->texels, texels.data(), texels.size())) ||
-      (rc = upload(&s->perlin, perlin.data(), perlin.size())) ||
-      (rc = upload(&s->lights, lights.data(), lights.size())) ||
-      (rc = upload(&s->motions, motions.data(), motions.size())) ||
-      (rc = upload(&s->seg_xf, seg_xf.data(), any_wrapped ? seg_xf.size() : 0)) ||
-      (rc = upload(&s->flat, flat.data(), flat.size())) ||
-      (rc = upload(&s->fwins, fwins.data(), fwins.size())) ||
-      (rc = upload(&s->fgroups, fgroups.data(), fgroups.size())) ||
-      (rc = upload(&s->bvh_nodes, bnodes.data(), bnodes.size())) ||
-      (rc = upload(&s->bvh_leaves, bleaves.data(), bleaves.size())) ||
-      (rc = upload(&s->bvh, bscn.data(), bscn.size())) ||
-      (rc = upload(&s->d_scenes, scn.data(), scn.size()))) {
+  s->device = dev;
+  s->n_cu = info_of(s->device).n_cu;
+  gather G;
+  G.add(&s->slots, slots);
+  G.add(&s->segments, segments);
+  G.add(&s->entries, entries);
+  G.add(&s->xforms, xforms);
+  G.add(&s->materials, materials);
+  G.add(&s->textures, textures);
+  G.add(&s->texels, texels);
+  G.add(&s->perlin, perlin);
+  G.add(&s->lights, lights);
+  G.add(&s->motions, motions);
+  G.add(&s->seg_xf, seg_xf, any_wrapped);
+  G.add(&s->flat, flat);
+  G.add(&s->fwins, fwins);
+  G.add(&s->fgroups, fgroups);
+  G.add(&s->bvh_nodes, bnodes);
+  G.add(&s->bvh_leaves, bleaves);
+  G.add(&s->bvh, bscn);
+  G.add(&s->d_scenes, scn);
+  if ((rc = G.upload(&s->arrays)) != TPT_OK) {
     free_scene(s);
     delete s;
     return rc;
@@ -840,7 +862,7 @@ int tpt_device_count(void) {
   int n = 0;
   if (hipGetDeviceCount(&n) != hipSuccess) return 0;
   int good = 0;
-  for (int d = 0; d < n; ++d) good += is_gfx950(d) ? 1 : 0;
+  for (int d = 0; d < n; ++d) good += info_of(d).gfx950 ? 1 : 0;
   return good;
 }
 
@@ -2044,8 +2066,7 @@ int tpt_guide_create(uint64_t seed, tpt_guide **out) {
   }
   auto *g = new tpt_guide();
   HIP_TRY(hipGetDevice(&g->device));
-  hipDeviceProp_t prop;
-  if (hipGetDeviceProperties(&prop, g->device) == hipSuccess) g->n_cu = prop.multiProcessorCount;
+  g->n_cu = info_of(g->device).n_cu;
   g->train_blocks = g->n_cu;
   const size_t np = G_NPARAM_PAD + 1;
   HIP_TRY(hipMalloc(&g->params, np * sizeof(float)));

@@ -15,6 +15,7 @@
 #include <limits>
 #include <random>
 #include <stdexcept>
+#include <vector>
 
 #include "../scene/camera.h"
 #include "../scene/hitable.h"
@@ -59,22 +60,33 @@ namespace {
 // Orders hitables by their box's lower corner on one axis.  Same predicate as
 // the reference's box_axis_compare (src/hitable.cc:10-30): "a before b" unless
 // isgreaterequal(a.min[axis], b.min[axis]); boxes are queried at time (0,0).
-struct lower_corner_before {
-  int axis;
-  bool operator()(const hitable *a, const hitable *b) const {
-    AABB ba, bb;
-    const bool ok_a = a->bounding_box(0, 0, ba);
-    const bool ok_b = b->bounding_box(0, 0, bb);
-    if (!ok_a || !ok_b) throw std::runtime_error("bvh_node: a child has no bounding box");
-    return !std::isgreaterequal(ba.min_.e[axis], bb.min_.e[axis]);
-  }
+// The corners are taken once per node instead of in every comparison (the
+// same comparisons in the same order, so the same permutation).
+struct keyed {
+  float key;
+  hitable *h;
 };
+struct lower_corner_before {
+  bool operator()(const keyed &a, const keyed &b) const { return !std::isgreaterequal(a.key, b.key); }
+};
+
+void sort_by_corner(hitable **l, int n, int axis) {
+  if (n < 2) return;
+  std::vector<keyed> k(n);
+  for (int i = 0; i < n; ++i) {
+    AABB b;
+    if (!l[i]->bounding_box(0, 0, b)) throw std::runtime_error("bvh_node: a child has no bounding box");
+    k[i] = keyed{b.min_.e[axis], l[i]};
+  }
+  std::sort(k.begin(), k.end(), lower_corner_before());
+  for (int i = 0; i < n; ++i) l[i] = k[i].h;
+}
 }  // namespace
 
 bvh_node::bvh_node(hitable **l, int n, float time0, float time1) {
   // The axis draw precedes the sort and the child builds (pre-order draws).
   const int axis = static_cast<int>(drand_r(0, 3.0));
-  std::sort(l, l + n, lower_corner_before{axis < 0 ? 0 : (axis > 2 ? 2 : axis)});
+  sort_by_corner(l, n, axis < 0 ? 0 : (axis > 2 ? 2 : axis));
   if (n == 1) {
     left_ = right_ = l[0];
   } else if (n == 2) {
