@@ -159,40 +159,63 @@ __device__ __forceinline__ bf16x8 relu_bf16x8(bf16x8 v) {
   return __builtin_bit_cast(bf16x8, __builtin_elementwise_max(x, s16x8{0, 0, 0, 0, 0, 0, 0, 0}));
 }
 
-// Forward pass of 16 samples (one per lane column l%16) in the 16x16x32
-// layout: xb = this lane's first-layer B operands, xt = LDS inference tiles,
-// bias = LDS biases.  out[mt][r] = output 16 mt + 4 (l/16) + r.  The
-// accumulators start at the biases (no separate bias add).
-__device__ __forceinline__ void guide_forward_x32(const bf16x8 xb_in[2], const uint32_t *xt, const float *bias,
-                                                  f32x4 out[3]) {
+// Forward pass of NB groups of 16 samples (one per lane column l%16) in the
+// 16x16x32 layout: xb[g] = this lane's first-layer B operands of group g, xt =
+// LDS inference tiles, bias = LDS biases.  out[g][mt][r] = output 16 mt + 4
+// (l/16) + r.  The accumulators start at the biases (no separate bias add).
+// Every weight tile read from LDS serves all NB groups.
+template <int NB>
+__device__ __forceinline__ void guide_forward_groups(bf16x8 xb[NB][2], const uint32_t *xt, const float *bias,
+                                                     f32x4 out[NB][3]) {
   const int l = __lane_id();
   const int fg = l >> 4;
   const bf16x8 *tiles = reinterpret_cast<const bf16x8 *>(xt);
   const f32x4 *bias4 = reinterpret_cast<const f32x4 *>(bias);  // bias4[4 t + fg]: rows 16 t + 4 fg .. + 3
-  bf16x8 xb[2] = {xb_in[0], xb_in[1]};
 #pragma unroll
   for (int layer = 0; layer < 3; ++layer) {
-    f32x4 acc[4];
+    f32x4 acc[NB][4];
 #pragma unroll
     for (int mt = 0; mt < 4; ++mt) {
-      acc[mt] = bias4[4 * (4 * layer + mt) + fg];
+      const f32x4 b = bias4[4 * (4 * layer + mt) + fg];
 #pragma unroll
-      for (int s = 0; s < 2; ++s)
-        acc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(tiles[(GX_BASE[layer] + 2 * mt + s) * 64 + l], xb[s],
-                                                          acc[mt], 0, 0, 0);
+      for (int g = 0; g < NB; ++g) acc[g][mt] = b;
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        const bf16x8 w = tiles[(GX_BASE[layer] + 2 * mt + s) * 64 + l];
+#pragma unroll
+        for (int g = 0; g < NB; ++g)
+          acc[g][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, xb[g][s], acc[g][mt], 0, 0, 0);
+      }
     }
-    xb[0] = relu_bf16x8(pack8(acc[0], acc[1]));
-    xb[1] = relu_bf16x8(pack8(acc[2], acc[3]));
+#pragma unroll
+    for (int g = 0; g < NB; ++g) {
+      xb[g][0] = relu_bf16x8(pack8(acc[g][0], acc[g][1]));
+      xb[g][1] = relu_bf16x8(pack8(acc[g][2], acc[g][3]));
+    }
     __builtin_amdgcn_sched_barrier(0);
   }
 #pragma unroll
   for (int mt = 0; mt < 3; ++mt) {
-    out[mt] = bias4[4 * (12 + mt) + fg];
+    const f32x4 b = bias4[4 * (12 + mt) + fg];
 #pragma unroll
-    for (int s = 0; s < 2; ++s)
-      out[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(tiles[(GX_BASE[3] + 2 * mt + s) * 64 + l], xb[s], out[mt], 0,
-                                                        0, 0);
+    for (int g = 0; g < NB; ++g) out[g][mt] = b;
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      const bf16x8 w = tiles[(GX_BASE[3] + 2 * mt + s) * 64 + l];
+#pragma unroll
+      for (int g = 0; g < NB; ++g)
+        out[g][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, xb[g][s], out[g][mt], 0, 0, 0);
+    }
   }
+}
+
+__device__ __forceinline__ void guide_forward_x32(const bf16x8 xb_in[2], const uint32_t *xt, const float *bias,
+                                                  f32x4 out[3]) {
+  bf16x8 xb[1][2] = {{xb_in[0], xb_in[1]}};
+  f32x4 o[1][3];
+  guide_forward_groups<1>(xb, xt, bias, o);
+#pragma unroll
+  for (int mt = 0; mt < 3; ++mt) out[mt] = o[0][mt];
 }
 
 // ---------------------------------------------------------------- vMF mix ---

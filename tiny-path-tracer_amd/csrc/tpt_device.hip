@@ -2135,9 +2135,16 @@ int tpt_guide_set_params(tpt_guide *g, const float *host) {
 int tpt_guide_infer(tpt_guide *g, const float *d_in, uint64_t n, float *d_out, void *stream) {
   if (!g || (n && (!d_in || !d_out))) return tpt::fail(TPT_ERR_INVALID, "tpt_guide_infer: null argument");
   if (n == 0) return TPT_OK;
-  const uint32_t blocks = static_cast<uint32_t>(std::min<uint64_t>((n + 63) / 64, static_cast<uint64_t>(g->n_cu) * 8));
-  hipLaunchKernelGGL(k_guide_infer, dim3(blocks), dim3(256), 0, static_cast<hipStream_t>(stream), g->xtiles,
-                     g->params, d_in, n, d_out);
+  // 5 blocks of 31 KB LDS per CU stay resident; each stages the weights once
+  const uint32_t blocks =
+      static_cast<uint32_t>(std::min<uint64_t>((n + GI_ROWS - 1) / GI_ROWS, static_cast<uint64_t>(g->n_cu) * 5));
+  const bool vec = (reinterpret_cast<uintptr_t>(d_out) & 15u) == 0;
+  if (vec)
+    hipLaunchKernelGGL(k_guide_infer<true>, dim3(blocks), dim3(256), 0, static_cast<hipStream_t>(stream), g->xtiles,
+                       g->params, d_in, n, d_out);
+  else
+    hipLaunchKernelGGL(k_guide_infer<false>, dim3(blocks), dim3(256), 0, static_cast<hipStream_t>(stream), g->xtiles,
+                       g->params, d_in, n, d_out);
   HIP_TRY(hipGetLastError());
   return TPT_OK;
 }
