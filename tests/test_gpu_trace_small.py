@@ -8,7 +8,8 @@ import pytest
 
 pytestmark = pytest.mark.gpu
 
-SCENES = ["cornell555", "ref_cornell_box", "ref_sphere_cornell_box", "ref_light_spheres", "ref_two_perlin_spheres"]
+SCENES = ["cornell555", "ref_cornell_box", "ref_sphere_cornell_box", "ref_light_spheres", "ref_two_perlin_spheres",
+          "cornell_smoke"]
 
 
 def unit(v):

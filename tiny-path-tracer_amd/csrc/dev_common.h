@@ -39,11 +39,12 @@ __device__ __forceinline__ float comp(v3 a, uint32_t i) { return i == 0 ? a.x : 
 // bytes each, through scalar loads.  rect: plane k, in-plane centres c0, c1
 // and half-extents h0, h1.  sphere: centre (k, c0, c1), radius h0.  box (six
 // rects of one list that close a box): low corner (k, c0, c1), high corner
-// (h0, h1, x).  win: its record in flat_wins (a box: of its low x face, then
+// (h0, h1, x).  medium (bounded by a closed box): the box and its density.  win: its record in flat_wins (a box: of its low x face, then
 // high x, low y, high y, low z, high z).
 struct flat_scan {
   float k, c0, c1, h0, h1, x;
-  uint32_t win, pad;
+  uint32_t win;
+  float density;
 };
 // What its winner needs, 80 bytes.
 struct flat_win {
@@ -51,11 +52,12 @@ struct flat_win {
   uint32_t slot, entry, mat;  // as in hit_t
   float box[6];               // the innermost box around it
   uint32_t boxed;             // 0: there is none, or it is passed whenever the winner is certain
-  uint32_t xform, kind, leaf;  // wrapper chain or ~0u; TPT_SLOT_RECT or TPT_SLOT_SPHERE; leaf id
+  uint32_t xform, kind, leaf;  // wrapper chain or ~0u; TPT_SLOT_RECT, _SPHERE or _MEDIUM; leaf id
   uint32_t order, pad;         // its place in the order of segments, slots and entries
 };
 // Primitives seen through one wrapper chain, in this order: rects by normal
-// axis (counts in bits 0-7, 8-15, 16-23 of n), spheres (24-31), boxes (n_box);
+// axis (counts in bits 0-7, 8-15, 16-23 of n), spheres (24-31), boxes and
+// media (low and high half of n_box);
 // and the chain itself (nops 0: none), so that one load fetches all of it.
 struct flat_group {
   uint32_t n, n_box, nops, kinds;

@@ -51,9 +51,9 @@ __device__ __forceinline__ uint32_t claim_run(const pass_hdr &H, uint32_t *count
 
 // SWEEP, SPH, MEDIA: the walk, as for k_trace; SIMPLE: the shading, as for k_shade.
 // Waves per SIMD: 4 fit 128 VGPRs without spilling where one walk is compiled;
-// the general walk needs 3 waves' registers, the media walk 2.
+// the general walk needs 3 waves' registers, the general media walk 2.
 __host__ __device__ constexpr uint32_t path_waves(bool sweep, bool sph, bool simple, bool media) {
-  return media ? 2u : (sweep || sph || simple ? 4u : 3u);
+  return sweep || sph || (simple && !media) ? 4u : (media ? 2u : 3u);
 }
 
 template <bool SWEEP, bool MULTI, bool SPH, bool SIMPLE, bool MEDIA = false>
@@ -122,11 +122,11 @@ k_paths(scene_view S, const tpt_slot *__restrict__ slots, const tpt_entry *__res
     const item_ctx c{p.ent, job, px, smp};
     const scene_view Sj = view_of<MULTI>(S, P, job);
     hit_t h{0.0f, kNone, kNone, 0};
-    const ray_ctx rc = !SIMPLE && !SWEEP && !SPH && (P.motion | P.media) && live ? make_ray_ctx(P, c, p.depth)
+    const ray_ctx rc = (MEDIA || (!SIMPLE && !SWEEP && !SPH)) && (P.motion | P.media) && live ? make_ray_ctx(P, c, p.depth)
                                                                                  : ray_ctx{0.0f, 0u, 0u, 0u, 0u, 0u};
     bool got;
     if (SWEEP)
-      got = small_world(Sj, p.o, p.d, rc, 0.001f, kFltMax, &h, &st[ST_NODES], live);
+      got = small_world<false, MEDIA>(Sj, p.o, p.d, rc, 0.001f, kFltMax, &h, &st[ST_NODES], live);
     else if (SPH)
       got = sphere_world<!MULTI, PATH_THREADS>(Sj, p.o, p.d, rc, 0.001f, kFltMax, live, bstack + threadIdx.x, &h,
                                                &st[ST_NODES]);
@@ -141,7 +141,7 @@ k_paths(scene_view S, const tpt_slot *__restrict__ slots, const tpt_entry *__res
       } else {
         h.slot = kNone;
       }
-      if (!shade_hit<SIMPLE>(S, Sj, P, P.jobs[job], c, p, h, cls, st)) {
+      if (!shade_hit<SIMPLE, MEDIA || !SIMPLE>(S, Sj, P, P.jobs[job], c, p, h, cls, st)) {
         const pass_ent E = P.pass[MULTI ? p.ent : 0u];
         p.item = E.item_begin + (smp - E.s_begin) * P.jobs[job].n_pix + px;
         finish_sample<false>(P, Q, p, st);

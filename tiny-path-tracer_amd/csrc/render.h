@@ -448,7 +448,7 @@ __global__ void __launch_bounds__(TRACE_THREADS) __attribute__((amdgpu_waves_per
   static_assert(!(SWEEP && MULTI), "the wave-uniform sweep needs one scene");
   static_assert(!(SWEEP && SPH), "the sweep takes every leaf kind");
   static_assert(!(COUNT && SWEEP), "operations are counted in the walks of each lane");
-  static_assert(!(MEDIA && (SWEEP || SPH)), "media go through the general walk");
+  static_assert(!(MEDIA && SPH), "a sphere-only scene has no media");
   S.slots = slots;
   S.entries = entries;
   __shared__ uint32_t offs[NSUB];
@@ -507,7 +507,7 @@ __global__ void __launch_bounds__(TRACE_THREADS) __attribute__((amdgpu_waves_per
     const scene_view Sj = view_of<MULTI>(S, P, job);
     // (scenes with moving spheres or media use neither the sweep nor the
     // sphere-only walk)
-    const ray_ctx rc = !SWEEP && !SPH && (P.motion | P.media) && valid
+    const ray_ctx rc = (MEDIA || !SWEEP) && !SPH && (P.motion | P.media) && valid
                            ? make_ray_ctx(P, item_in_entry(P, ent, __float_as_uint(a.w)), depth)
                            : ray_ctx{0.0f, 0u, 0u, 0u, 0u, 0u};
     op_counts oc;
@@ -516,7 +516,7 @@ __global__ void __launch_bounds__(TRACE_THREADS) __attribute__((amdgpu_waves_per
       got = sphere_world<!MULTI, TRACE_THREADS>(Sj, v3{a.x, a.y, a.z}, v3{b.x, b.y, b.z}, rc, 0.001f, kFltMax, valid,
                                                 bstack + threadIdx.x, &h, &st[ST_NODES]);
     } else if (SWEEP) {
-      got = small_world(Sj, v3{a.x, a.y, a.z}, v3{b.x, b.y, b.z}, rc, 0.001f, kFltMax, &h, &st[ST_NODES], valid);
+      got = small_world<false, MEDIA>(Sj, v3{a.x, a.y, a.z}, v3{b.x, b.y, b.z}, rc, 0.001f, kFltMax, &h, &st[ST_NODES], valid);
     } else {
       got = trace_world<SPH, MEDIA>(Sj, v3{a.x, a.y, a.z}, v3{b.x, b.y, b.z}, rc, 0.001f, kFltMax, &h,
                                            &st[ST_NODES], valid, COUNT ? &oc : nullptr);
@@ -653,7 +653,7 @@ __device__ __forceinline__ void claim_and_append_ref(const render_params &P, con
 // One queued hit (or miss) of class cls with the plain sampler: the
 // reference's color() step for it.  Updates p (radiance, throughput, next
 // ray); true when the path goes on.  Shared by k_shade and k_tail.
-template <bool SIMPLE>
+template <bool SIMPLE, bool MEDIA = !SIMPLE>
 __device__ __forceinline__ bool shade_hit(const scene_view &S, const scene_view &Sj, const render_params &P,
                                           const job_dev &J, const item_ctx &c, path &p, const hit_t &h, uint32_t cls,
                                           uint32_t *st) {
@@ -696,7 +696,7 @@ __device__ __forceinline__ bool shade_hit(const scene_view &S, const scene_view 
       // (headers/material.h:74-80), so color() returns emitted (0): the
       // path ends black.  TPT_RENDER_MEDIA_SCATTER scatters as the book
       // intends (src/material.cc:72-77): random_in_unit_sphere, albedo.
-      if (!SIMPLE && P.media_scatter) {
+      if (MEDIA && P.media_scatter) {
         nd = in_unit_sphere(R);
         p.thr = p.thr * tex_value<SIMPLE>(S, M.tex, u, v, pt);
         cont = true;

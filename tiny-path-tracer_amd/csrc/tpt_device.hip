@@ -50,7 +50,7 @@ __global__ void __launch_bounds__(256) k_trace_closest(scene_view S, const tpt_s
   __shared__ uint32_t bstack[SPH ? kBvhDepth * 256 : 1];  // sphere_world's
   bool got;
   if (SWEEP)
-    got = small_world<true>(S, o, d, rc, tmin, tmax, &h, &nodes, live, &id);
+    got = small_world<!MEDIA, MEDIA>(S, o, d, rc, tmin, tmax, &h, &nodes, live, &id);
   else if (SPH)
     got = sphere_world<true, 256>(S, o, d, rc, tmin, tmax, live, bstack + threadIdx.x, &h, &nodes);
   else
@@ -173,6 +173,7 @@ struct tpt_scene {
   std::vector<uint8_t> sweep;     // per scene: wave-uniform traversal (small scenes)
   std::vector<uint8_t> sph;       // per scene: every leaf is a sphere
   std::vector<uint8_t> simple;    // per scene: constant textures, no light or one xz_rect light
+  std::vector<uint8_t> plain;     // per scene: as simple, but media are allowed
   std::vector<uint8_t> motion;    // per scene: has moving spheres (rays need their time)
   std::vector<uint8_t> media;     // per scene: has constant_medium (queries need media draws)
   std::vector<flat_range> flat_of;  // per scene: its part of flat and fgroups
@@ -453,12 +454,41 @@ float rebase_bits(float f, uint32_t base) {
 // list that close a box become one record.  sb, eb, xb, mb: the scene's first
 // slot, entry, transform and material in the pool.
 constexpr uint32_t kFlatMax = 64;  // most primitives of the pass
-enum { FLAT_SPHERE = 3, FLAT_BOX = 4 };
+enum { FLAT_SPHERE = 3, FLAT_BOX = 4, FLAT_MEDIUM = 5 };
 struct flat_item {
   flat_scan scan;
   flat_win win[6];  // one, or a box's faces
-  uint32_t cls;     // 0..2 rect by axis, FLAT_SPHERE, FLAT_BOX
+  uint32_t cls;     // 0..2 rect by axis, FLAT_SPHERE, FLAT_BOX, FLAT_MEDIUM
 };
+
+bool closed_box(const flat_item *r, float lo[3], float hi[3], int face[6]);
+
+// A medium whose boundary is six rects that close a box, as a record (its
+// boundary's wrapper chain is the record's).
+bool medium_box(const tpt_flat_scene &f, const float *w, flat_item *it) {
+  uint32_t first, count;
+  std::memcpy(&first, &w[0], 4);
+  std::memcpy(&count, &w[1], 4);
+  if (count != 6) return false;
+  flat_item r[6];
+  for (uint32_t i = 0; i < 6; ++i) {
+    const tpt_entry &e = f.entries[first + i];
+    if (e.b != TPT_SLOT_RECT) return false;
+    r[i] = flat_item{};
+    r[i].cls = (e.a >> 28) & 3u;
+    for (int k = 0; k < 5; ++k) r[i].win[0].f[k] = e.f[k];
+    r[i].win[0].xform = e.xform;
+  }
+  float lo[3], hi[3];
+  int face[6];
+  if (!closed_box(r, lo, hi, face)) return false;
+  it->cls = FLAT_MEDIUM;
+  it->scan.k = lo[0], it->scan.c0 = lo[1], it->scan.c1 = lo[2];
+  it->scan.h0 = hi[0], it->scan.h1 = hi[1], it->scan.x = hi[2];
+  it->scan.density = w[2];
+  it->win[0].xform = r[0].win[0].xform;
+  return true;
+}
 
 // The closed box of six rects (k, a0, a1, b0, b1 with axes), if they are one:
 // lo / hi corners and which of them is each face (low x, high x, low y, ...).
@@ -495,10 +525,10 @@ flat_range flat_records(const tpt_flat_scene &f, uint32_t sb, uint32_t eb, uint3
                  uint32_t leaf, uint32_t parent) {
     flat_item it{};
     flat_win &q = it.win[0];
-    const int nf = kind == TPT_SLOT_RECT ? 5 : 4;
+    const int nf = kind == TPT_SLOT_RECT ? 5 : (kind == TPT_SLOT_SPHERE ? 4 : 0);  // (a medium's hold indexes)
     for (int k = 0; k < nf; ++k) q.f[k] = w[k], ok = ok && std::fabs(w[k]) < 1e18f;
     flat_scan &p = it.scan;
-    p.k = w[0];
+    if (nf) p.k = w[0];
     if (kind == TPT_SLOT_RECT) {
       it.cls = (word >> 28) & 3u;
       p.c0 = 0.5f * (w[1] + w[2]), p.c1 = 0.5f * (w[3] + w[4]);
@@ -516,6 +546,10 @@ flat_range flat_records(const tpt_flat_scene &f, uint32_t sb, uint32_t eb, uint3
       it.cls = FLAT_SPHERE;
       p.c0 = w[1], p.c1 = w[2], p.h0 = w[3];
       for (int k = 0; k < 3; ++k) mag = std::fmax(mag, std::fabs(w[k]) + std::fabs(w[3]));
+    } else if (kind == TPT_SLOT_MEDIUM && xform == 0xFFFFFFFFu && medium_box(f, w, &it)) {
+      const flat_scan &b = it.scan;
+      for (float c : {b.k, b.c0, b.c1, b.h0, b.h1, b.x}) ok = ok && std::fabs(c) < 1e18f, mag = std::fmax(mag, std::fabs(c));
+      xform = q.xform;  // the pass groups it by its boundary's chain
     } else {
       ok = false;
     }
@@ -594,14 +628,14 @@ flat_range flat_records(const tpt_flat_scene &f, uint32_t sb, uint32_t eb, uint3
       fg.nops = x.nops, fg.kinds = x.kinds;
       std::memcpy(fg.p, x.p, sizeof(fg.p));
     }
-    for (uint32_t c = 0; c <= FLAT_BOX; ++c)
+    for (uint32_t c = 0; c <= FLAT_MEDIUM; ++c)
       for (flat_item &it : merged)
         if (it.win[0].xform == xf && it.cls == c) {
           it.scan.win = static_cast<uint32_t>(wins->size()) - r.win0;
           scans->push_back(it.scan);
           wins->insert(wins->end(), it.win, it.win + (c == FLAT_BOX ? 6 : 1));
-          if (c == FLAT_BOX)
-            ++fg.n_box;
+          if (c >= FLAT_BOX)
+            fg.n_box += c == FLAT_BOX ? 1u : 0x10000u;
           else
             fg.n += 1u << (8 * c);
         }
@@ -634,7 +668,7 @@ int create_pool(const tpt_flat_scene *scenes, uint32_t n, tpt_scene **out) {
   std::vector<uint32_t> seg_xf;
   bool any_wrapped = false;
   std::vector<scene_dev> scn(n);
-  std::vector<uint8_t> sweep(n), sph(n), simple(n), motion(n), media(n);
+  std::vector<uint8_t> sweep(n), sph(n), simple(n), plain(n), motion(n), media(n);
   std::vector<uint32_t> nslots(n), nleaves(n);
   std::vector<flat_scan> flat;
   std::vector<flat_win> fwins;
@@ -734,12 +768,12 @@ int create_pool(const tpt_flat_scene *scenes, uint32_t n, tpt_scene **out) {
     media[k] = 0;
     for (uint32_t i = 0; i < f.n_slots; ++i) media[k] |= (f.slots[i].b >> 28) == TPT_SLOT_MEDIUM;
     for (uint32_t e = 0; e < f.n_entries; ++e) media[k] |= f.entries[e].b == TPT_SLOT_MEDIUM;
-    // Wave-uniform sweeps pay for the union of the lanes' visits; that stays
-    // close to each lane's own count only when the whole tree is small.  (The
-    // sweep kernel is built without the ray-time replay and the media draws.)
+    // The uniform pass tests every primitive, so it is for small scenes.  (It
+    // is built without the ray-time replay, wrapped segments, and media not
+    // bounded by a closed box: flat_records has none then.)
     bool wrapped = false;
     for (uint32_t g = 0; f.segment_xforms && g < f.n_segments; ++g) wrapped |= f.segment_xforms[g] != TPT_SEGMENT_PLAIN;
-    sweep[k] = f.n_slots <= 64 && !motion[k] && !media[k] && !wrapped;
+    sweep[k] = f.n_slots <= 64 && !motion[k] && !wrapped;
     if (sweep[k]) {
       flat_of[k] = flat_records(f, static_cast<uint32_t>(sb), static_cast<uint32_t>(eb), static_cast<uint32_t>(xb),
                                 static_cast<uint32_t>(mb), &flat, &fwins, &fgroups);
@@ -748,9 +782,9 @@ int create_pool(const tpt_flat_scene *scenes, uint32_t n, tpt_scene **out) {
     if (wrapped) sph[k] = 0;  // the sphere-only walk is built without segment transforms
     std::memset(&bscn[k], 0, sizeof(bscn[k]));
     if (sph[k]) bscn[k] = build_bvh(f, static_cast<uint32_t>(sb), &bnodes, &bleaves);
-    simple[k] = !motion[k] && !media[k] &&
-                (f.n_lights == 0 || (f.light_mode == 0 && f.lights[0].kind == TPT_LIGHT_XZ_RECT));
-    for (uint32_t t = 0; t < f.n_textures; ++t) simple[k] = simple[k] && f.textures[t].kind == TPT_TEX_CONSTANT;
+    plain[k] = !motion[k] && (f.n_lights == 0 || (f.light_mode == 0 && f.lights[0].kind == TPT_LIGHT_XZ_RECT));
+    for (uint32_t t = 0; t < f.n_textures; ++t) plain[k] = plain[k] && f.textures[t].kind == TPT_TEX_CONSTANT;
+    simple[k] = plain[k] && !media[k];
     nslots[k] = f.n_slots;
     nleaves[k] = f.n_leaves;
   }
@@ -791,6 +825,7 @@ int create_pool(const tpt_flat_scene *scenes, uint32_t n, tpt_scene **out) {
   s->sweep = sweep;
   s->sph = sph;
   s->simple = simple;
+  s->plain = plain;
   s->motion = motion;
   s->media = media;
   s->flat_of = flat_of;
@@ -890,7 +925,11 @@ int tpt_trace_closest_timed(tpt_scene *s, const float *d_rays, const float *d_ti
   const uint64_t blocks = (n + 255) / 256;
   if (blocks > 0x7FFFFFFFull) return tpt::fail(TPT_ERR_INVALID, "tpt_trace_closest: too many rays");
   const scene_view S = s->view(0);
-  if (s->sweep[0])
+  if (s->sweep[0] && s->media[0])
+    hipLaunchKernelGGL((k_trace_closest<true, true>), dim3(static_cast<uint32_t>(blocks)), dim3(256), 0,
+                       static_cast<hipStream_t>(stream), S, S.slots, S.entries, d_rays, d_time, n, t_min, t_max,
+                       d_leaf, d_t, d_rec, d_mat);
+  else if (s->sweep[0])
     hipLaunchKernelGGL((k_trace_closest<true, false>), dim3(static_cast<uint32_t>(blocks)), dim3(256), 0,
                        static_cast<hipStream_t>(stream), S, S.slots, S.entries, d_rays, d_time, n, t_min, t_max,
                        d_leaf, d_t, d_rec, d_mat);
@@ -993,6 +1032,7 @@ struct bounce_launch {
   bool sweep, multi, guided;
   bool sph;     // every leaf of the launch's scenes is a sphere
   bool simple;  // their textures are constant and their light root absent or one xz_rect
+  bool plain;   // as simple, but media are allowed
   bool tail;    // passes end with a fused k_tail launch (simple scenes, sweep or sphere-only walk)
   bool count;   // TPT_RENDER_COUNT_OPS: the counting variant of k_trace, no fused tail
 };
@@ -1025,7 +1065,7 @@ void launch_tail(const bounce_launch &B, hipStream_t st, uint32_t parity, uint32
 }
 
 // Blocks per CU of k_paths: its occupancy target, in waves per SIMD, one block of 4 waves each.
-uint32_t path_blocks_per_cu(const bounce_launch &B) { return path_waves(B.sweep, B.sph, B.simple, B.P.media != 0); }
+uint32_t path_blocks_per_cu(const bounce_launch &B) { return path_waves(B.sweep, B.sph, B.simple || B.plain, B.P.media != 0); }
 
 template <bool SWEEP, bool MULTI, bool SPH, bool SIMPLE, bool MEDIA>
 void launch_paths_t(const bounce_launch &B, hipStream_t st, uint32_t grid) {
@@ -1034,6 +1074,8 @@ void launch_paths_t(const bounce_launch &B, hipStream_t st, uint32_t grid) {
 }
 
 void launch_paths(const bounce_launch &B, hipStream_t st, uint32_t grid) {
+  if (B.sweep && B.P.media) return B.plain ? launch_paths_t<true, false, false, true, true>(B, st, grid)
+                                           : launch_paths_t<true, false, false, false, true>(B, st, grid);
   if (B.P.media) return B.multi ? launch_paths_t<false, true, false, false, true>(B, st, grid)
                                 : launch_paths_t<false, false, false, false, true>(B, st, grid);
   if (B.sweep) return B.simple ? launch_paths_t<true, false, false, true, false>(B, st, grid)
@@ -1051,7 +1093,10 @@ void launch_paths(const bounce_launch &B, hipStream_t st, uint32_t grid) {
 template <bool COUNT>
 void launch_trace_t(const bounce_launch &B, hipStream_t st, uint32_t parity) {
   const dim3 g(B.grid), b(TRACE_THREADS);
-  if (B.sweep && !COUNT)
+  if (B.sweep && B.P.media && !COUNT)
+    hipLaunchKernelGGL((k_trace<true, false, false, true, false>), g, b, 0, st, B.S, B.S.slots, B.S.entries, B.P,
+                       B.Q, parity);
+  else if (B.sweep && !COUNT)
     hipLaunchKernelGGL((k_trace<true, false, false, false, false>), g, b, 0, st, B.S, B.S.slots, B.S.entries, B.P,
                        B.Q, parity);
   else if (B.multi && B.P.media)
@@ -1288,9 +1333,11 @@ int render_core(tpt_scene *s, const tpt_job *jobs, uint32_t n_jobs, const tpt_la
   B.sweep = !multi && s->sweep[jobs[0].scene];
   B.sph = true;
   B.simple = true;
+  B.plain = true;
   for (uint32_t j = 0; j < n_jobs; ++j) {
     B.sph = B.sph && s->sph[jobs[j].scene];
     B.simple = B.simple && s->simple[jobs[j].scene];
+    B.plain = B.plain && s->plain[jobs[j].scene];
     if (s->motion[jobs[j].scene]) B.P.motion = 1;
     if (s->media[jobs[j].scene]) B.P.media = 1;
   }

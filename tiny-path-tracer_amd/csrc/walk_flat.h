@@ -201,6 +201,61 @@ __device__ __forceinline__ bool flat_exact(const scene_view &S, uint32_t id, flo
   return got;
 }
 
+// A constant_medium (src/hitable.cc:98-128) bounded by a closed box.  Certain
+// where the line enters the box by one face and leaves it by another, apart
+// from their neighbours by more than et and from each other by more than the
+// 0.0001 between the reference's two boundary queries: those then return the
+// exact times of the two faces, which are computed here, and the rest of
+// medium_t follows with the same arithmetic.  (With the caller's t_max in place
+// of the nearest hit so far: a free path that ends beyond that hit is then
+// offered beyond it.)  Undecided lanes are offered at the lowest time.  Smoke
+// box 400x400 64 spp: 6.0 -> 2.1 ms against the general media walk, which
+// evaluates both boundary queries rect by rect at 2 waves per SIMD.
+__device__ __forceinline__ void flat_medium(const scene_view &S, flat_scan_ptr p, v3 o, v3 d, v3 wd, v3 inv,
+                                            const ray_ctx &rc, float et, float tlo, float tmin, float tmax,
+                                            flat_best &best) {
+  const float x0 = (p->k - o.x) * inv.x, x1 = (p->h0 - o.x) * inv.x;
+  const float y0 = (p->c0 - o.y) * inv.y, y1 = (p->h1 - o.y) * inv.y;
+  const float z0 = (p->c1 - o.z) * inv.z, z1 = (p->x - o.z) * inv.z;
+  const float nx = fminf(x0, x1), ny = fminf(y0, y1), nz = fminf(z0, z1);
+  const float fx = fmaxf(x0, x1), fy = fmaxf(y0, y1), fz = fmaxf(z0, z1);
+  const float n = max3f(nx, ny, nz), f = fminf(fminf(fx, fy), fz);
+  const float fe = f + et;
+  const bool pos = n <= fe && fe >= tlo;
+  if (__ballot(pos) == 0ull) return;
+  const float n2 = __builtin_amdgcn_fmed3f(nx, ny, nz), f2 = __builtin_amdgcn_fmed3f(fx, fy, fz);
+  const bool sure = f - n > 0.0002f + et + 0x1p-18f * (fabsf(n) + fabsf(f)) && n - n2 > et && f2 - f > et;
+  float t = tlo, e = INFINITY;
+  bool hit = pos;
+  if (pos && sure) {
+    const bool ax = n == nx, ay = n == ny, bx = f == fx, by = f == fy;
+    const float k1 = ax ? (n == x0 ? p->k : p->h0) : (ay ? (n == y0 ? p->c0 : p->h1) : (n == z0 ? p->c1 : p->x));
+    const float k2 = bx ? (f == x0 ? p->k : p->h0) : (by ? (f == y0 ? p->c0 : p->h1) : (f == z0 ? p->c1 : p->x));
+    float t1 = (k1 - (ax ? o.x : (ay ? o.y : o.z))) / (ax ? d.x : (ay ? d.y : d.z));
+    float t2 = (k2 - (bx ? o.x : (by ? o.y : o.z))) / (bx ? d.x : (by ? d.y : d.z));
+    hit = false;
+    // beyond t = 2048 the 0.0001 may round away: the second query then finds
+    // the entry face again, and the medium is missed
+    if (t1 >= static_cast<float>(static_cast<double>(t1) + 0.0001)) t2 = t1;
+    if (t1 < tmin) t1 = tmin;
+    if (t2 > tmax) t2 = tmax;
+    if (t1 < t2) {
+      const float len = sqrtf(wd.x * wd.x + wd.y * wd.y + wd.z * wd.z);
+      const float inside = (t2 - t1) * len;
+      typedef const TPT_SCALAR flat_win *flat_win_ptr;
+      const uint4 w = medium_draws(rc, ((flat_win_ptr)(S.fwins))[p->win].leaf);
+      const float hit_distance =
+          static_cast<float>(static_cast<double>(-1.0f / p->density) * log(static_cast<double>(u01(w.x))));
+      if (hit_distance < inside) {
+        hit = true;
+        t = t1 + hit_distance / len;
+        e = -INFINITY;
+      }
+    }
+  }
+  flat_offer<false>(best, hit, t, e, p->win);
+}
+
 // All lanes of the wave call together.  Returns the hit of lanes that are
 // live and not slow; *slow: the lane needs the exact walk.  *leaf: the hit's
 // leaf id.
@@ -213,12 +268,14 @@ __device__ __forceinline__ bool flat_exact(const scene_view &S, uint32_t id, flo
 // hit by every rect at t = NaN and passes every box, whatever its direction:
 // the last rect in the reference's order wins (flat_nan).
 //
+// MEDIA: the scene holds constant_media (all bounded by closed boxes).
+//
 // TIES: two rects at the same time (the bottom of a box that stands on the
 // floor, seen from inside it) are both evaluated and the reference's rule
 // applied, the smaller t, at equal t the later one.  Paths do not get there;
 // for a caller's own rays it keeps such lanes off the exact walk.
-template <bool TIES>
-__device__ __forceinline__ bool flat_world(const scene_view &S, v3 o, v3 d, float tmin, float tmax, bool live,
+template <bool TIES, bool MEDIA>
+__device__ __forceinline__ bool flat_world(const scene_view &S, v3 o, v3 d, const ray_ctx &rc, float tmin, float tmax, bool live,
                                            hit_t *out, uint32_t *nodes, bool *slow, uint32_t *leaf = nullptr) {
   const bool zx = d.x == 0.0f, zy = d.y == 0.0f, zz = d.z == 0.0f;
   const v3 inv{zx ? __builtin_amdgcn_rcpf(d.x) : recip_rn(d.x), zy ? __builtin_amdgcn_rcpf(d.y) : recip_rn(d.y),
@@ -240,7 +297,7 @@ __device__ __forceinline__ bool flat_world(const scene_view &S, v3 o, v3 d, floa
   flat_group_ptr groups = (flat_group_ptr)(S.fgroups);
   uint32_t visits = 0;
   for (uint32_t g = 0; g < S.n_fgroups; ++g) {
-    const uint32_t n = groups[g].n, n_box = groups[g].n_box, nops = groups[g].nops, kinds = groups[g].kinds;
+    const uint32_t n = groups[g].n, n_box = groups[g].n_box & 0xFFFFu, n_med = groups[g].n_box >> 16, nops = groups[g].nops, kinds = groups[g].kinds;
     v3 lo = o, ld = d, li = inv;
     float et = mi;
     if (nops) {
@@ -258,7 +315,7 @@ __device__ __forceinline__ bool flat_world(const scene_view &S, v3 o, v3 d, floa
       odd = odd || !(et < 0x1p60f);
     }
     if (any_zero)  // (a zero x or z component seen through a rotation is tiny, or made the lane odd)
-      odd = odd || flat_in_plane(p, n, n_box, lo, zero && zx && !nops, zero && zy, zero && zz && !nops);
+      odd = odd || flat_in_plane(p, n, n_box + n_med, lo, zero && zx && !nops, zero && zy, zero && zz && !nops);
     et *= 0.375f * m;
     p = flat_rects<TIES, 0>(p, n & 255u, lo, ld, li, m, tlo, best);
     p = flat_rects<TIES, 1>(p, (n >> 8) & 255u, lo, ld, li, m, tlo, best);
@@ -269,7 +326,9 @@ __device__ __forceinline__ bool flat_world(const scene_view &S, v3 o, v3 d, floa
       flat_offer<TIES>(best, h, t, -INFINITY, p->win);
     }
     for (uint32_t k = n_box; k > 0; --k, ++p) flat_box<TIES>(p, lo, li, et, tlo, best);
-    visits += (n & 255u) + ((n >> 8) & 255u) + ((n >> 16) & 255u) + (n >> 24) + n_box;
+    if (MEDIA)
+      for (uint32_t k = n_med; k > 0; --k, ++p) flat_medium(S, p, lo, ld, d, li, rc, et, tlo, tmin, tmax, best);
+    visits += (n & 255u) + ((n >> 8) & 255u) + ((n >> 16) & 255u) + (n >> 24) + n_box + n_med;
   }
   *nodes += live ? visits : 0u;
   // beyond t_max by more than its error: a certain miss
@@ -311,6 +370,7 @@ __device__ __forceinline__ bool flat_world(const scene_view &S, v3 o, v3 d, floa
 // missed box is dropped there), and is exact for NaN times too.  About 1400
 // instructions for the Cornell box; segment_exact, a stack machine per lane,
 // takes about 11000.
+template <bool MEDIA>
 __device__ __forceinline__ bool segment_combine(const scene_view &S, uint32_t start, uint32_t end, v3 o, v3 d, v3 inv,
                                                 const ray_ctx &rc, float tmin, float tmax, hit_t *out) {
   float ts[64];
@@ -334,7 +394,7 @@ __device__ __forceinline__ bool segment_combine(const scene_view &S, uint32_t st
       id = left ? ids[k + 1] : ids[kr];
     } else {
       uint32_t entry, mat;
-      have = leaf_t<false, false>(S, s, kind, o, d, rc, tmin, tmax, &t, &entry, &mat);
+      have = leaf_t<false, MEDIA>(S, s, kind, o, d, rc, tmin, tmax, &t, &entry, &mat);
       if (kind == TPT_SLOT_LIST && have) id |= (entry - s.a + 1) << 8;
     }
     ts[k] = t;
@@ -352,11 +412,11 @@ __device__ __forceinline__ bool segment_combine(const scene_view &S, uint32_t st
 
 // Closest hit of a small scene: the uniform pass, then the exact recursion for
 // the lanes that need it.  All lanes of the wave call together.
-template <bool TIES = false>
+template <bool TIES = false, bool MEDIA = false>
 __device__ __forceinline__ bool small_world(const scene_view &S, v3 o, v3 d, const ray_ctx &rc, float tmin, float tmax,
                                             hit_t *out, uint32_t *nodes, bool live, uint32_t *leaf = nullptr) {
   bool slow;
-  bool got = flat_world<TIES>(S, o, d, tmin, tmax, live, out, nodes, &slow, leaf);
+  bool got = flat_world<TIES, MEDIA>(S, o, d, rc, tmin, tmax, live, out, nodes, &slow, leaf);
   if (__ballot(slow) != 0ull) {
     const v3 inv{1.0f / d.x, 1.0f / d.y, 1.0f / d.z};
     hit_t best{0.0f, kNone, kNone, 0};
@@ -365,7 +425,7 @@ __device__ __forceinline__ bool small_world(const scene_view &S, v3 o, v3 d, con
     for (uint32_t g = 0; g < S.n_segments; ++g) {
       const uint32_t start = S.segments[2 * g], end = S.segments[2 * g + 1];
       hit_t h;
-      if (start < end && segment_combine(S, start, end, o, d, inv, rc, tmin, cur, &h)) {
+      if (start < end && segment_combine<MEDIA>(S, start, end, o, d, inv, rc, tmin, cur, &h)) {
         best = h;
         cur = h.t;
         any = true;
