@@ -99,7 +99,7 @@ __device__ __forceinline__ void flat_test(const flat_rect &p, v3 o, v3 d, v3 inv
   const float x = fabsf(__builtin_fmaf(t, d0, o0) - p.c0) - p.h0;
   const float y = fabsf(__builtin_fmaf(t, d1, o1) - p.c1) - p.h1;
   const float e = fmaxf(x, y);
-  flat_offer<TIES>(best, e <= m && t >= tlo, t, e, p.win);
+  flat_offer<TIES>(best, (e <= m) & (t >= tlo), t, e, p.win);
 }
 
 template <bool TIES, int AXIS>
@@ -134,8 +134,8 @@ __device__ __forceinline__ void flat_box(flat_scan_ptr p, v3 o, v3 inv, float et
   const float n2 = __builtin_amdgcn_fmed3f(nx, ny, nz), f2 = __builtin_amdgcn_fmed3f(fx, fy, fz);
   const bool in = n >= tlo;
   const float fe = f + et;
-  const bool pos = n <= fe && fe >= tlo && (f >= tlo || in || f2 <= fe);
-  const bool sure = f - n > et && (in ? n - n2 : f2 - f) > et;
+  const bool pos = (n <= fe) & (fe >= tlo) & ((f >= tlo) | in | (f2 <= fe));
+  const bool sure = (f - n > et) & ((in ? n - n2 : f2 - f) > et);
   const float t = sure ? (in ? n : f) : tlo;
   // the face: a plane of that axis, the one whose time it is
   const bool ax = t == (in ? nx : fx), ay = t == (in ? ny : fy);
@@ -162,15 +162,17 @@ __device__ __forceinline__ void flat_touch(const scene_view &S) {
 // NaN wherever the ray is.
 __device__ __forceinline__ bool flat_in_plane(flat_scan_ptr p, uint32_t n, uint32_t n_box, v3 o, bool zx, bool zy,
                                               bool zz) {
+  // (bitwise: a short circuit would branch per lane, and what is computed past
+  // it would no longer count as uniform)
   bool in = false;
   const uint32_t n0 = n & 255u, n1 = (n >> 8) & 255u, n2 = (n >> 16) & 255u;
-  for (uint32_t k = 0; k < n0; ++k, ++p) in = in || (zx && p->k == o.x);
-  for (uint32_t k = 0; k < n1; ++k, ++p) in = in || (zy && p->k == o.y);
-  for (uint32_t k = 0; k < n2; ++k, ++p) in = in || (zz && p->k == o.z);
+  for (uint32_t k = 0; k < n0; ++k, ++p) in |= zx & (p->k == o.x);
+  for (uint32_t k = 0; k < n1; ++k, ++p) in |= zy & (p->k == o.y);
+  for (uint32_t k = 0; k < n2; ++k, ++p) in |= zz & (p->k == o.z);
   p += n >> 24;
   for (uint32_t k = 0; k < n_box; ++k, ++p)
-    in = in || (zx && (p->k == o.x || p->h0 == o.x)) || (zy && (p->c0 == o.y || p->h1 == o.y)) ||
-         (zz && (p->c1 == o.z || p->x == o.z));
+    in |= (zx & ((p->k == o.x) | (p->h0 == o.x))) | (zy & ((p->c0 == o.y) | (p->h1 == o.y))) |
+          (zz & ((p->c1 == o.z) | (p->x == o.z)));
   return in;
 }
 
@@ -221,7 +223,7 @@ __device__ __forceinline__ void flat_medium(const scene_view &S, flat_scan_ptr p
   const float fx = fmaxf(x0, x1), fy = fmaxf(y0, y1), fz = fmaxf(z0, z1);
   const float n = max3f(nx, ny, nz), f = fminf(fminf(fx, fy), fz);
   const float fe = f + et;
-  const bool pos = n <= fe && fe >= tlo;
+  const bool pos = (n <= fe) & (fe >= tlo);
   if (__ballot(pos) == 0ull) return;
   const float n2 = __builtin_amdgcn_fmed3f(nx, ny, nz), f2 = __builtin_amdgcn_fmed3f(fx, fy, fz);
   const bool sure = f - n > 0.0002f + et + 0x1p-18f * (fabsf(n) + fabsf(f)) && n - n2 > et && f2 - f > et;
@@ -312,10 +314,10 @@ __device__ __forceinline__ bool flat_world(const scene_view &S, v3 o, v3 d, cons
       }
       li = v3{__builtin_amdgcn_rcpf(ld.x), inv.y, __builtin_amdgcn_rcpf(ld.z)};
       et = max3f(fabsf(li.x), my, fabsf(li.z));
-      odd = odd || !(et < 0x1p60f);
+      odd |= !(et < 0x1p60f);
     }
     if (any_zero)  // (a zero x or z component seen through a rotation is tiny, or made the lane odd)
-      odd = odd || flat_in_plane(p, n, n_box + n_med, lo, zero && zx && !nops, zero && zy, zero && zz && !nops);
+      odd |= flat_in_plane(p, n, n_box + n_med, lo, zero & zx & !nops, zero & zy, zero & zz & !nops);
     et *= 0.375f * m;
     p = flat_rects<TIES, 0>(p, n & 255u, lo, ld, li, m, tlo, best);
     p = flat_rects<TIES, 1>(p, (n >> 8) & 255u, lo, ld, li, m, tlo, best);
