@@ -80,3 +80,25 @@ def test_paths_pooled_jobs_equal_bounce_loop(tpt, device, which):
     for k in COUNTS:
         assert sa[k] == sb[k], k
     assert sa["tail_launches"] == (1 if which == "spheres" else 0) and sb["tail_launches"] == 0
+
+
+@pytest.mark.parametrize("name", ["cornell555", "ref_cornell_box", "random_spheres"])
+@pytest.mark.parametrize("general", [False, True])
+def test_pinhole_skips_the_lens_loop(tpt, device, name, general):
+    """A zero lens without -0 coordinates skips the lens draws.
+
+    Moving the camera from x = +0 to x = -0 takes the loop instead, and no value
+    of a path depends on that sign: equal bits.
+    """
+    import torch
+
+    sc = tpt.Scene.named(name)
+    i = sc.host.info
+    got = []
+    for x in (0.0, -0.0):
+        cam = tpt.camera_make((x, *tuple(i.lookfrom)[1:]), tuple(i.lookat), (0.0, 1.0, 0.0), i.vfov, 61 / 67, 0.0,
+                              i.focus)
+        got.append(sc.render(width=61, height=67, spp=5, seed=5, camera=cam, tail=not general))
+    (a, qa, sa), (b, qb, sb) = got
+    assert torch.equal(a, b) and torch.equal(qa, qb)
+    assert all(sa[k] == sb[k] for k in COUNTS)

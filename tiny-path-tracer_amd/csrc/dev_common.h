@@ -145,6 +145,7 @@ __device__ __forceinline__ float u01(uint32_t x) { return static_cast<float>(x >
 
 struct stream {
   uint32_t pixel, sample, bounce, k0, k1, draw;
+  bool primed;
   uint4 cache;
   __device__ __forceinline__ void init(uint32_t p, uint32_t s, uint32_t b, uint64_t seed) {
     pixel = p;
@@ -153,9 +154,16 @@ struct stream {
     k0 = static_cast<uint32_t>(seed);
     k1 = static_cast<uint32_t>(seed >> 32);
     draw = 0;
+    primed = false;
+  }
+  // The first four draws at once: where the classes of a wave's hits branch
+  // apart, they then share one Philox block instead of computing one each.
+  __device__ __forceinline__ void prime() {
+    cache = philox(pixel, sample, bounce, 0u, k0, k1);
+    primed = true;
   }
   __device__ __forceinline__ float next() {
-    if ((draw & 3u) == 0) cache = philox(pixel, sample, bounce, draw >> 2, k0, k1);
+    if ((draw & 3u) == 0 && !(primed && draw == 0)) cache = philox(pixel, sample, bounce, draw >> 2, k0, k1);
     const uint32_t w = draw & 3u;
     ++draw;
     const uint32_t x = w == 0 ? cache.x : (w == 1 ? cache.y : (w == 2 ? cache.z : cache.w));

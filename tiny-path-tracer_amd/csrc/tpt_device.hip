@@ -1010,6 +1010,18 @@ std::vector<pass_plan> plan_passes(const tpt_job *jobs, uint32_t n_jobs, uint64_
   return out;
 }
 
+// Whether the lens offset of raygen is 0 and adding it changes no bit: no lens,
+// finite lens axes, and no -0 in what it is added to.
+bool pinhole(const tpt_camera &c) {
+  bool ok = c.lens_radius == 0.0f;
+  for (int k = 0; k < 3; ++k) {
+    ok = ok && std::isfinite(c.u[k]) && std::isfinite(c.v[k]);
+    ok = ok && !(c.origin[k] == 0.0f && std::signbit(c.origin[k])) &&
+         !(c.lower_left[k] == 0.0f && std::signbit(c.lower_left[k]));
+  }
+  return ok;
+}
+
 template <class T>
 int grow_device(T **p, uint32_t *cap, uint32_t need) {
   if (need <= *cap) return TPT_OK;
@@ -1324,6 +1336,7 @@ int render_core(tpt_scene *s, const tpt_job *jobs, uint32_t n_jobs, const tpt_la
     d.seed = J.seed;
     d.background = J.background;
     d.scene = J.scene;
+    d.pinhole = pinhole(J.camera);
     d.sum = J.d_sum;
     d.sumsq = J.d_sumsq;
   }
@@ -1833,6 +1846,7 @@ int render_noalloc(tpt_scene *s, const tpt_camera *camera, const tpt_render_desc
   jd.seed = desc->seed;
   jd.background = desc->background;
   jd.scene = 0;
+  jd.pinhole = pinhole(*camera);
   jd.sum = d_sum;
   jd.sumsq = d_sumsq;
 

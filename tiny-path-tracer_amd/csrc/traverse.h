@@ -513,32 +513,47 @@ __device__ __forceinline__ uint32_t leaf_id(const scene_view &S, const hit_t &h)
   return s.b & TPT_PAYLOAD_MASK;
 }
 
+// The winner's primitive and the ray in its frame.
+struct hit_geo {
+  float f[5];
+  uint32_t kind, word, xf;  // xf: wrapper chain or kNone
+  v3 lo, ld;
+};
+
 // Full hit_record of the winner: point, normal (flip applied), u, v.
 // MEDIUM_NORMAL: draw a medium hit's arbitrary normal as constant_medium::hit
 // does; the shading kernels skip it (the isotropic phase function ignores the
-// normal) and report (0, 1, 0).
+// normal) and report (0, 1, 0).  geo: the winner's primitive and local ray, of
+// a scene without wrapped segments, where the trace has them at hand.
 template <bool MEDIUM_NORMAL = false>
 __device__ __forceinline__ void hit_record(const scene_view &S, const hit_t &h, v3 o, v3 d, const ray_ctx &rc, v3 *p,
-                                           v3 *n, float *u, float *v) {
-  const slot_t s = load_slot(&S.slots[h.slot]);
-  uint32_t kind = s.b >> 28;
-  float f[5] = {s.f[0], s.f[1], s.f[2], s.f[3], s.f[4]};
-  uint32_t word = s.a;
+                                           v3 *n, float *u, float *v, const hit_geo *geo = nullptr) {
+  float f[5];
+  uint32_t kind, word, xf = kNone;
   v3 lo = o, ld = d;
-  uint32_t xf = kNone;
   // the wrappers of the winner's segment, if any (outermost, applied first)
   uint32_t sx = TPT_SEGMENT_PLAIN;
-  if (S.seg_xf)
-    for (uint32_t g = 0; g < S.n_segments; ++g)
-      if (h.slot >= S.segments[2 * g] && h.slot < S.segments[2 * g + 1]) sx = S.seg_xf[g];
-  if ((sx & TPT_SEGMENT_PLAIN) != TPT_SEGMENT_PLAIN) to_local(S.xforms[sx & TPT_SEGMENT_PLAIN], &lo, &ld);
-  if (kind == TPT_SLOT_LIST) {
-    const tpt_entry en = S.entries[h.entry];
-    for (int k = 0; k < 5; ++k) f[k] = en.f[k];
-    word = en.a;
-    kind = en.b;
-    xf = en.xform;
-    if (xf != kNone) to_local(S.xforms[xf], &lo, &ld);
+  if (geo) {
+    for (int k = 0; k < 5; ++k) f[k] = geo->f[k];
+    kind = geo->kind, word = geo->word, xf = geo->xf;
+    lo = geo->lo, ld = geo->ld;
+  } else {
+    const slot_t s = load_slot(&S.slots[h.slot]);
+    kind = s.b >> 28;
+    for (int k = 0; k < 5; ++k) f[k] = s.f[k];
+    word = s.a;
+    if (S.seg_xf)
+      for (uint32_t g = 0; g < S.n_segments; ++g)
+        if (h.slot >= S.segments[2 * g] && h.slot < S.segments[2 * g + 1]) sx = S.seg_xf[g];
+    if ((sx & TPT_SEGMENT_PLAIN) != TPT_SEGMENT_PLAIN) to_local(S.xforms[sx & TPT_SEGMENT_PLAIN], &lo, &ld);
+    if (kind == TPT_SLOT_LIST) {
+      const tpt_entry en = S.entries[h.entry];
+      for (int k = 0; k < 5; ++k) f[k] = en.f[k];
+      word = en.a;
+      kind = en.b;
+      xf = en.xform;
+      if (xf != kNone) to_local(S.xforms[xf], &lo, &ld);
+    }
   }
   const float t = h.t;
   v3 pt{lo.x + t * ld.x, lo.y + t * ld.y, lo.z + t * ld.z};

@@ -181,17 +181,20 @@ __device__ __forceinline__ bool flat_in_plane(flat_scan_ptr p, uint32_t n, uint3
 // the reference's order.
 __device__ __forceinline__ bool flat_exact(const scene_view &S, uint32_t id, float t, v3 o, v3 d, v3 inv, float tmin,
                                            float tmax, bool lost, hit_t *h, uint32_t *leaf, uint32_t *order,
-                                           bool *rect) {
+                                           bool *rect, hit_geo *geo) {
   const float4 *q = reinterpret_cast<const float4 *>(S.fwins + id);
   const float4 q0 = q[0], q1 = q[1], q2 = q[2], q3 = q[3], q4 = q[4];
   const uint32_t word = __float_as_uint(q1.w), xf = __float_as_uint(q3.w);
   *rect = __float_as_uint(q4.x) == TPT_SLOT_RECT;
   bool got = true;
-  if (*rect) {
-    v3 lo = o, ld = d;
-    if (xf != kNone) to_local(S.xforms[xf], &lo, &ld);
-    const float f[5] = {q0.x, q0.y, q0.z, q0.w, q1.x};
-    got = rect_t(f, (word >> 28) & 3u, lo, ld, tmin, tmax, &t);
+  v3 lo = o, ld = d;
+  if (xf != kNone) to_local(S.xforms[xf], &lo, &ld);
+  const float f[5] = {q0.x, q0.y, q0.z, q0.w, q1.x};
+  if (*rect) got = rect_t(f, (word >> 28) & 3u, lo, ld, tmin, tmax, &t);
+  if (geo) {
+    for (int k = 0; k < 5; ++k) geo->f[k] = f[k];
+    geo->kind = __float_as_uint(q4.x), geo->word = word, geo->xf = xf;
+    geo->lo = lo, geo->ld = ld;
   }
   if (__float_as_uint(q3.z) && !lost) {
     const slot_t b{{q2.x, q2.y, q2.z, q2.w, q3.x, q3.y}, 0u, 0u};
@@ -259,8 +262,8 @@ __device__ __forceinline__ void flat_medium(const scene_view &S, flat_scan_ptr p
 }
 
 // All lanes of the wave call together.  Returns the hit of lanes that are
-// live and not slow; *slow: the lane needs the exact walk.  *leaf: the hit's
-// leaf id.
+// live and not slow; *slow: the lane needs the exact walk.  *leaf, *geo (may be
+// null): the hit's leaf id, its primitive and local ray.
 //
 // Zero direction components are ordinary here (lights without a sampler of
 // their own send rays along x): their reciprocal is infinite as the
@@ -278,7 +281,7 @@ __device__ __forceinline__ void flat_medium(const scene_view &S, flat_scan_ptr p
 // for a caller's own rays it keeps such lanes off the exact walk.
 template <bool TIES, bool MEDIA>
 __device__ __forceinline__ bool flat_world(const scene_view &S, v3 o, v3 d, const ray_ctx &rc, float tmin, float tmax, bool live,
-                                           hit_t *out, uint32_t *nodes, bool *slow, uint32_t *leaf = nullptr) {
+                                           hit_t *out, uint32_t *nodes, bool *slow, uint32_t *leaf, hit_geo *geo) {
   const bool zx = d.x == 0.0f, zy = d.y == 0.0f, zz = d.z == 0.0f;
   const v3 inv{zx ? __builtin_amdgcn_rcpf(d.x) : recip_rn(d.x), zy ? __builtin_amdgcn_rcpf(d.y) : recip_rn(d.y),
                zz ? __builtin_amdgcn_rcpf(d.z) : recip_rn(d.z)};
@@ -348,12 +351,12 @@ __device__ __forceinline__ bool flat_world(const scene_view &S, v3 o, v3 d, cons
   if (live && have && !amb) {
     uint32_t order, id;
     bool rect;
-    got = flat_exact(S, best.id, best.t1, o, d, inv, tmin, tmax, lost, out, &id, &order, &rect);
+    got = flat_exact(S, best.id, best.t1, o, d, inv, tmin, tmax, lost, out, &id, &order, &rect, geo);
     if (TIES && !lost && !(best.t2 > best.t1 + fabsf(best.t1) * 0x1p-18f)) {
       hit_t h;
       uint32_t order2, id2;
       bool rect2;
-      const bool got2 = flat_exact(S, best.id2, best.t2, o, d, inv, tmin, tmax, false, &h, &id2, &order2, &rect2);
+      const bool got2 = flat_exact(S, best.id2, best.t2, o, d, inv, tmin, tmax, false, &h, &id2, &order2, &rect2, nullptr);
       got = got && rect && rect2;
       if (got && got2 && (h.t < out->t || (h.t == out->t && order2 > order))) *out = h, id = id2;
     }
@@ -416,9 +419,10 @@ __device__ __forceinline__ bool segment_combine(const scene_view &S, uint32_t st
 // the lanes that need it.  All lanes of the wave call together.
 template <bool TIES = false, bool MEDIA = false>
 __device__ __forceinline__ bool small_world(const scene_view &S, v3 o, v3 d, const ray_ctx &rc, float tmin, float tmax,
-                                            hit_t *out, uint32_t *nodes, bool live, uint32_t *leaf = nullptr) {
+                                            hit_t *out, uint32_t *nodes, bool live, uint32_t *leaf = nullptr,
+                                            hit_geo *geo = nullptr) {
   bool slow;
-  bool got = flat_world<TIES, MEDIA>(S, o, d, rc, tmin, tmax, live, out, nodes, &slow, leaf);
+  bool got = flat_world<TIES, MEDIA>(S, o, d, rc, tmin, tmax, live, out, nodes, &slow, leaf, geo);
   if (__ballot(slow) != 0ull) {
     const v3 inv{1.0f / d.x, 1.0f / d.y, 1.0f / d.z};
     hit_t best{0.0f, kNone, kNone, 0};
@@ -437,6 +441,18 @@ __device__ __forceinline__ bool small_world(const scene_view &S, v3 o, v3 d, con
       got = any;
       *out = best;
       if (leaf && any) *leaf = leaf_id(S, best);
+      if (geo && any) {
+        const slot_t s = load_slot(&S.slots[best.slot]);
+        for (int k = 0; k < 5; ++k) geo->f[k] = s.f[k];
+        geo->kind = s.b >> 28, geo->word = s.a, geo->xf = kNone;
+        geo->lo = o, geo->ld = d;
+        if (best.entry != kNone) {
+          const tpt_entry en = S.entries[best.entry];
+          for (int k = 0; k < 5; ++k) geo->f[k] = en.f[k];
+          geo->kind = en.b, geo->word = en.a, geo->xf = en.xform;
+          if (en.xform != kNone) to_local(S.xforms[en.xform], &geo->lo, &geo->ld);
+        }
+      }
     }
   }
   return got;
