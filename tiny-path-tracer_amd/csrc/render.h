@@ -857,7 +857,7 @@ __global__ void __launch_bounds__(guide_shade_threads(SIMPLE)) __attribute__((am
   __shared__ uint32_t offs[NSUB];
   __shared__ uint32_t pre[NSUB + 1];
   __shared__ uint2 outs[guide_shade_threads(SIMPLE) * 10];  // entry e: outputs 4k..4k+3 as bf16 in outs[10 e + k]
-  guide_stage_weights(wt, P.g_tiles, GX_TILES * GX_TILE_WORDS);
+  guide_stage_weights<guide_shade_threads(SIMPLE), GX_TILES>(wt, P.g_tiles);
   for (int i = threadIdx.x; i < G_BIAS; i += blockDim.x) bias[i] = P.g_params[G_B1 + i];
   if (threadIdx.x < NSUB) offs[threadIdx.x] = mc_at(parity, Q_DIFFUSE, threadIdx.x);
   __syncthreads();

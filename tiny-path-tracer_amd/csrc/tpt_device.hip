@@ -847,10 +847,9 @@ struct tpt_guide {
   int device = 0;
   int n_cu = 256;
   float *params = nullptr;   // G_NPARAM_PAD + 1 (mix logit)
-  float *adam_m = nullptr, *adam_v = nullptr;
+  float *adam_m = nullptr, *adam_v = nullptr;  // adam_m: the allocation that holds the arrays down to scratch
   uint32_t *xtiles = nullptr;  // inference tiles, GX_TILES x 256 words
   uint32_t *rtiles = nullptr;  // training tiles, GR_TILES x 256 words
-  float *gacc = nullptr;       // gradient accumulator (G_NPARAM_PAD + 2), cleared by k_guide_adam
   float *partial = nullptr;    // train blocks x G_PARTIAL
   float *scratch = nullptr;    // gradient / loss staging (G_NPARAM_PAD + 2)
   int train_blocks = 0;
@@ -870,7 +869,8 @@ int guide_pack(tpt_guide *g, hipStream_t stream) {
 }
 
 // One fused forward/backward pass over rows [row0, row0 + n) (cyclic in
-// n_total), partials reduced by k_guide_reduce (mode 0: gradient, 1: Adam).
+// n_total; row0 < n_total, n <= n_total), partials consumed by k_guide_finish
+// (mode 0: gradient, 1: Adam).
 int guide_step(tpt_guide *g, const float *rows, uint64_t n, uint64_t row0, uint64_t n_total, int mode, float lr,
                float *grad, float *loss_dev, hipStream_t stream) {
   const int blocks =
@@ -880,12 +880,10 @@ int guide_step(tpt_guide *g, const float *rows, uint64_t n, uint64_t row0, uint6
                      n_total, g->partial);
   HIP_TRY(hipGetLastError());
   if (mode == 1) ++g->step;
-  const dim3 rgrid((G_NPARAM_PAD + 2 + 255) / 256, (blocks + PART_CHUNK - 1) / PART_CHUNK);
-  hipLaunchKernelGGL(k_guide_reduce, rgrid, dim3(256), 0, stream, g->partial, blocks, g->gacc);
-  hipLaunchKernelGGL(k_guide_adam, dim3((G_NPARAM_PAD + 2 + 255) / 256), dim3(256), 0, stream, g->gacc, g->params,
-                     g->adam_m, g->adam_v, grad, loss_dev, mode, lr, g->step);
+  hipLaunchKernelGGL(k_guide_finish, dim3((G_NPARAM_PAD + 2 + GF_PARAMS - 1) / GF_PARAMS), dim3(GF_THREADS), 0, stream,
+                     g->partial, blocks, g->params, g->adam_m, g->adam_v, grad, loss_dev, mode, lr, g->step,
+                     reinterpret_cast<uint16_t *>(g->xtiles), reinterpret_cast<uint16_t *>(g->rtiles));
   HIP_TRY(hipGetLastError());
-  if (mode == 1) return guide_pack(g, stream);
   return TPT_OK;
 }
 
@@ -2130,20 +2128,19 @@ int tpt_guide_create(uint64_t seed, tpt_guide **out) {
   g->n_cu = info_of(g->device).n_cu;
   g->train_blocks = g->n_cu;
   const size_t np = G_NPARAM_PAD + 1;
-  HIP_TRY(hipMalloc(&g->params, np * sizeof(float)));
-  HIP_TRY(hipMalloc(&g->adam_m, np * sizeof(float)));
-  HIP_TRY(hipMalloc(&g->adam_v, np * sizeof(float)));
-  HIP_TRY(hipMalloc(&g->xtiles, GX_TILES * GX_TILE_WORDS * sizeof(uint32_t)));
-  HIP_TRY(hipMemset(g->xtiles, 0, GX_TILES * GX_TILE_WORDS * sizeof(uint32_t)));
-  HIP_TRY(hipMalloc(&g->rtiles, GR_TILES * 256 * sizeof(uint32_t)));
-  HIP_TRY(hipMemset(g->rtiles, 0, GR_TILES * 256 * sizeof(uint32_t)));
-  HIP_TRY(hipMalloc(&g->gacc, (G_NPARAM_PAD + 2) * sizeof(float)));
-  HIP_TRY(hipMemset(g->gacc, 0, (G_NPARAM_PAD + 2) * sizeof(float)));
-  HIP_TRY(hipMalloc(&g->partial, static_cast<size_t>(g->train_blocks) * G_PARTIAL * sizeof(float)));
-  HIP_TRY(hipMalloc(&g->scratch, (G_NPARAM_PAD + 2) * sizeof(float)));
+  // one allocation for all of it; the Adam moments and the tiles start as zeros
+  const auto pad = [](size_t words) { return (words + 63) / 64 * 64; };
+  const size_t zeros = 2 * pad(np) + GX_TILES * GX_TILE_WORDS + GR_TILES * 256;
+  const size_t rest = 2 * pad(np + 1) + static_cast<size_t>(g->train_blocks) * G_PARTIAL;
+  HIP_TRY(hipMalloc(&g->adam_m, (zeros + rest) * sizeof(float)));
+  HIP_TRY(hipMemset(g->adam_m, 0, zeros * sizeof(float)));
+  g->adam_v = g->adam_m + pad(np);
+  g->xtiles = reinterpret_cast<uint32_t *>(g->adam_v + pad(np));
+  g->rtiles = g->xtiles + GX_TILES * GX_TILE_WORDS;
+  g->params = g->adam_m + zeros;
+  g->scratch = g->params + pad(np + 1);
+  g->partial = g->scratch + pad(np + 1);
   HIP_TRY(hipMemcpy(g->params, h.data(), np * sizeof(float), hipMemcpyHostToDevice));
-  HIP_TRY(hipMemset(g->adam_m, 0, np * sizeof(float)));
-  HIP_TRY(hipMemset(g->adam_v, 0, np * sizeof(float)));
   HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_guide_train),
                               hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(k_guide_train_lds())));
   const int rc = guide_pack(g, nullptr);
@@ -2156,14 +2153,7 @@ int tpt_guide_create(uint64_t seed, tpt_guide **out) {
 int tpt_guide_destroy(tpt_guide *g) {
   if (!g) return TPT_OK;
   (void)hipDeviceSynchronize();
-  (void)hipFree(g->params);
   (void)hipFree(g->adam_m);
-  (void)hipFree(g->adam_v);
-  (void)hipFree(g->xtiles);
-  (void)hipFree(g->rtiles);
-  (void)hipFree(g->gacc);
-  (void)hipFree(g->partial);
-  (void)hipFree(g->scratch);
   (void)hipFree(g->rec_side);
   (void)hipFree(g->rec_rows);
   delete g;
