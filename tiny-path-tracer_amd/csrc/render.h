@@ -1036,16 +1036,30 @@ __global__ void __launch_bounds__(256) k_tail(scene_view S, const tpt_slot *__re
   const uint32_t home = blockIdx.x % NSUB;
   uint32_t st[ST_COUNT] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
   const uint32_t stride = gridDim.x * blockDim.x;
-  for (uint32_t base = blockIdx.x * blockDim.x; base < count; base += stride) {
-    const uint32_t qi = base + threadIdx.x;
-    bool live = qi < count;
-    path p{};
-    if (live) {
-      const uint32_t r = find_region(pre, NSUB, qi);
-      p = load_ray(in, r * Q.region + (qi - pre[r]));
+  // The wave's records: 64 at `chunk`, the next 64 a stride on; lanes whose path
+  // has ended take the next ones, so a wave stays full while there are any.
+  uint32_t chunk = blockIdx.x * blockDim.x + __builtin_amdgcn_readfirstlane(threadIdx.x / 64) * 64, used = 0;
+  bool live = false;
+  path p{};
+  for (;;) {
+    unsigned long long dead = __ballot(!live);
+    while (dead != 0ull && chunk < count) {
+      const uint32_t left = min(64u, count - chunk) - used;
+      const uint32_t rank = lane_prefix(dead);
+      const bool take = !live && rank < left;
+      if (take) {
+        const uint32_t qi = chunk + used + rank, r = find_region(pre, NSUB, qi);
+        p = load_ray(in, r * Q.region + (qi - pre[r]));
+        live = true;
+      }
+      const uint32_t taken = __popcll(__ballot(take));
+      used += taken;
+      if (taken == left) chunk += stride, used = 0;
+      dead = __ballot(!live);
     }
     // wave-uniform: the sweep needs every lane of the wave
-    while (__ballot(live) != 0ull) {
+    if (__ballot(live) == 0ull) break;
+    {
       const item_ctx c = live ? item_in_entry(P, MULTI ? p.ent : 0u, p.item) : item_ctx{0u, 0u, 0u, 0u};
       const scene_view Sj = view_of<MULTI>(S, P, c.job);
       hit_t h{0.0f, kNone, kNone, 0};

@@ -1033,6 +1033,7 @@ int grow_device(T **p, uint32_t *cap, uint32_t need) {
 
 // Live-count polls of the bounce loop (see render_core).
 constexpr uint64_t kPoll = 16, kPollFirst = 8, kPollTail = 4;
+constexpr uint32_t kEarlyTail = 4;  // guided vertices per path up to which the tail follows them directly
 
 struct bounce_launch {
   scene_view S;
@@ -1527,9 +1528,10 @@ int render_core(tpt_scene *s, const tpt_job *jobs, uint32_t n_jobs, const tpt_la
   double tail_ms = 0.0;
   uint64_t n_tail = 0;
   auto run_tail = [&](uint32_t q, uint64_t live) -> int {
-    // at least NSUB blocks (the hand-back appends stay within their regions)
-    const uint32_t blocks =
-        static_cast<uint32_t>(std::max<uint64_t>(NSUB, std::min<uint64_t>(grid, (live + 255) / 256)));
+    // at most what stays resident, a multiple of NSUB, and at least NSUB blocks:
+    // a region's blocks hand back at most their share of the records
+    const uint64_t most = std::max<uint64_t>(std::min<uint64_t>(grid, 4ull * s->n_cu) / NSUB * NSUB, NSUB);
+    const uint32_t blocks = static_cast<uint32_t>(std::max<uint64_t>(NSUB, std::min<uint64_t>(most, (live + 255) / 256)));
     if (profile) HIP_TRY(hipEventRecord(s->events[0], ws));
     launch_tail(B, ws, q, blocks);
     if (profile) {
@@ -1589,7 +1591,13 @@ int render_core(tpt_scene *s, const tpt_job *jobs, uint32_t n_jobs, const tpt_la
       }
     } else {
       int batch = 0;
-      uint64_t next_poll = (B.tail ? kPollFirst : static_cast<uint64_t>(poll)) - 1;
+      // Guided, every item's path in flight from the start, and the guide asked
+      // at its first few diffuse vertices only: after that many iterations nearly
+      // every path goes on unguided, so the tail (whose waves refill from the
+      // queue) takes them at once, and again what each shading of handed-back
+      // vertices leaves.
+      const bool early = B.tail && B.guided && exhausted && P.guide_verts <= kEarlyTail;
+      uint64_t next_poll = (early ? P.guide_verts : (B.tail ? kPollFirst : static_cast<uint64_t>(poll))) - 1;
       for (uint64_t it = 0; it < max_iter; ++it) {
         const uint32_t parity = static_cast<uint32_t>(it & 1u);
         if (profile) HIP_TRY(hipEventRecord(s->events[2 * batch], ws));
@@ -1608,7 +1616,7 @@ int render_core(tpt_scene *s, const tpt_job *jobs, uint32_t n_jobs, const tpt_la
             break;
           }
           exhausted = exhausted || live < cap;
-          if (B.tail && exhausted && live <= tail_live) {
+          if (B.tail && exhausted && (early || live <= tail_live)) {
             if ((rc = run_tail(parity ^ 1u, live)) != TPT_OK) return rc;
             if (!B.guided) {
               drained = true;
@@ -1619,6 +1627,13 @@ int render_core(tpt_scene *s, const tpt_job *jobs, uint32_t n_jobs, const tpt_la
             launch_shade(B, ws, parity ^ 1u);
             ++it;
             if ((rc = live_count(parity, &live)) != TPT_OK) return rc;
+            // a path is handed back at most guide_verts times
+            for (uint32_t q = parity; early && live > 0; q ^= 1u) {
+              if ((rc = run_tail(q, live)) != TPT_OK) return rc;
+              launch_shade(B, ws, q);
+              ++it;
+              if ((rc = live_count(q ^ 1u, &live)) != TPT_OK) return rc;
+            }
             if (live == 0) {
               drained = true;
               break;
