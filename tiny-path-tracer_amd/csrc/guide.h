@@ -209,15 +209,6 @@ __device__ __forceinline__ void guide_forward_groups(bf16x8 xb[NB][2], const uin
   }
 }
 
-__device__ __forceinline__ void guide_forward_x32(const bf16x8 xb_in[2], const uint32_t *xt, const float *bias,
-                                                  f32x4 out[3]) {
-  bf16x8 xb[1][2] = {{xb_in[0], xb_in[1]}};
-  f32x4 o[1][3];
-  guide_forward_groups<1>(xb, xt, bias, o);
-#pragma unroll
-  for (int mt = 0; mt < 3; ++mt) out[mt] = o[0][mt];
-}
-
 // ---------------------------------------------------------------- vMF mix ---
 struct vmf_mix {
   float mu[G_LOBES][3];

@@ -828,10 +828,13 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SIMPLE
 
 // Guided mode, diffuse queue: network inference fused with the guided
 // shading.  Each lane gathers one entry (path, hit record, encoding inputs);
-// the wave then runs four MFMA passes of 16 entries, lane l taking the inputs
-// of entry 16j + l%16 by shuffle.  A pass leaves outputs 16mt + 4(l/16) .. +3
+// the wave then runs MFMA passes over two groups of 16 entries (a weight tile
+// read serves both: 768 -> 755 us per 4.9 million vertices), lane l taking the
+// inputs of entry 16j + l%16 by shuffle.  A pass leaves outputs 16mt + 4(l/16) .. +3
 // of that entry in lane l's D tiles; they go to the wave's rows of an LDS
-// table (bf16) from which every lane reads its own entry's 40 outputs.
+// table (bf16) from which every lane reads its own entry's 40 outputs.  What
+// bounds it: vector issue (61% busy), about 3500 instructions per 64 vertices,
+// half of them the mixture and its sampling.
 //
 // One-sample MIS of the guide g with the reference sampler q (the
 // reference's mixture_pdf(hitable_pdf, cosine_pdf), src/material.cc:3-17,
@@ -849,6 +852,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SIMPLE
 __host__ __device__ constexpr uint32_t guide_shade_threads(bool simple) { return simple ? 512u : 256u; }
 __host__ __device__ constexpr uint32_t guide_shade_blocks_per_cu(bool simple) { return simple ? 2u : 3u; }
 
+constexpr int GS_GROUPS = 2;  // groups of 16 entries per network pass
 template <bool MULTI, bool SIMPLE = false>
 __global__ void __launch_bounds__(guide_shade_threads(SIMPLE)) __attribute__((amdgpu_waves_per_eu(SIMPLE ? 4 : 3))) k_guide_shade(scene_view S, render_params P, render_state Q, uint32_t parity) {
   const pass_hdr H = *P.hdr;
@@ -906,22 +910,25 @@ __global__ void __launch_bounds__(guide_shade_threads(SIMPLE)) __attribute__((am
       }
     }
 #pragma unroll 1
-    for (uint32_t j = 0; j < 4; ++j) {
+    for (uint32_t j = 0; j < 4; j += GS_GROUPS) {
       if (base + wave_base + 16 * j >= total) break;  // wave-uniform
-      const int src = static_cast<int>(16 * j) + sl;
-      float x9[9];
+      bf16x8 xb[GS_GROUPS][2];
+      f32x4 o[GS_GROUPS][3];
 #pragma unroll
-      for (int k = 0; k < 9; ++k) x9[k] = __shfl(in9[k], src);
-      bf16x8 xb[2];
-      guide_xfeatures(fg, fg == 0 ? x9[0] : (fg == 1 ? x9[1] : x9[2]), x9 + 3, xb);
-      f32x4 o[3];
-      guide_forward_x32(xb, wt, bias, o);
-      uint2 *row = outs + (wave_base + 16 * j + sl) * 10;
+      for (int q = 0; q < GS_GROUPS; ++q) {
+        const int src = static_cast<int>(16 * (j + q)) + sl;
+        float x9[9];
 #pragma unroll
-      for (int mt = 0; mt < 3; ++mt) {
-        const int k = 4 * mt + fg;
+        for (int k = 0; k < 9; ++k) x9[k] = __shfl(in9[k], src);
+        guide_xfeatures(fg, fg == 0 ? x9[0] : (fg == 1 ? x9[1] : x9[2]), x9 + 3, xb[q]);
+      }
+      guide_forward_groups<GS_GROUPS>(xb, wt, bias, o);
+#pragma unroll
+      for (int e = 0; e < 3 * GS_GROUPS; ++e) {
+        const int q = e / 3, mt = e % 3, k = 4 * mt + fg;
+        uint2 *row = outs + (wave_base + 16 * (j + q) + sl) * 10;
         if (k < 10) {
-          const bf16x4 b = pack4(o[mt][0], o[mt][1], o[mt][2], o[mt][3]);
+          const bf16x4 b = pack4(o[q][mt][0], o[q][mt][1], o[q][mt][2], o[q][mt][3]);
           row[k] = make_uint2(static_cast<uint32_t>(static_cast<uint16_t>(b[0])) |
                                   (static_cast<uint32_t>(static_cast<uint16_t>(b[1])) << 16),
                               static_cast<uint32_t>(static_cast<uint16_t>(b[2])) |
