@@ -1573,10 +1573,6 @@ int render_core(tpt_scene *s, const tpt_job *jobs, uint32_t n_jobs, const tpt_la
         exhausted = exhausted || live < cap;
         if (B.tail && exhausted && live <= tail_live) {
           if ((rc = run_tail(0, live)) != TPT_OK) return rc;
-          if (!B.guided) {
-            drained = true;
-            break;
-          }
           // handed-back guided vertices: shade them and bring their paths
           // back to queue 0, where the next replay starts
           launch_shade(B, ws, 0);
@@ -1591,12 +1587,13 @@ int render_core(tpt_scene *s, const tpt_job *jobs, uint32_t n_jobs, const tpt_la
       }
     } else {
       int batch = 0;
-      // Guided, every item's path in flight from the start, and the guide asked
-      // at its first few diffuse vertices only: after that many iterations nearly
+      // (B.tail here means guided: plain renders take k_paths.)  Every item's path
+      // in flight from the start, and the guide asked at its first few diffuse
+      // vertices only: after that many iterations nearly
       // every path goes on unguided, so the tail (whose waves refill from the
       // queue) takes them at once, and again what each shading of handed-back
       // vertices leaves.
-      const bool early = B.tail && B.guided && exhausted && P.guide_verts <= kEarlyTail;
+      const bool early = B.tail && exhausted && P.guide_verts <= kEarlyTail;
       uint64_t next_poll = (early ? P.guide_verts : (B.tail ? kPollFirst : static_cast<uint64_t>(poll))) - 1;
       for (uint64_t it = 0; it < max_iter; ++it) {
         const uint32_t parity = static_cast<uint32_t>(it & 1u);
@@ -1618,10 +1615,6 @@ int render_core(tpt_scene *s, const tpt_job *jobs, uint32_t n_jobs, const tpt_la
           exhausted = exhausted || live < cap;
           if (B.tail && exhausted && (early || live <= tail_live)) {
             if ((rc = run_tail(parity ^ 1u, live)) != TPT_OK) return rc;
-            if (!B.guided) {
-              drained = true;
-              break;
-            }
             // handed-back guided vertices: shade them; their paths continue
             // in queue `parity`, the input of iteration it + 2
             launch_shade(B, ws, parity ^ 1u);
