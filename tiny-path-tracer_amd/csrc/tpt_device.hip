@@ -1165,18 +1165,25 @@ void launch_shade(const bounce_launch &B, hipStream_t st, uint32_t parity) {
   }
 }
 
-// Column sums of `rows` per-block statistics rows into out[0..ST_COUNT).
-__global__ void __launch_bounds__(256) k_stats_total(const unsigned long long *stats, uint32_t rows,
-                                                       unsigned long long *out) {
-  __shared__ unsigned long long part[256];
-  constexpr uint32_t kLanes = 256 / ST_COUNT;  // partial sums per counter
+// Column sums of `rows` per-block statistics rows into out[0..ST_COUNT).  One
+// block, bound by the latency of its chain of loads: 16 in flight per thread
+// (8192 rows: 100 us with 256 threads and one at a time, 30 us so).
+constexpr uint32_t kTotalThreads = 1024;
+__global__ void __launch_bounds__(kTotalThreads) k_stats_total(const unsigned long long *__restrict__ stats,
+                                                               uint32_t rows, unsigned long long *__restrict__ out) {
+  __shared__ unsigned long long part[kTotalThreads];
+  constexpr uint32_t kLanes = kTotalThreads / ST_COUNT;  // partial sums per counter
   const uint32_t k = threadIdx.x % ST_COUNT, lane = threadIdx.x / ST_COUNT;
   unsigned long long v = 0;
-  for (uint32_t r = lane; r < rows; r += kLanes) v += stats[static_cast<size_t>(r) * ST_COUNT + k];
+  if (lane < kLanes) {
+#pragma unroll 16
+    for (uint32_t r = lane; r < rows; r += kLanes) v += stats[static_cast<size_t>(r) * ST_COUNT + k];
+  }
   part[threadIdx.x] = v;
   __syncthreads();
   if (threadIdx.x < ST_COUNT) {
     unsigned long long t = 0;
+#pragma unroll 17
     for (uint32_t l = 0; l < kLanes; ++l) t += part[l * ST_COUNT + threadIdx.x];
     out[threadIdx.x] = t;
   }
@@ -1260,7 +1267,7 @@ int render_paths(tpt_scene *s, const std::vector<job_dev> &jd, const std::vector
       hipLaunchKernelGGL(k_accumulate<false>, ag, dim3(256), 0, ws, B.P, static_cast<const float *>(s->Q.res));
   }
   unsigned long long *tot = reinterpret_cast<unsigned long long *>(s->tables + at_tot);
-  hipLaunchKernelGGL(k_stats_total, dim3(1), dim3(256), 0, ws, static_cast<const unsigned long long *>(s->Q.stats),
+  hipLaunchKernelGGL(k_stats_total, dim3(1), dim3(kTotalThreads), 0, ws, static_cast<const unsigned long long *>(s->Q.stats),
                      grid, tot);
   HIP_TRY(hipGetLastError());
   HIP_TRY(hipEventRecord(s->ev_end, ws));
@@ -1649,9 +1656,15 @@ int render_core(tpt_scene *s, const tpt_job *jobs, uint32_t n_jobs, const tpt_la
   }
   HIP_TRY(hipGetLastError());
   HIP_TRY(hipEventRecord(e1, ws));
-  std::vector<unsigned long long> st(static_cast<size_t>(n_stat) * ST_COUNT);
-  HIP_TRY(hipMemcpyAsync(st.data(), s->Q.stats, st.size() * sizeof(unsigned long long), hipMemcpyDeviceToHost, ws));
+  // the totals, between the first two counters, come back through the pinned count buffer
+  static_assert(8 * sizeof(uint32_t) + ST_COUNT * sizeof(unsigned long long) <= CSTRIDE * sizeof(uint32_t), "gap");
+  unsigned long long tot[ST_COUNT], *d_tot = reinterpret_cast<unsigned long long *>(s->Q.counters + 8);
+  hipLaunchKernelGGL(k_stats_total, dim3(1), dim3(kTotalThreads), 0, ws, static_cast<const unsigned long long *>(s->Q.stats),
+                     n_stat, d_tot);
+  HIP_TRY(hipGetLastError());
+  HIP_TRY(hipMemcpyAsync(s->host_count, d_tot, sizeof(tot), hipMemcpyDeviceToHost, ws));
   HIP_TRY(hipStreamSynchronize(ws));
+  std::memcpy(tot, s->host_count, sizeof(tot));
   if (use_graph) {
     HIP_TRY(hipEventRecord(s->ev_out, ws));
     HIP_TRY(hipStreamWaitEvent(cs, s->ev_out, 0));
@@ -1662,9 +1675,6 @@ int render_core(tpt_scene *s, const tpt_job *jobs, uint32_t n_jobs, const tpt_la
   (void)hipEventDestroy(e1);
   if (!drained) return tpt::fail(TPT_ERR_HIP, "tpt_render: bounce loop did not drain");
   if (stats) {
-    unsigned long long tot[ST_COUNT] = {0};
-    for (uint32_t b = 0; b < n_stat; ++b)
-      for (int k = 0; k < ST_COUNT; ++k) tot[k] += st[static_cast<size_t>(b) * ST_COUNT + k];
     stats->paths = tot[ST_PATHS];
     stats->segments = tot[ST_SEGMENTS];
     stats->light_queries = tot[ST_LIGHT];
@@ -1943,7 +1953,7 @@ int render_noalloc(tpt_scene *s, const tpt_camera *camera, const tpt_render_desc
                        P, static_cast<const float *>(Q.res));
     s0 += take;
   }
-  hipLaunchKernelGGL(k_stats_total, dim3(1), dim3(256), 0, ws, static_cast<const unsigned long long *>(Q.stats),
+  hipLaunchKernelGGL(k_stats_total, dim3(1), dim3(kTotalThreads), 0, ws, static_cast<const unsigned long long *>(Q.stats),
                      grid, d_totals);
   HIP_TRY(hipGetLastError());
   // the totals come back through the scene's pinned count buffer (8 KB)
