@@ -256,6 +256,7 @@ def cpu_baseline(scene, w, h, spp, every, depth):
     else:
         O = Oracle()
         s = O.scene(scene)
+        spp = min(spp, 16)  # no snapshots to reach: enough for its rate
         t0 = time.perf_counter()
         s.render(w, h, spp, max_depth=depth, rng_mode=1, nthreads=cores)
         dt = time.perf_counter() - t0

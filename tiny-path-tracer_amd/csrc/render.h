@@ -1016,7 +1016,10 @@ __global__ void __launch_bounds__(guide_shade_threads(SIMPLE)) __attribute__((am
 // in registers: the trace of k_trace (the same walk), then shade_hit, the
 // shading of k_shade, until the path ends.  Same functions and Philox streams,
 // so every sample equals the bounce loop's bit for bit.  SIMPLE scenes only
-// (constant textures, at most one rect light, no motion or media).
+// (constant textures, at most one rect light, no motion or media).  A wave's
+// lanes take the next record when their path ends, so it may also be given
+// every path of a pass: guided renders do so after the guided vertices (Cornell
+// box 600 x 600 x 16: 509 us in place of 1.1 ms of bounces and the old tail).
 //
 // Guided mode: a path that reaches a guided diffuse vertex needs the network
 // (k_guide_shade, a wave-wide MFMA pass); it is handed back instead, its
