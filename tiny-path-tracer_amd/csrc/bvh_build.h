@@ -204,7 +204,6 @@ inline bvh_scene build_bvh(const tpt_flat_scene &f, uint32_t sb, std::vector<bvh
   bvh_builder b;
   b.nodes = nodes;
   b.items.reserve(all.size());
-  nodes->reserve(nodes->size() + all.size());
   bvh_builder::box field;
   for (uint32_t i = n_big; i < all.size(); ++i) {
     b.items.push_back({{all[i].c[0], all[i].c[1], all[i].c[2]}, std::fabs(all[i].r), leaf0 + i});
