@@ -8,7 +8,7 @@
 #include <cstring>
 #include <vector>
 
-#include "dev_common.h"
+#include "records.h"
 
 namespace tptd {
 
@@ -92,9 +92,10 @@ struct bvh_builder {
     }
     return mid;
   }
+  // (compared as floats: a conversion to int is only defined in its range)
   static int bin(float c, float lo, float scale) {
-    const int q = static_cast<int>((c - lo) * scale);
-    return q < kBins - 1 ? q : kBins - 1;
+    const float q = (c - lo) * scale;
+    return q < kBins - 1 ? (q > 0.0f ? static_cast<int>(q) : 0) : kBins - 1;
   }
 
   // Builds [first, first + count) with at most `levels` levels of nodes;
@@ -122,9 +123,12 @@ struct bvh_builder {
         float best = INFINITY;
         int axis = -1, at = 0;
         // large sets along their widest axis only: the other cuts matter near the leaves
+        // (no bins where the centres are so close that their scale overflows)
         for (int k = 0; k < 3; ++k)
-          if (k == wide || (count <= 512 && hi[k] - lo[k] > 0.25f * (hi[wide] - lo[wide])))
-            cut(first, count, k, lo[k], kBins / (hi[k] - lo[k]), &best, &axis, &at);
+          if (k == wide || (count <= 512 && hi[k] - lo[k] > 0.25f * (hi[wide] - lo[wide]))) {
+            const float scale = kBins / (hi[k] - lo[k]);
+            if (std::isfinite(scale)) cut(first, count, k, lo[k], scale, &best, &axis, &at);
+          }
         if (axis >= 0) {
           const float scale = kBins / (hi[axis] - lo[axis]), l = lo[axis];
           const auto it = std::partition(items.begin() + first, items.begin() + first + count,
@@ -132,7 +136,7 @@ struct bvh_builder {
           mid = static_cast<uint32_t>(it - items.begin()) - first;
         }
       }
-      if (mid == 0 || mid == count) {  // no room for an uneven split, or equal centres
+      if (mid == 0 || mid == count) {  // no room for an uneven split, or centres (almost) equal
         mid = count / 2;
         std::nth_element(items.begin() + first, items.begin() + first + mid, items.begin() + first + count,
                          [&](const item &a, const item &b) { return a.c[wide] < b.c[wide]; });
