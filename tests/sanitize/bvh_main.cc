@@ -1,12 +1,16 @@
 // The host build of the sphere tree (csrc/bvh_build.h) on scenes whose centres
 // spread by anything from nothing to 1e14, among them spreads too small for a
 // finite bin scale.  Each tree is checked: every sphere below the root once, each
-// box holding its subtree, no more levels than the walk's stack takes.
+// box holding its subtree, no more levels than the walk's stack takes.  And the
+// check of a scene's own boxes (csrc/tree_check.h): passed by every named scene,
+// failed by each way of breaking a tree.
 #include <cstdio>
 #include <cstdlib>
 #include <random>
+#include <string>
 
 #include "../../tiny-path-tracer_amd/csrc/bvh_build.h"
+#include "../../tiny-path-tracer_amd/csrc/tree_check.h"
 
 using namespace tptd;
 
@@ -70,10 +74,56 @@ std::vector<tpt_slot> spheres(uint32_t n, float spread, int axes, float r) {
   return s;
 }
 
+bool regular() {
+  bool ok = true;
+  std::string names = tpt_scene_names();
+  for (size_t a = 0; a < names.size();) {
+    const size_t b = std::min(names.find(',', a), names.size());
+    std::string name = names.substr(a, b - a);
+    a = b + 1;
+    if (name == "random_spheres_n<N>") name = "random_spheres_n3000";
+    tpt_host_scene *hs = nullptr;
+    if (tpt_host_scene_build(name.c_str(), 5489, &hs) != TPT_OK) continue;  // (no earth map here)
+    tpt_flat_scene f;
+    bool good = tpt_host_scene_flat(hs, &f) == TPT_OK && regular_trees(f);
+    std::vector<tpt_slot> own(f.slots, f.slots + f.n_slots);
+    f.slots = own.data();
+    uint32_t tried = 0;
+    for (uint32_t i = 0; i < f.n_slots && tried < 200; ++i) {
+      const tpt_slot was = own[i];
+      if ((was.b >> 28) != TPT_SLOT_BOX) continue;
+      ++tried;
+      const bool inner = i + 1 < f.n_slots && (own[i + 1].b >> 28) == TPT_SLOT_BOX;
+      if (inner) {  // a bound that no longer reaches its child's
+        own[i].f[1] = std::nextafter(own[i + 1].f[1], INFINITY);
+        good = good && !regular_trees(f);
+        own[i] = was;
+        own[i].f[5] = NAN;
+        good = good && !regular_trees(f);
+        own[i] = was;
+      }
+      own[i].a = was.a - 1;
+      good = good && !regular_trees(f);
+      own[i] = was;
+      if ((was.b & TPT_PAYLOAD_MASK) != TPT_NO_RIGHT) {
+        own[i].b = was.b + 1;
+        good = good && !regular_trees(f);
+        own[i].b = TPT_NO_RIGHT;
+        good = good && !regular_trees(f);
+        own[i] = was;
+      }
+    }
+    std::printf("%-28s %6u slots, %u boxes broken: %s\n", name.c_str(), f.n_slots, tried, good ? "ok" : "BAD");
+    tpt_host_scene_destroy(hs);
+    ok = ok && good;
+  }
+  return ok;
+}
+
 }  // namespace
 
 int main() {
-  bool ok = true;
+  bool ok = regular();
   char name[64];
   for (uint32_t n : {1u, 2u, 3u, 8u, 9u, 12u, 20u, 513u, 4000u})
     for (float spread : {0.0f, 1e-45f, 1e-39f, 2e-38f, 4.7e-38f, 1e-37f, 1e-20f, 1.0f, 1e14f})

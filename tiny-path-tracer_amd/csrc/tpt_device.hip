@@ -15,6 +15,7 @@
 #include "guide_train.h"
 #include "paths.h"
 #include "render.h"
+#include "tree_check.h"
 
 #include <random>
 
@@ -784,6 +785,8 @@ int create_pool(const tpt_flat_scene *scenes, uint32_t n, tpt_scene **out) {
     bool wrapped = false;
     for (uint32_t g = 0; f.segment_xforms && g < f.n_segments; ++g) wrapped |= f.segment_xforms[g] != TPT_SEGMENT_PLAIN;
     sweep[k] = f.n_slots <= 64 && !motion[k] && !wrapped;
+    const bool regular = (sweep[k] || sph[k]) && regular_trees(f);  // what both walks take for granted
+    sweep[k] = sweep[k] && regular;
     if (sweep[k]) {
       flat_of[k] = flat_records(f, static_cast<uint32_t>(sb), static_cast<uint32_t>(eb), static_cast<uint32_t>(xb),
                                 static_cast<uint32_t>(mb), &flat, &fwins, &fgroups);
@@ -791,7 +794,8 @@ int create_pool(const tpt_flat_scene *scenes, uint32_t n, tpt_scene **out) {
     }
     if (wrapped) sph[k] = 0;  // the sphere-only walk is built without segment transforms
     std::memset(&bscn[k], 0, sizeof(bscn[k]));
-    if (sph[k]) bscn[k] = build_bvh(f, static_cast<uint32_t>(sb), &bnodes, &bleaves);
+    bscn[k].root = kBvhNone;
+    if (sph[k] && regular) bscn[k] = build_bvh(f, static_cast<uint32_t>(sb), &bnodes, &bleaves);
     plain[k] = !motion[k] && (f.n_lights == 0 || (f.light_mode == 0 && f.lights[0].kind == TPT_LIGHT_XZ_RECT));
     for (uint32_t t = 0; t < f.n_textures; ++t) plain[k] = plain[k] && f.textures[t].kind == TPT_TEX_CONSTANT;
     simple[k] = plain[k] && !media[k];

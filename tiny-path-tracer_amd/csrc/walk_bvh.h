@@ -17,12 +17,12 @@
 //
 // Why the answer is the reference's, bit for bit.  bvh_node::hit tests a
 // sphere exactly when its parent node's box passes the slab test (the boxes
-// above are supersets, and slab arithmetic is monotone in the bounds), and
-// keeps the smallest t, at equal t the last sphere in its order.  So the
-// answer is the minimum over the spheres that are hit and whose parent box
-// passes: any tree may find the candidates, as long as it skips none.  Each
-// candidate is then tested with the reference's arithmetic, its parent box
-// too, and ties go by its rank.
+// above are supersets, as tree_check.h makes sure, and slab arithmetic is
+// monotone in the bounds), and keeps the smallest t, at equal t the last sphere
+// in its order.  So the answer is the minimum over the spheres that are hit and
+// whose parent box passes: any tree may find the candidates, as long as it skips
+// none.  Each candidate is then tested with the reference's arithmetic, its
+// parent box too, and ties go by its rank.
 //
 // No candidate is skipped because every box is grown by the distance at which
 // float rounding can still report a hit.  With u = 2^-24 and D the distance of
