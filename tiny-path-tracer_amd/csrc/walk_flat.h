@@ -293,10 +293,14 @@ __device__ __forceinline__ bool flat_world(const scene_view &S, v3 o, v3 d, cons
   // (fmaxf drops NaNs: they are looked for in the sum)
   const float sum = ((o.x + o.y) + o.z) + ((d.x + d.y) + d.z);
   const bool lost = o.x != o.x && o.y != o.y && o.z != o.z;
-  bool odd = !(big < 0x1p60f) || sum != sum || !(fabsf(tmax) < INFINITY) || !(tmin <= tmax);
+  // Every time below is finite then, so an infinite limit is as good as the
+  // largest number, but for a zero direction: that one hits every rect at t = +-inf.
+  const bool unlimited = !(tmax <= kFltMaxT) || !(tmin >= -kFltMaxT);
+  const float t_near = fmaxf(tmin, -kFltMaxT), t_far = fminf(tmax, kFltMaxT);
+  bool odd = !(big < 0x1p60f) || sum != sum || !(tmin <= tmax) || (unlimited & zx & zy & zz);
   const bool zero = live && !odd && (zx || zy || zz);
   const bool any_zero = __ballot(zero) != 0ull;
-  const float tlo = tmin - fabsf(tmin) * 0x1p-19f;
+  const float tlo = t_near - fabsf(t_near) * 0x1p-19f;
   flat_best best{INFINITY, INFINITY, INFINITY, -INFINITY, kNone, kNone};
   flat_scan_ptr p = (flat_scan_ptr)(S.flat);
   flat_group_ptr groups = (flat_group_ptr)(S.fgroups);
@@ -337,14 +341,15 @@ __device__ __forceinline__ bool flat_world(const scene_view &S, v3 o, v3 d, cons
   }
   *nodes += live ? visits : 0u;
   // beyond t_max by more than its error: a certain miss
-  bool have = best.id != kNone && !(best.t1 > tmax + fabsf(tmax) * 0x1p-19f);
+  bool have = best.id != kNone && !(best.t1 > t_far + fabsf(t_far) * 0x1p-19f);
   bool amb = odd;
-  if (lost && tmin <= tmax && fabsf(tmax) < INFINITY) {
+  if (lost && tmin <= tmax) {
     best.id = S.flat_nan;
     have = best.id != kNone;
     amb = false;
   } else if (have) {
-    amb = amb || best.e1 > -m || !(best.t1 > tmin + fabsf(tmin) * 0x1p-19f) || !(best.t1 < tmax - fabsf(tmax) * 0x1p-19f) ||
+    amb = amb || best.e1 > -m || !(best.t1 > t_near + fabsf(t_near) * 0x1p-19f) ||
+          !(best.t1 < t_far - fabsf(t_far) * 0x1p-19f) ||
           !((TIES ? best.t3 : best.t2) > best.t1 + fabsf(best.t1) * 0x1p-18f);
   }
   bool got = false;
