@@ -153,6 +153,7 @@ struct flat_range {
   uint32_t scan0 = 0, win0 = 0, group0 = 0, n_groups = 0, n_scans = 0;
   uint32_t nan_win = 0xFFFFFFFFu;
   float mag = 0.0f;
+  bool walk = false;  // path launches walk all the same
 };
 
 // A scene handle: one or more flattened scenes packed into one pool (indices
@@ -464,12 +465,34 @@ float rebase_bits(float f, uint32_t base) {
 // its slots and lists, grouped by wrapper chain; six rects in a row of one
 // list that close a box become one record.  sb, eb, xb, mb: the scene's first
 // slot, entry, transform and material in the pool.
-constexpr uint32_t kFlatMax = 64;  // most primitives of the pass
+//
+// Every scene that the pass can take (at most 64 slots, the width of
+// segment_combine's mask) goes through it, however long its lists: against the
+// wave's sweep that it replaced, 2^21 rays in lists of 66 to 2400 rects that
+// close boxes 214 -> 79 us to 6.3 -> 2.4 ms, in 100 and 300 spheres 240 -> 167
+// and 640 -> 488 us, in 32 lists of 4 to 50 spheres under a bvh 415 -> 230 us to
+// 3.1 -> 2.3 ms.  (Per-lane walks of these take 0.46 to 1.05 times the sweep's
+// speed, and guided renders of them have no k_tail.)
+//
+// One kind of scene is rendered faster by path launches that walk (walk): many
+// spheres, whose exact test is the pass's most expensive, in lists whose parent
+// boxes few rays cross.  400 x 401 x 16, pass and walk, with the mean share of the
+// scene's box area that those boxes have: 32 lists of 4, 8, 16, 50 spheres, 5 to 7%:
+// 449 and 448 us, 1.02 and 0.78 ms, 2.23 and 1.56, 8.1 and 6.3; 8 lists of 50, 13%:
+// 1.60 and 1.59 ms; 32 lists of 8, 16, 50, 17 to 20%: 0.69 and 1.36 ms, 1.44 and 3.1,
+// 7.6 and 13.1.
+constexpr uint32_t kFlatSpheres = 128;
+constexpr size_t kGroupMax = 255;  // most records of a class in one group (its counts are bytes)
 enum { FLAT_SPHERE = 3, FLAT_BOX = 4, FLAT_MEDIUM = 5 };
-struct flat_item {
+struct flat_item {  // a primitive
   flat_scan scan;
-  flat_win win[6];  // one, or a box's faces
-  uint32_t cls;     // 0..2 rect by axis, FLAT_SPHERE, FLAT_BOX, FLAT_MEDIUM
+  flat_win win;
+  uint32_t cls;  // 0..2 rect by axis, FLAT_SPHERE, FLAT_MEDIUM
+};
+struct flat_rec {  // a record: an item, or the box of six
+  flat_scan scan;
+  uint32_t cls, at;
+  int face[6];
 };
 
 bool closed_box(const flat_item *r, float lo[3], float hi[3], int face[6]);
@@ -487,8 +510,8 @@ bool medium_box(const tpt_flat_scene &f, const float *w, flat_item *it) {
     if (e.b != TPT_SLOT_RECT) return false;
     r[i] = flat_item{};
     r[i].cls = (e.a >> 28) & 3u;
-    for (int k = 0; k < 5; ++k) r[i].win[0].f[k] = e.f[k];
-    r[i].win[0].xform = e.xform;
+    for (int k = 0; k < 5; ++k) r[i].win.f[k] = e.f[k];
+    r[i].win.xform = e.xform;
   }
   float lo[3], hi[3];
   int face[6];
@@ -497,7 +520,7 @@ bool medium_box(const tpt_flat_scene &f, const float *w, flat_item *it) {
   it->scan.k = lo[0], it->scan.c0 = lo[1], it->scan.c1 = lo[2];
   it->scan.h0 = hi[0], it->scan.h1 = hi[1], it->scan.x = hi[2];
   it->scan.density = w[2];
-  it->win[0].xform = r[0].win[0].xform;
+  it->win.xform = r[0].win.xform;
   return true;
 }
 
@@ -512,7 +535,7 @@ bool closed_box(const flat_item *r, float lo[3], float hi[3], int face[6]) {
         at[n++] = i;
       }
     if (n != 2) return false;
-    const float k0 = r[at[0]].win[0].f[0], k1 = r[at[1]].win[0].f[0];
+    const float k0 = r[at[0]].win.f[0], k1 = r[at[1]].win.f[0];
     if (!(k0 != k1)) return false;
     const int l = k0 < k1 ? 0 : 1;
     lo[a] = std::fmin(k0, k1), hi[a] = std::fmax(k0, k1);
@@ -520,9 +543,9 @@ bool closed_box(const flat_item *r, float lo[3], float hi[3], int face[6]) {
   }
   for (int i = 0; i < 6; ++i) {
     const uint32_t a = r[i].cls, u = a == 0 ? 1 : 0, v = a == 2 ? 1 : 2;  // in-plane axes
-    const float *f = r[i].win[0].f;
+    const float *f = r[i].win.f;
     if (f[1] != lo[u] || f[2] != hi[u] || f[3] != lo[v] || f[4] != hi[v]) return false;
-    if (r[i].win[0].xform != r[0].win[0].xform || r[i].win[0].slot != r[0].win[0].slot) return false;
+    if (r[i].win.xform != r[0].win.xform || r[i].win.slot != r[0].win.slot) return false;
   }
   return true;
 }
@@ -532,10 +555,17 @@ flat_range flat_records(const tpt_flat_scene &f, uint32_t sb, uint32_t eb, uint3
   std::vector<flat_item> items;
   float mag = 0.0f;
   bool ok = true;
+  uint32_t root = kNone, n_spheres = 0;
+  float expected = 0.0f;  // spheres that a ray through the scene tests in a walk: by their boxes' areas
+  const auto area = [&](uint32_t slot) {
+    const float *b = f.slots[slot].f;
+    const float x = b[3] - b[0], y = b[4] - b[1], z = b[5] - b[2];
+    return x * y + y * z + z * x;
+  };
   auto add = [&](const float *w, uint32_t kind, uint32_t word, uint32_t xform, uint32_t slot, uint32_t entry,
                  uint32_t leaf, uint32_t parent) {
     flat_item it{};
-    flat_win &q = it.win[0];
+    flat_win &q = it.win;
     const int nf = kind == TPT_SLOT_RECT ? 5 : (kind == TPT_SLOT_SPHERE ? 4 : 0);  // (a medium's hold indexes)
     for (int k = 0; k < nf; ++k) q.f[k] = w[k], ok = ok && std::fabs(w[k]) < 1e18f;
     flat_scan &p = it.scan;
@@ -555,6 +585,8 @@ flat_range flat_records(const tpt_flat_scene &f, uint32_t sb, uint32_t eb, uint3
       }
     } else if (kind == TPT_SLOT_SPHERE) {
       it.cls = FLAT_SPHERE;
+      ++n_spheres;
+      expected += parent == kNone ? 1.0f : area(parent) / area(root);
       p.c0 = w[1], p.c1 = w[2], p.h0 = w[3];
       for (int k = 0; k < 3; ++k) mag = std::fmax(mag, std::fabs(w[k]) + std::fabs(w[3]));
     } else if (kind == TPT_SLOT_MEDIUM && xform == 0xFFFFFFFFu && medium_box(f, w, &it)) {
@@ -575,6 +607,7 @@ flat_range flat_records(const tpt_flat_scene &f, uint32_t sb, uint32_t eb, uint3
   };
   for (uint32_t g = 0; g < f.n_segments; ++g) {
     std::vector<uint32_t> open;  // boxes around slot i
+    root = f.segments[2 * g];
     for (uint32_t i = f.segments[2 * g]; i < f.segments[2 * g + 1]; ++i) {
       const tpt_slot &s = f.slots[i];
       while (!open.empty() && f.slots[open.back()].a <= i) open.pop_back();
@@ -604,58 +637,72 @@ flat_range flat_records(const tpt_flat_scene &f, uint32_t sb, uint32_t eb, uint3
     reach = std::fmax(reach, 1.5f * off);
   }
   flat_range r;
-  if (!ok || items.empty() || items.size() > kFlatMax) return r;
-  // the last rect in the order of slots and entries
-  uint32_t nan_slot = kNone, nan_entry = kNone;
-  for (const flat_item &it : items)
-    if (it.win[0].kind == TPT_SLOT_RECT) nan_slot = it.win[0].slot, nan_entry = it.win[0].entry;
-  std::vector<flat_item> merged;
-  for (size_t i = 0; i < items.size();) {
-    float lo[3], hi[3];
-    int face[6];
-    if (i + 6 <= items.size() && items[i].win[0].entry != kNone && closed_box(&items[i], lo, hi, face)) {
-      flat_item b{};
-      b.cls = FLAT_BOX;
-      b.scan.k = lo[0], b.scan.c0 = lo[1], b.scan.c1 = lo[2];
-      b.scan.h0 = hi[0], b.scan.h1 = hi[1], b.scan.x = hi[2];
-      for (int k = 0; k < 6; ++k) b.win[k] = items[i + face[k]].win[0];
-      merged.push_back(b);
-      i += 6;
-    } else {
-      merged.push_back(items[i++]);
-    }
-  }
+  if (!ok || items.empty() || items.size() >= (1u << 24)) return r;  // (segment_combine's entry numbers)
   r.scan0 = static_cast<uint32_t>(scans->size());
   r.win0 = static_cast<uint32_t>(wins->size());
   r.group0 = static_cast<uint32_t>(groups->size());
   r.mag = mag + reach;
-  std::vector<uint32_t> chains;
-  for (const flat_item &it : merged)
-    if (std::find(chains.begin(), chains.end(), it.win[0].xform) == chains.end()) chains.push_back(it.win[0].xform);
-  for (uint32_t xf : chains) {
+  // records by wrapper chain, in the order of the chains' first primitives, and class
+  struct chain {
+    uint32_t xform;
+    std::vector<flat_rec> of[FLAT_MEDIUM + 1];
+  };
+  std::vector<chain> chains;
+  std::vector<uint32_t> index(f.n_xforms + 1, kNone);  // of a transform's chain (last: no wrapper)
+  uint32_t last_rect = kNone;
+  for (size_t i = 0; i < items.size();) {
+    const flat_item &it = items[i];
+    flat_rec b{it.scan, it.cls, static_cast<uint32_t>(i), {0, 0, 0, 0, 0, 0}};
+    float lo[3], hi[3];
+    int face[6];
+    if (i + 6 <= items.size() && it.win.entry != kNone && closed_box(&items[i], lo, hi, face)) {
+      b.cls = FLAT_BOX;
+      std::memcpy(b.face, face, sizeof(face));
+      b.scan.k = lo[0], b.scan.c0 = lo[1], b.scan.c1 = lo[2];
+      b.scan.h0 = hi[0], b.scan.h1 = hi[1], b.scan.x = hi[2];
+    }
+    uint32_t &c = index[it.win.xform == kNone ? f.n_xforms : it.win.xform - xb];
+    if (c == kNone) {
+      c = static_cast<uint32_t>(chains.size());
+      chains.push_back(chain{it.win.xform, {}});
+    }
+    chains[c].of[b.cls].push_back(b);
+    const size_t step = b.cls == FLAT_BOX ? 6 : 1;
+    if (it.win.kind == TPT_SLOT_RECT) last_rect = static_cast<uint32_t>(i + step - 1);
+    i += step;
+  }
+  for (chain &ch : chains) {
     flat_group fg{};
-    if (xf != kNone) {
-      const tpt_xform &x = f.xforms[xf - xb];
+    if (ch.xform != kNone) {
+      const tpt_xform &x = f.xforms[ch.xform - xb];
       fg.nops = x.nops, fg.kinds = x.kinds;
       std::memcpy(fg.p, x.p, sizeof(fg.p));
     }
-    for (uint32_t c = 0; c <= FLAT_MEDIUM; ++c)
-      for (flat_item &it : merged)
-        if (it.win[0].xform == xf && it.cls == c) {
-          it.scan.win = static_cast<uint32_t>(wins->size()) - r.win0;
-          scans->push_back(it.scan);
-          wins->insert(wins->end(), it.win, it.win + (c == FLAT_BOX ? 6 : 1));
+    size_t longest = 0;
+    for (const auto &v : ch.of) longest = std::max(longest, v.size());
+    for (size_t first = 0; first < longest; first += kGroupMax) {
+      fg.n = fg.n_box = 0;
+      for (uint32_t c = 0; c <= FLAT_MEDIUM; ++c)
+        for (size_t i = first; i < std::min(ch.of[c].size(), first + kGroupMax); ++i) {
+          flat_rec &b = ch.of[c][i];
+          b.scan.win = static_cast<uint32_t>(wins->size()) - r.win0;
+          scans->push_back(b.scan);
+          for (int k = 0; k < (c == FLAT_BOX ? 6 : 1); ++k) {
+            const uint32_t at = b.at + static_cast<uint32_t>(b.face[k]);
+            if (at == last_rect) r.nan_win = static_cast<uint32_t>(wins->size()) - r.win0;
+            wins->push_back(items[at].win);
+          }
           if (c >= FLAT_BOX)
             fg.n_box += c == FLAT_BOX ? 1u : 0x10000u;
           else
             fg.n += 1u << (8 * c);
         }
-    groups->push_back(fg);
+      groups->push_back(fg);
+    }
   }
-  r.n_groups = static_cast<uint32_t>(chains.size());
-  r.n_scans = static_cast<uint32_t>(merged.size());
-  for (uint32_t w = r.win0; nan_slot != kNone && w < wins->size(); ++w)
-    if ((*wins)[w].slot == nan_slot && (*wins)[w].entry == nan_entry) r.nan_win = w - r.win0;
+  r.n_groups = static_cast<uint32_t>(groups->size()) - r.group0;
+  r.n_scans = static_cast<uint32_t>(scans->size()) - r.scan0;
+  r.walk = n_spheres > kFlatSpheres && expected * 8.0f < static_cast<float>(n_spheres);
   return r;
 }
 
@@ -779,7 +826,7 @@ int create_pool(const tpt_flat_scene *scenes, uint32_t n, tpt_scene **out) {
     media[k] = 0;
     for (uint32_t i = 0; i < f.n_slots; ++i) media[k] |= (f.slots[i].b >> 28) == TPT_SLOT_MEDIUM;
     for (uint32_t e = 0; e < f.n_entries; ++e) media[k] |= f.entries[e].b == TPT_SLOT_MEDIUM;
-    // The uniform pass tests every primitive, so it is for small scenes.  (It
+    // The uniform pass tests every primitive, so it is for scenes of few slots.  (It
     // is built without the ray-time replay, wrapped segments, and media not
     // bounded by a closed box: flat_records has none then.)
     bool wrapped = false;
@@ -1381,8 +1428,10 @@ int render_core(tpt_scene *s, const tpt_job *jobs, uint32_t n_jobs, const tpt_la
   B.P.scenes = s->d_scenes;
   B.P.guide_verts = ~0u;
   B.P.media_scatter = (L.flags & TPT_RENDER_MEDIA_SCATTER) ? 1u : 0u;
-  if (!guide && !B.count && !(L.flags & TPT_RENDER_NO_TAIL))
+  if (!guide && !B.count && !(L.flags & TPT_RENDER_NO_TAIL)) {
+    B.sweep = B.sweep && !s->flat_of[jobs[0].scene].walk;
     return render_paths(s, jd, plan_passes(jobs, n_jobs, kPassItemsPaths), B, profile, stats, cs);
+  }
   const std::vector<pass_plan> plan =
       plan_passes(jobs, n_jobs, guide && L.guiding ? kPassItemsRecording : kPassItems);
   uint32_t max_items = 0, max_ent = 0;

@@ -1,10 +1,10 @@
 // Closest hit of small scenes: one uniform pass over every primitive instead
 // of a tree walk, with the exact reference arithmetic kept for the winner.
 //
-// What bounds it: VALU issue.  The sweep of segment_sweep evaluates each slab
-// and each rect exactly where a lane's own walk visits it: an IEEE division
-// and two axis selects per rect, and a wave pays for the union of its lanes'
-// visits with about a third of them idle.  Here every lane tests every
+// What bounds it: VALU issue.  The sweep before it, where the wave went through
+// the slots together, evaluated each slab and each rect exactly where a lane's own
+// walk visits it: an IEEE division and two axis selects per rect, and a wave paid
+// for the union of its lanes' visits with about a third of them idle.  Here every lane tests every
 // primitive by approximations with error bounds (one reciprocal per ray and
 // axis, two fused multiply-adds per rect), nothing diverges, and records come
 // through the scalar cache.  Only the nearest candidate is then evaluated
@@ -15,8 +15,8 @@
 // Measured, sweep -> this pass: Cornell 1200x1200 128 spp 41.4 -> 25.8 ms, the
 // reference's box 160x120 4 spp 0.67 -> 0.31 ms, 4.2M rays with records 182 ->
 // 143 us, a guided 600x600 pass 3.82 -> 3.27 ms.  A rect costs 18 instructions,
-// a box of six 44.  Scenes of more than 64 slots or 64 primitives keep their
-// tree walks, which a ray leaves after a few boxes.
+// a box of six 44.  Scenes of more than 64 slots keep their tree walks, which a
+// ray leaves after a few boxes.
 //
 // Lanes where the approximations cannot decide take the exact walk instead
 // (*slow): a candidate within its error of an edge, of t_min or t_max, or of a
@@ -146,10 +146,12 @@ __device__ __forceinline__ void flat_box(flat_scan_ptr p, v3 o, v3 inv, float et
 
 // Touches every cache line of the scene's records at once, for a kernel that
 // traces one ray per thread: the loads that follow one another in the pass then
-// hit the scalar cache (a 1009-ray call: 15.1 -> 9.3 us).
+// hit the scalar cache (a 1009-ray call: 15.1 -> 9.3 us).  At most kFlatTouch
+// records, half of that cache's 16 KB.
+constexpr uint32_t kFlatTouch = 256;
 __device__ __forceinline__ void flat_touch(const scene_view &S) {
   typedef const TPT_SCALAR uint32_t *word_ptr;
-  const uint32_t ng = S.n_fgroups * (sizeof(flat_group) / 64), ns = (S.n_flat * sizeof(flat_scan) + 63) / 64;
+  const uint32_t ng = S.n_fgroups * (sizeof(flat_group) / 64), ns = (min(S.n_flat, kFlatTouch) * sizeof(flat_scan) + 63) / 64;
   uint32_t x = 0;
   for (uint32_t i = 0; i < ng; ++i) x |= ((word_ptr)(S.fgroups))[16 * i];
 #pragma unroll 4
