@@ -70,6 +70,9 @@ k_paths(scene_view S, const tpt_slot *__restrict__ slots, const tpt_entry *__res
   // the wave's generated camera rays that no lane has taken yet: o, d, pixel, sample, entry
   __shared__ float pool[PATH_WAVES][9][64];
   __shared__ uint32_t bstack[SPH ? kBvhDepth * PATH_THREADS : 1];  // sphere_world's
+  __shared__ unsigned long long carried;
+  if (threadIdx.x == 0) carried = 0;
+  __syncthreads();
   const uint32_t wave = threadIdx.x / 64, lane = __lane_id();
   float(*mine)[64] = pool[wave];
   uint32_t pool_at = 0, pool_n = 0;  // wave-uniform
@@ -78,7 +81,7 @@ k_paths(scene_view S, const tpt_slot *__restrict__ slots, const tpt_entry *__res
   uint32_t st[ST_COUNT] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
   bool live = false;
   path p{};
-  uint32_t px = 0, smp = 0;
+  uint32_t px = 0, smp = 0, turn = 0;
   for (;;) {
     unsigned long long dead = __ballot(!live);
     while (dead != 0ull && (pool_n != 0u || more)) {
@@ -138,6 +141,7 @@ k_paths(scene_view S, const tpt_slot *__restrict__ slots, const tpt_entry *__res
                                                &st[ST_NODES]);
     else
       got = trace_world<false, MEDIA>(Sj, p.o, p.d, rc, 0.001f, kFltMax, &h, &st[ST_NODES], live);
+    carry_visits(&carried, st, ++turn);
     if (live) {
       ++st[ST_SEGMENTS];
       uint32_t cls = Q_TERMINAL;
@@ -157,7 +161,7 @@ k_paths(scene_view S, const tpt_slot *__restrict__ slots, const tpt_entry *__res
     }
   }
   st[ST_TAIL] = st[ST_SEGMENTS];
-  block_stats(Q.stats, st, ST_BASIC);
+  block_stats<true>(Q.stats, st, ST_BASIC, &carried);
 }
 
 }  // namespace tptd

@@ -28,6 +28,8 @@
 #ifndef TPT_CSRC_RENDER_H
 #define TPT_CSRC_RENDER_H
 
+#include <type_traits>
+
 #include "guide.h"
 #include "shade.h"
 #include "walk_bvh.h"
@@ -263,16 +265,33 @@ __device__ __forceinline__ uint32_t claim_item(const pass_hdr &H, uint32_t *coun
   return item;
 }
 
+// Where a lane carries many paths (k_paths, k_tail), its 32-bit count of visits
+// could wrap: half way there it moves to the block's 64-bit one (in LDS, zeroed by
+// the kernel; block_stats adds it).  Looked at every kCarryTurns segments, in which
+// a lane makes less than 2^31 visits (2^25 each; a comparison in every segment cost
+// 10 us of a 160 x 120 preview's 294).
+constexpr uint32_t kCarryTurns = 64;
+__device__ __forceinline__ void carry_visits(unsigned long long *carried, uint32_t *st, uint32_t turn) {
+  if (turn % kCarryTurns != 0u || __ballot(st[ST_NODES] >> 31) == 0ull) return;
+  atomicAdd(carried, static_cast<unsigned long long>(st[ST_NODES]));
+  st[ST_NODES] = 0;
+}
+
 // Adds per-thread counts into this block's stats row (no global atomics).
-__device__ __forceinline__ void block_stats(unsigned long long *stats, const uint32_t *v, int n) {
+// carried: see carry_visits; with it a wave's sums may exceed 32 bits (those of
+// one bounce do not, and 64-bit sums in every launch cost a guided frame 1%).
+template <bool CARRIED = false>
+__device__ __forceinline__ void block_stats(unsigned long long *stats, const uint32_t *v, int n,
+                                            const unsigned long long *carried = nullptr) {
   __shared__ unsigned long long acc[ST_COUNT];
   if (threadIdx.x < ST_COUNT) acc[threadIdx.x] = 0;
   __syncthreads();
   for (int k = 0; k < n; ++k) {
-    uint32_t x = v[k];
+    std::conditional_t<CARRIED, unsigned long long, uint32_t> x = v[k];
     for (int off = 32; off > 0; off >>= 1) x += __shfl_xor(x, off);
     if (__lane_id() == 0 && x) atomicAdd(&acc[k], static_cast<unsigned long long>(x));
   }
+  if (CARRIED && threadIdx.x == 0) atomicAdd(&acc[ST_NODES], *carried);  // (complete since the first barrier)
   __syncthreads();
   if (threadIdx.x < static_cast<uint32_t>(n)) stats[blockIdx.x * ST_COUNT + threadIdx.x] += acc[threadIdx.x];
 }
@@ -1037,6 +1056,8 @@ __global__ void __launch_bounds__(256) k_tail(scene_view S, const tpt_slot *__re
   __shared__ uint32_t offs[NSUB];
   __shared__ uint32_t pre[NSUB + 1];
   __shared__ uint32_t bstack[SPH ? kBvhDepth * 256 : 1];  // sphere_world's
+  __shared__ unsigned long long carried;
+  if (threadIdx.x == 0) carried = 0;
   if (threadIdx.x < NSUB) offs[threadIdx.x] = rc_at(parity, threadIdx.x);
   __syncthreads();
   region_prefix(Q.counters, offs, NSUB, pre);
@@ -1051,6 +1072,7 @@ __global__ void __launch_bounds__(256) k_tail(scene_view S, const tpt_slot *__re
   uint32_t chunk = blockIdx.x * blockDim.x + __builtin_amdgcn_readfirstlane(threadIdx.x / 64) * 64, used = 0;
   bool live = false;
   path p{};
+  uint32_t turn = 0;
   for (;;) {
     unsigned long long dead = __ballot(!live);
     while (dead != 0ull && chunk < count) {
@@ -1077,6 +1099,7 @@ __global__ void __launch_bounds__(256) k_tail(scene_view S, const tpt_slot *__re
       const bool got = SWEEP ? small_world(Sj, p.o, p.d, rc, 0.001f, kFltMax, &h, &st[ST_NODES], live)
                              : sphere_world<!MULTI, 256>(Sj, p.o, p.d, rc, 0.001f, kFltMax, live, bstack + threadIdx.x,
                                                          &h, &st[ST_NODES]);
+      carry_visits(&carried, st, ++turn);
       uint32_t cls = Q_TERMINAL;
       if (live) {
         ++st[ST_SEGMENTS];
@@ -1106,7 +1129,7 @@ __global__ void __launch_bounds__(256) k_tail(scene_view S, const tpt_slot *__re
       }
     }
   }
-  block_stats(Q.stats, st, ST_BASIC);
+  block_stats<true>(Q.stats, st, ST_BASIC, &carried);
 }
 
 // Each job's sum/sumsq += its samples of the pass, in sample order per pixel.
