@@ -92,10 +92,9 @@ struct bvh_builder {
     }
     return mid;
   }
-  // (compared as floats: a conversion to int is only defined in its range)
+  // (limited as a float: a conversion to int is only defined in its range)
   static int bin(float c, float lo, float scale) {
-    const float q = (c - lo) * scale;
-    return q < kBins - 1 ? (q > 0.0f ? static_cast<int>(q) : 0) : kBins - 1;
+    return static_cast<int>(upper(lower((c - lo) * scale, kBins - 1), 0.0f));
   }
 
   // Builds [first, first + count) with at most `levels` levels of nodes;

@@ -16,26 +16,35 @@ namespace tptd {
 // Flattened hitables are always so; a caller's own arrays need not be, and are
 // walked box by box then.
 inline bool regular_trees(const tpt_flat_scene &f) {
-  std::vector<uint32_t> end(f.n_slots);  // of slot i's subtree
+  struct node {
+    const tpt_slot *s;
+    uint32_t kids;
+  };
+  std::vector<node> open;  // boxes around slot i
+  open.reserve(64);
   for (uint32_t g = 0; g < f.n_segments; ++g) {
     const uint32_t a = f.segments[2 * g], b = f.segments[2 * g + 1];
-    for (uint32_t i = b; i-- > a;) {
-      const tpt_slot &s = f.slots[i];
-      end[i] = i + 1;
-      if ((s.b >> 28) != TPT_SLOT_BOX) continue;
-      const uint32_t right = s.b & TPT_PAYLOAD_MASK;
-      const uint32_t child[2] = {i + 1, right == TPT_NO_RIGHT ? i + 1 : right};
-      for (const uint32_t c : child) {
-        if (c >= b) return false;
-        if ((f.slots[c].b >> 28) != TPT_SLOT_BOX) continue;
-        for (int k = 0; k < 3; ++k)
-          if (!(s.f[k] <= f.slots[c].f[k] && f.slots[c].f[3 + k] <= s.f[3 + k])) return false;
+    open.clear();
+    for (uint32_t i = a; i <= b; ++i) {
+      while (!open.empty() && open.back().s->a == i) {
+        if (open.back().kids != ((open.back().s->b & TPT_PAYLOAD_MASK) == TPT_NO_RIGHT ? 1u : 2u)) return false;
+        open.pop_back();
       }
-      if (right != TPT_NO_RIGHT && end[i + 1] != right) return false;
-      end[i] = end[child[1]];
-      if (end[i] != s.a) return false;
+      if (i == b) break;
+      const tpt_slot &s = f.slots[i];
+      const bool box = (s.b >> 28) == TPT_SLOT_BOX;
+      if (!open.empty()) {
+        node &p = open.back();
+        if (++p.kids > 1 && (p.kids > 2 || (p.s->b & TPT_PAYLOAD_MASK) != i)) return false;
+        for (int k = 0; box && k < 3; ++k)
+          if (!(p.s->f[k] <= s.f[k] && s.f[3 + k] <= p.s->f[3 + k])) return false;
+        if (box && s.a > p.s->a) return false;
+      } else if (i != a) {
+        return false;
+      }
+      if (box) open.push_back(node{&s, 0});
     }
-    if (a < b && end[a] != b) return false;
+    if (!open.empty()) return false;
   }
   return true;
 }
