@@ -43,7 +43,7 @@ struct tree {
   }
 };
 
-bool check(const char *name, const std::vector<tpt_slot> &slots) {
+bool check(const char *name, const std::vector<tpt_slot> &slots, bool ready = true) {
   const uint32_t seg[2] = {0, static_cast<uint32_t>(slots.size())};
   tpt_flat_scene f;
   std::memset(&f, 0, sizeof(f));
@@ -56,7 +56,7 @@ bool check(const char *name, const std::vector<tpt_slot> &slots) {
   if (v.ready && v.root != kBvhNone) t.visit(v.root, 0, lo, hi);
   uint32_t missing = 0;
   for (size_t i = 0; v.ready && i < t.seen.size(); ++i) missing += t.seen[i] != (i < v.n_big ? 0 : 1);
-  const bool ok = t.ok && missing == 0 && t.deepest <= kBvhDepth;
+  const bool ok = t.ok && missing == 0 && t.deepest <= kBvhDepth && (v.ready != 0) == ready && v.n_big <= kMostBig;
   std::printf("%-28s %6zu spheres, ready %u, %2u levels: %s\n", name, slots.size(), v.ready, t.deepest, ok ? "ok" : "BAD");
   return ok;
 }
@@ -135,6 +135,14 @@ int main() {
   for (int i = 0; i < 20; ++i) s[i].f[0] = (i & 1) ? 1e-39f : 0.0f, s[i].f[1] = s[i].f[2] = 0.0f;
   ok = check("a cluster a denormal wide", s) && ok;
   s[3].f[1] = NAN;
-  ok = check("a NaN centre", s) && ok;
+  ok = check("a NaN centre", s, false) && ok;
+  // radii: however large, only a few much larger than the rest stay outside
+  for (float r : {2.0f, 2.5f, 300.0f}) {
+    std::snprintf(name, sizeof(name), "radius %g", r);
+    s = spheres(500, 1000.0f, 3, r);
+    ok = check(name, s) && ok;
+    for (int i = 0; i < 20; ++i) s[25 * i].f[3] = r * (3.0f + i);
+    ok = check(name, s) && ok;
+  }
   return ok ? 0 : 1;
 }

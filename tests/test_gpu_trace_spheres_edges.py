@@ -13,10 +13,23 @@ def spheres(kind, rng):
     if kind == "a denormal apart":  # no finite bin scale, whole or in part
         c[:100] = c[0]
         c[:100, 0] = 1e-39 * rng.integers(0, 9, 100)
+    if kind == "all big":  # no sphere set aside: radii 2.5 to 9.9
+        r = rng.uniform(2.5, 9.9, 300)
+        c *= 4
+    if kind == "big ones among big":  # 16 above 4 times the 17th, one as large as that
+        r = rng.uniform(2.5, 4.0, 300)
+        r[100], r[:16] = 16.0, np.linspace(64.5, 300.0, 16)
+        r[8:16] *= -1
+        r[101:] = np.minimum(r[101:], 3.9)
+        c *= 10
+    if kind == "one among big":
+        r[:] = 2.5
+        r[7] = 1000.0
+        c *= 4
     return np.concatenate([c, r[:, None]], 1).astype(np.float32)
 
 
-@pytest.mark.parametrize("kind", ["a denormal apart"])
+@pytest.mark.parametrize("kind", ["a denormal apart", "all big", "big ones among big", "one among big"])
 @pytest.mark.parametrize("tree", [True, False])
 def test_edges_equal_general_walk(tpt, device, kind, tree):
     import torch

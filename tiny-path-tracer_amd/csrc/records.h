@@ -44,7 +44,7 @@ struct flat_group {
 // in the reference's tree (infinite: none), its slot, and its rank among equal t.
 constexpr uint32_t kBvhLeaf = 0x80000000u, kBvhNone = 0xFFFFFFFFu;
 constexpr uint32_t kBvhDepth = 24;  // most levels of nodes (2^24 spheres fit a balanced one)
-constexpr float kWalkBigRadius = 2.0f;  // spheres above it are tested by every ray
+constexpr float kWalkBigRadius = 2.0f;  // spheres above it are tested by every ray (but see build_bvh)
 constexpr float kBvhPad = 5.6e-7f;  // 1.25 * 7.5 u
 struct bvh_node {
   float b[3][4];
@@ -58,7 +58,9 @@ struct bvh_scene {
   float lo[3], hi[3];  // bounds of the spheres in the tree
   float pad, mag;      // kBvhPad over their smallest radius; the largest coordinate magnitude
   uint32_t root, big0, n_big;  // big spheres: leaves [big0, big0 + n_big)
-  uint32_t multi, ready, unused[3];  // more than one segment; a tree was built
+  uint32_t multi, ready;       // more than one segment; a tree was built
+  float radius;                // none in the tree has a larger one
+  uint32_t unused[2];
 };
 
 }  // namespace tptd

@@ -33,9 +33,9 @@
 // takes D to the farthest corner of the spheres' bounds.  kBvhPad and
 // kBvhPadD are these constants times 1.25; 8u (|o| + M) more covers the fused
 // slab arithmetic.  Along the ray, a computed root lies within 8e-4 (|t| +
-// r/|d|) of the padded chord; the slack of sphere_walk_bound (19 times that, for
-// radii up to kWalkBigRadius) is applied at both ends.  Bigger spheres are not
-// in the tree: every ray tests them.
+// r/|d|) of the padded chord; a slack of 2^-6 (|t| + R/|d|), 19 times that for
+// radii up to R, the largest in the tree, is applied at both ends.  Bigger spheres
+// are tested by every ray.
 //
 // Rays with a direction component that is 0, tiny or huge, a NaN, or bounds
 // that are not numbers take the walk of traverse.h.
@@ -97,7 +97,7 @@ __device__ __forceinline__ bool bvh_world(const scene_view &S, const bvh_scene &
   const float pad = fminf(V.pad * d2, kBvhPadD * __builtin_amdgcn_sqrtf(d2)) + (mo + V.mag) * 0x1p-21f;
   const v3 al{(o.x + pad) * inv.x, (o.y + pad) * inv.y, (o.z + pad) * inv.z};
   const v3 ah{(o.x - pad) * inv.x, (o.y - pad) * inv.y, (o.z - pad) * inv.z};
-  const float reach = 0x1p-6f * kWalkBigRadius * __builtin_amdgcn_rsqf(d.x * d.x + d.y * d.y + d.z * d.z) +
+  const float reach = 0x1p-6f * V.radius * __builtin_amdgcn_rsqf(d.x * d.x + d.y * d.y + d.z * d.z) +
                       S.walk_ulp * mi;
   const float t0 = tmin - fabsf(tmin) * 0x1p-6f - reach;
   bvh_best best{INFINITY, tmax + fabsf(tmax) * 0x1p-6f + reach, kNone, 0u};
@@ -169,7 +169,7 @@ __device__ __forceinline__ bool sphere_world(const scene_view &S, v3 o, v3 d, co
     typedef const TPT_SCALAR bvh_scene *bvh_scene_ptr;
     bvh_scene_ptr p = (bvh_scene_ptr)(S.bvh);
     for (int k = 0; k < 3; ++k) V.lo[k] = p->lo[k], V.hi[k] = p->hi[k];
-    V.pad = p->pad, V.mag = p->mag;
+    V.pad = p->pad, V.mag = p->mag, V.radius = p->radius;
     V.root = p->root, V.big0 = p->big0, V.n_big = p->n_big, V.multi = p->multi, V.ready = p->ready;
   } else {
     V = *S.bvh;
