@@ -70,8 +70,8 @@ k_paths(scene_view S, const tpt_slot *__restrict__ slots, const tpt_entry *__res
   // the wave's generated camera rays that no lane has taken yet: o, d, pixel, sample, entry
   __shared__ float pool[PATH_WAVES][9][64];
   __shared__ uint32_t bstack[SPH ? kBvhDepth * PATH_THREADS : 1];  // sphere_world's
-  __shared__ unsigned long long carried;
-  if (threadIdx.x == 0) carried = 0;
+  __shared__ unsigned long long acc[ST_BASIC];  // path_stats's
+  if (threadIdx.x < ST_BASIC) acc[threadIdx.x] = 0;
   __syncthreads();
   const uint32_t wave = threadIdx.x / 64, lane = __lane_id();
   float(*mine)[64] = pool[wave];
@@ -81,7 +81,8 @@ k_paths(scene_view S, const tpt_slot *__restrict__ slots, const tpt_entry *__res
   uint32_t st[ST_COUNT] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
   bool live = false;
   path p{};
-  uint32_t px = 0, smp = 0, turn = 0;
+  uint32_t px = 0, smp = 0;
+  unsigned long long visits = 0;
   for (;;) {
     unsigned long long dead = __ballot(!live);
     while (dead != 0ull && (pool_n != 0u || more)) {
@@ -132,16 +133,17 @@ k_paths(scene_view S, const tpt_slot *__restrict__ slots, const tpt_entry *__res
     const ray_ctx rc = (MEDIA || (!SIMPLE && !SWEEP && !SPH)) && (P.motion | P.media) && live ? make_ray_ctx(P, c, p.depth)
                                                                                  : ray_ctx{0.0f, 0u, 0u, 0u, 0u, 0u};
     bool got;
+    uint32_t nodes = 0;
     hit_geo geo{};
     if (SWEEP)
-      got = small_world<false, MEDIA>(Sj, p.o, p.d, rc, 0.001f, kFltMax, &h, &st[ST_NODES], live, nullptr,
+      got = small_world<false, MEDIA>(Sj, p.o, p.d, rc, 0.001f, kFltMax, &h, &nodes, live, nullptr,
                                       kGeo ? &geo : nullptr);
     else if (SPH)
       got = sphere_world<!MULTI, PATH_THREADS>(Sj, p.o, p.d, rc, 0.001f, kFltMax, live, bstack + threadIdx.x, &h,
-                                               &st[ST_NODES]);
+                                               &nodes);
     else
-      got = trace_world<false, MEDIA>(Sj, p.o, p.d, rc, 0.001f, kFltMax, &h, &st[ST_NODES], live);
-    carry_visits(&carried, st, ++turn);
+      got = trace_world<false, MEDIA>(Sj, p.o, p.d, rc, 0.001f, kFltMax, &h, &nodes, live);
+    if (!SWEEP) visits += nodes;
     if (live) {
       ++st[ST_SEGMENTS];
       uint32_t cls = Q_TERMINAL;
@@ -160,8 +162,7 @@ k_paths(scene_view S, const tpt_slot *__restrict__ slots, const tpt_entry *__res
       }
     }
   }
-  st[ST_TAIL] = st[ST_SEGMENTS];
-  block_stats<true>(Q.stats, st, ST_BASIC, &carried);
+  path_stats(Q.stats, acc, st, visits, SWEEP ? S.n_flat : 0u);
 }
 
 }  // namespace tptd

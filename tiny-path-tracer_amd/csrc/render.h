@@ -28,8 +28,6 @@
 #ifndef TPT_CSRC_RENDER_H
 #define TPT_CSRC_RENDER_H
 
-#include <type_traits>
-
 #include "guide.h"
 #include "shade.h"
 #include "walk_bvh.h"
@@ -265,35 +263,51 @@ __device__ __forceinline__ uint32_t claim_item(const pass_hdr &H, uint32_t *coun
   return item;
 }
 
-// Where a lane carries many paths (k_paths, k_tail), its 32-bit count of visits
-// could wrap: half way there it moves to the block's 64-bit one (in LDS, zeroed by
-// the kernel; block_stats adds it).  Looked at every kCarryTurns segments, in which
-// a lane makes less than 2^31 visits (2^25 each; a comparison in every segment cost
-// 10 us of a 160 x 120 preview's 294).
-constexpr uint32_t kCarryTurns = 64;
-__device__ __forceinline__ void carry_visits(unsigned long long *carried, uint32_t *st, uint32_t turn) {
-  if (turn % kCarryTurns != 0u || __ballot(st[ST_NODES] >> 31) == 0ull) return;
-  atomicAdd(carried, static_cast<unsigned long long>(st[ST_NODES]));
-  st[ST_NODES] = 0;
-}
-
 // Adds per-thread counts into this block's stats row (no global atomics).
-// carried: see carry_visits; with it a wave's sums may exceed 32 bits (those of
-// one bounce do not, and 64-bit sums in every launch cost a guided frame 1%).
-template <bool CARRIED = false>
-__device__ __forceinline__ void block_stats(unsigned long long *stats, const uint32_t *v, int n,
-                                            const unsigned long long *carried = nullptr) {
+__device__ __forceinline__ void block_stats(unsigned long long *stats, const uint32_t *v, int n) {
   __shared__ unsigned long long acc[ST_COUNT];
   if (threadIdx.x < ST_COUNT) acc[threadIdx.x] = 0;
   __syncthreads();
   for (int k = 0; k < n; ++k) {
-    std::conditional_t<CARRIED, unsigned long long, uint32_t> x = v[k];
+    uint32_t x = v[k];
     for (int off = 32; off > 0; off >>= 1) x += __shfl_xor(x, off);
     if (__lane_id() == 0 && x) atomicAdd(&acc[k], static_cast<unsigned long long>(x));
   }
-  if (CARRIED && threadIdx.x == 0) atomicAdd(&acc[ST_NODES], *carried);  // (complete since the first barrier)
   __syncthreads();
   if (threadIdx.x < static_cast<uint32_t>(n)) stats[blockIdx.x * ST_COUNT + threadIdx.x] += acc[threadIdx.x];
+}
+
+// The same for kernels whose lanes carry many paths (k_paths, k_tail): their visits
+// are counted in 64 bits, and a wave's sums may exceed 32 (those of one bounce do
+// not, and 64-bit sums in each of its launches cost a guided frame 1%).  records:
+// of the uniform pass, which visits each in every segment, or 0: see visits.  acc:
+// ST_BASIC sums in LDS, zeroed by the kernel.  The sums go side by side: one after
+// the other they took 2 us of a preview.
+__device__ __forceinline__ void path_stats(unsigned long long *stats, unsigned long long *acc, const uint32_t *v,
+                                           unsigned long long visits, uint32_t records) {
+  unsigned long long seg = v[ST_SEGMENTS], light = v[ST_LIGHT];
+  uint32_t nan = v[ST_NAN], paths = v[ST_PATHS];
+  for (int off = 32; off > 0; off >>= 1) {
+    seg += __shfl_xor(seg, off);
+    light += __shfl_xor(light, off);
+    if (!records) visits += __shfl_xor(visits, off);
+    nan += __shfl_xor(nan, off);
+    paths += __shfl_xor(paths, off);
+  }
+  if (__lane_id() == 0) {
+    atomicAdd(&acc[ST_SEGMENTS], seg);
+    atomicAdd(&acc[ST_LIGHT], light);
+    if (!records) atomicAdd(&acc[ST_NODES], visits);
+    atomicAdd(&acc[ST_NAN], static_cast<unsigned long long>(nan));
+    atomicAdd(&acc[ST_PATHS], static_cast<unsigned long long>(paths));
+  }
+  __syncthreads();
+  if (threadIdx.x < ST_BASIC) {
+    unsigned long long x = acc[threadIdx.x];
+    if (threadIdx.x == ST_TAIL) x = acc[ST_SEGMENTS];
+    if (records && threadIdx.x == ST_NODES) x = acc[ST_SEGMENTS] * records;
+    stats[blockIdx.x * ST_COUNT + threadIdx.x] += x;
+  }
 }
 
 // Path record, 48 bytes in 3 planes (depth and pass entry share a word: both
@@ -1056,8 +1070,8 @@ __global__ void __launch_bounds__(256) k_tail(scene_view S, const tpt_slot *__re
   __shared__ uint32_t offs[NSUB];
   __shared__ uint32_t pre[NSUB + 1];
   __shared__ uint32_t bstack[SPH ? kBvhDepth * 256 : 1];  // sphere_world's
-  __shared__ unsigned long long carried;
-  if (threadIdx.x == 0) carried = 0;
+  __shared__ unsigned long long acc[ST_BASIC];  // path_stats's
+  if (threadIdx.x < ST_BASIC) acc[threadIdx.x] = 0;
   if (threadIdx.x < NSUB) offs[threadIdx.x] = rc_at(parity, threadIdx.x);
   __syncthreads();
   region_prefix(Q.counters, offs, NSUB, pre);
@@ -1072,7 +1086,7 @@ __global__ void __launch_bounds__(256) k_tail(scene_view S, const tpt_slot *__re
   uint32_t chunk = blockIdx.x * blockDim.x + __builtin_amdgcn_readfirstlane(threadIdx.x / 64) * 64, used = 0;
   bool live = false;
   path p{};
-  uint32_t turn = 0;
+  unsigned long long visits = 0;
   for (;;) {
     unsigned long long dead = __ballot(!live);
     while (dead != 0ull && chunk < count) {
@@ -1096,14 +1110,14 @@ __global__ void __launch_bounds__(256) k_tail(scene_view S, const tpt_slot *__re
       const scene_view Sj = view_of<MULTI>(S, P, c.job);
       hit_t h{0.0f, kNone, kNone, 0};
       const ray_ctx rc{0.0f, 0u, 0u, 0u, 0u, 0u};
-      const bool got = SWEEP ? small_world(Sj, p.o, p.d, rc, 0.001f, kFltMax, &h, &st[ST_NODES], live)
+      uint32_t nodes = 0;
+      const bool got = SWEEP ? small_world(Sj, p.o, p.d, rc, 0.001f, kFltMax, &h, &nodes, live)
                              : sphere_world<!MULTI, 256>(Sj, p.o, p.d, rc, 0.001f, kFltMax, live, bstack + threadIdx.x,
-                                                         &h, &st[ST_NODES]);
-      carry_visits(&carried, st, ++turn);
+                                                         &h, &nodes);
+      if (!SWEEP) visits += nodes;
       uint32_t cls = Q_TERMINAL;
       if (live) {
         ++st[ST_SEGMENTS];
-        ++st[ST_TAIL];
         if (got) {
           h.mat &= TPT_PAYLOAD_MASK;
           const uint32_t kind = S.materials[h.mat].kind;
@@ -1129,7 +1143,7 @@ __global__ void __launch_bounds__(256) k_tail(scene_view S, const tpt_slot *__re
       }
     }
   }
-  block_stats<true>(Q.stats, st, ST_BASIC, &carried);
+  path_stats(Q.stats, acc, st, visits, SWEEP ? S.n_flat : 0u);
 }
 
 // Each job's sum/sumsq += its samples of the pass, in sample order per pixel.
