@@ -62,7 +62,7 @@ k_paths(scene_view S, const tpt_slot *__restrict__ slots, const tpt_entry *__res
         render_state Q) {
   S.slots = slots;
   S.entries = entries;
-  // What the sweep knows of the hit, and the first draws of the shading: not in
+  // What the uniform pass knows of the hit, and the first draws of the shading: not in
   // the media variants, which have no registers left (smoke box 8% slower), and
   // not behind the tree walks (random spheres: 0.6% slower with the draws).
   constexpr bool kGeo = SWEEP && !MEDIA;

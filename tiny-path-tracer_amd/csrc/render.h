@@ -470,22 +470,23 @@ __global__ void __launch_bounds__(256) k_init(render_params P, render_state Q) {
   }
 }
 
-// SWEEP: the uniform pass of small scenes (walk_flat.h).  SPH:
-// every leaf of the scene (or pool) is a sphere; without the rect and list
-// code the kernel fits 64 registers, 8 waves per SIMD.  MEDIA: the scenes hold
-// constant_media (their code costs registers, so only this variant has it).  The slot/entry arrays come
-// in as separate restrict arguments so that wave-uniform loads from them can
-// use the scalar data path.  COUNT: also counts the walk's operations by kind
-// (TPT_RENDER_COUNT_OPS; the other variants are built without that code).
-// The path record is parked in LDS during the walk (see below); the uniform
-// pass then fits 71 VGPRs.
+// SWEEP: the uniform pass of small scenes (walk_flat.h).  SPH: every leaf of the
+// scene (or pool) is a sphere, and rays take the tree of walk_bvh.h.  Its stack and
+// the record stash below hold 37 KB of LDS per block: 4 blocks per CU, 4 waves per
+// SIMD (with the registers held to 64 for 8 waves as well the time is the same).
+// MEDIA: the scenes hold constant_media (their code costs registers, so only this
+// variant has it).  The slot/entry arrays come in as separate restrict arguments so
+// that wave-uniform loads from them can use the scalar data path.  COUNT: also
+// counts the walk's operations by kind (TPT_RENDER_COUNT_OPS; the other variants are
+// built without that code), spheres in the general walk at 8 waves.  The path record
+// is parked in LDS during the walk (see below); the uniform pass then fits 71 VGPRs.
 constexpr uint32_t TRACE_THREADS = 256;  // k_trace's block size (its record stash holds one record per thread)
 template <bool SWEEP, bool MULTI, bool SPH = false, bool MEDIA = false, bool COUNT = false>
-__global__ void __launch_bounds__(TRACE_THREADS) __attribute__((amdgpu_waves_per_eu(SPH ? 8 : (MEDIA ? 1 : (SWEEP ? 6 : 5))))) k_trace(scene_view S, const tpt_slot *__restrict__ slots,
+__global__ void __launch_bounds__(TRACE_THREADS) __attribute__((amdgpu_waves_per_eu(SPH ? (COUNT ? 8 : 4) : (MEDIA ? 1 : (SWEEP ? 6 : 5))))) k_trace(scene_view S, const tpt_slot *__restrict__ slots,
                                                const tpt_entry *__restrict__ entries, render_params P,
                                                render_state Q, uint32_t parity) {
-  static_assert(!(SWEEP && MULTI), "the wave-uniform sweep needs one scene");
-  static_assert(!(SWEEP && SPH), "the sweep takes every leaf kind");
+  static_assert(!(SWEEP && MULTI), "the uniform pass needs one scene");
+  static_assert(!(SWEEP && SPH), "the uniform pass takes every leaf kind");
   static_assert(!(COUNT && SWEEP), "operations are counted in the walks of each lane");
   static_assert(!(MEDIA && SPH), "a sphere-only scene has no media");
   S.slots = slots;
@@ -507,9 +508,8 @@ __global__ void __launch_bounds__(TRACE_THREADS) __attribute__((amdgpu_waves_per
   // The record read before the walk is stored here and read back after it:
   // only the ray stays in registers across the walk.  The compiler barrier
   // before the read-back keeps the compiler from forwarding the stored values
-  // in registers.  Measured: sphere-only walk at 8 waves, 19 instead of 23 spilled VGPRs, batch64 +3%;
-  // the general walk spills 2-11 instead of 6-13 VGPRs (no change in time on
-  // box_list).
+  // in registers.  Measured: the general walk spills 2-11 instead of 6-13 VGPRs (no
+  // change in time on a list of boxes).
   __shared__ float4 stash[3 * TRACE_THREADS];
   __shared__ uint32_t bstack[SPH && !COUNT ? kBvhDepth * TRACE_THREADS : 1];  // sphere_world's
   for (uint32_t base = blockIdx.x * blockDim.x; base < count; base += stride) {
@@ -544,8 +544,8 @@ __global__ void __launch_bounds__(TRACE_THREADS) __attribute__((amdgpu_waves_per
     const uint32_t ent = MULTI ? __float_as_uint(b.w) >> 16 : 0u;
     const uint32_t job = MULTI ? P.pass[ent].job : 0u;
     const scene_view Sj = view_of<MULTI>(S, P, job);
-    // (scenes with moving spheres or media use neither the sweep nor the
-    // sphere-only walk)
+    // (scenes with moving spheres use neither the uniform pass nor the tree; media
+    // only the pass)
     const ray_ctx rc = (MEDIA || !SWEEP) && !SPH && (P.motion | P.media) && valid
                            ? make_ray_ctx(P, item_in_entry(P, ent, __float_as_uint(a.w)), depth)
                            : ray_ctx{0.0f, 0u, 0u, 0u, 0u, 0u};
@@ -1063,7 +1063,7 @@ template <bool SWEEP, bool MULTI, bool SPH, bool GUIDED>
 __global__ void __launch_bounds__(256) k_tail(scene_view S, const tpt_slot *__restrict__ slots,
                                               const tpt_entry *__restrict__ entries, render_params P,
                                               render_state Q, uint32_t parity) {
-  static_assert(!(SWEEP && MULTI), "the wave-uniform sweep needs one scene");
+  static_assert(!(SWEEP && MULTI), "the uniform pass needs one scene");
   static_assert(SWEEP != SPH, "small scenes or sphere-only ones");
   S.slots = slots;
   S.entries = entries;
@@ -1103,7 +1103,7 @@ __global__ void __launch_bounds__(256) k_tail(scene_view S, const tpt_slot *__re
       if (taken == left) chunk += stride, used = 0;
       dead = __ballot(!live);
     }
-    // wave-uniform: the sweep needs every lane of the wave
+    // wave-uniform: the walks need every lane of the wave
     if (__ballot(live) == 0ull) break;
     {
       const item_ctx c = live ? item_in_entry(P, MULTI ? p.ent : 0u, p.item) : item_ctx{0u, 0u, 0u, 0u};

@@ -182,7 +182,7 @@ struct tpt_scene {
   uint32_t n_slots = 0, n_segments = 0, n_lights = 0;
   // the pool's scenes
   std::vector<scene_dev> scn;
-  std::vector<uint8_t> sweep;     // per scene: wave-uniform traversal (small scenes)
+  std::vector<uint8_t> sweep;     // per scene: takes the uniform pass (small scenes)
   std::vector<uint8_t> sph;       // per scene: every leaf is a sphere
   std::vector<uint8_t> simple;    // per scene: constant textures, no light or one xz_rect light
   std::vector<uint8_t> plain;     // per scene: as simple, but media are allowed
@@ -1105,7 +1105,7 @@ struct bounce_launch {
   bool sph;     // every leaf of the launch's scenes is a sphere
   bool simple;  // their textures are constant and their light root absent or one xz_rect
   bool plain;   // as simple, but media are allowed
-  bool tail;    // passes end with a fused k_tail launch (simple scenes, sweep or sphere-only walk)
+  bool tail;    // passes end with a fused k_tail launch (simple scenes, uniform pass or sphere-only)
   bool count;   // TPT_RENDER_COUNT_OPS: the counting variant of k_trace, no fused tail
 };
 
