@@ -1119,13 +1119,8 @@ void launch_tail(const bounce_launch &B, hipStream_t st, uint32_t parity, uint32
     else
       hipLaunchKernelGGL((k_tail<true, false, false, false>), g, b, 0, st, B.S, B.S.slots, B.S.entries, B.P, B.Q,
                          parity);
-  } else if (B.multi) {
-    if (B.guided)
-      hipLaunchKernelGGL((k_tail<false, true, true, true>), g, b, 0, st, B.S, B.S.slots, B.S.entries, B.P, B.Q,
-                         parity);
-    else
-      hipLaunchKernelGGL((k_tail<false, true, true, false>), g, b, 0, st, B.S, B.S.slots, B.S.entries, B.P, B.Q,
-                         parity);
+  } else if (B.multi) {  // (guided: several plain jobs take k_paths)
+    hipLaunchKernelGGL((k_tail<false, true, true, true>), g, b, 0, st, B.S, B.S.slots, B.S.entries, B.P, B.Q, parity);
   } else {
     if (B.guided)
       hipLaunchKernelGGL((k_tail<false, false, true, true>), g, b, 0, st, B.S, B.S.slots, B.S.entries, B.P, B.Q,
