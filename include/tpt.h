@@ -455,7 +455,10 @@ int tpt_render_jobs(tpt_scene *scene, const tpt_job *jobs, uint32_t n_jobs, cons
  * without graph replay, then grid sizes of 16 and 32 blocks per CU at the best
  * capacity, then graph replay of 8 iterations at the best of those.  Writes
  * the fastest settings into *best (its flags, guiding and guide_vertices are
- * kept).  *best_ms: that calibration's wall time. */
+ * kept; TPT_RENDER_NO_TAIL and TPT_RENDER_COUNT_OPS hold for the calibration
+ * too).  *best_ms: that calibration's wall time.  Plain jobs without these flags
+ * run the same under every setting (see TPT_RENDER_NO_TAIL): one calibration is
+ * timed, and *best takes the largest capacity, 64 blocks per CU and no graph. */
 int tpt_autotune(tpt_scene *scene, const tpt_job *jobs, uint32_t n_jobs, tpt_guide *guide, uint32_t calib_spp,
                  tpt_launch *best, float *best_ms);
 

@@ -2141,7 +2141,8 @@ int tpt_autotune(tpt_scene *s, const tpt_job *jobs, uint32_t n_jobs, tpt_guide *
     cj[j].d_sumsq = nullptr;
   }
   tpt_launch base = *best;
-  base.flags = 0;
+  // the flags that choose the render's route stay: what is timed is what will run
+  base.flags &= TPT_RENDER_NO_TAIL | TPT_RENDER_COUNT_OPS;
   base.guiding = 0;  // calibration renders do not record training rows
   float best_t = 3.0e38f;
   tpt_launch pick = base;
@@ -2163,11 +2164,14 @@ int tpt_autotune(tpt_scene *s, const tpt_job *jobs, uint32_t n_jobs, tpt_guide *
     }
     return TPT_OK;
   };
-  for (uint32_t k = 0; k < n_caps && rc == TPT_OK; ++k) rc = trial(caps[k], 64, 0);
+  // Plain renders keep no queues (k_paths), so every setting renders alike: one
+  // calibration gives the time, the largest capacity stands for all.
+  const bool one = !guide && base.flags == 0;
+  for (uint32_t k = one ? n_caps - 1 : 0; k < n_caps && rc == TPT_OK; ++k) rc = trial(caps[k], 64, 0);
   const uint32_t cap_pick = pick.queue_capacity;
   for (uint32_t b : {16u, 32u})
-    if (rc == TPT_OK) rc = trial(cap_pick, b, 0);
-  if (rc == TPT_OK) rc = trial(cap_pick, pick.blocks_per_cu, 8);
+    if (rc == TPT_OK && !one) rc = trial(cap_pick, b, 0);
+  if (rc == TPT_OK && !one) rc = trial(cap_pick, pick.blocks_per_cu, 8);
   release();
   if (rc != TPT_OK) return rc;
   pick.flags = best->flags;
