@@ -21,20 +21,14 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBS = 8000.0
-# Algorithmic HBM bytes per closest-hit segment, split by kernel: k_trace
-# reads the ray (24 B) and its queue entry (4 B) and writes the hit (t, slot,
-# entry, material: 16 B) and one material-queue entry (4 B); k_shade reads the
-# hit (16 B), the ray (24 B), path state (throughput 12, radiance 12, pixel,
-# sample, depth 12 B) and its queue entry (4 B), writes the next ray (24 B),
-# throughput and radiance (24 B) and the next queue entry (4 B); per finished
-# path it adds the accumulator read-modify-write (24 B).
-TRACE_BYTES_PER_SEGMENT = 48
-SHADE_BYTES_PER_SEGMENT = 116
-ACCUM_BYTES_PER_PATH = 24
-# Counted VALU work of the closest-hit walk, lane-operations per operation:
-# a slab test 18, a sphere test 30 (its FP64 roots apart), a rect test 14, a
-# wrapper chain (translate + rotate_y) 25.  Peak: the non-packed FP32 lane
-# rate, 256 CUs x 4 SIMDs x 16 lanes x 2.4 GHz.
+# A plain frame renders in path launches (k_paths): a path stays in registers, so
+# all it cannot do without in HBM is its result, 12 bytes written once.
+PATH_BYTES = 12
+# Counted VALU work of the reference's own walk over the scene (what a counting
+# render of the bounce loop visits; the timed launches test less, or more, by walks
+# of their own), lane-operations per operation: a slab test 18, a sphere test 30
+# (its FP64 roots apart), a rect test 14, a wrapper chain (translate + rotate_y) 25.
+# Peak: the non-packed FP32 lane rate, 256 CUs x 4 SIMDs x 16 lanes x 2.4 GHz.
 LANE_OPS = {"box_tests": 18, "sphere_tests": 30, "rect_tests": 14, "xforms": 25}
 VALU_PEAK_TLANE_OPS = 39.32
 COUNT_SPP = 64
@@ -401,7 +395,7 @@ TRAIN_FLOP_PER_ROW = 80640  # forward 26,880 + backward data and weights (2x)
 
 def guide_train(tpt, torch, args):
     """One step = one Adam step of the guiding network on 2^18 training rows
-    (fused forward/backward, reduction, Adam, tile packing), on synthetic
+    (fused forward/backward, then reduction, Adam and tile packing), on synthetic
     rows of the recorded layout, cycling through 2^20 of them."""
     rng = np.random.default_rng(7)
     n = 1 << 20
@@ -440,11 +434,50 @@ def guide_train(tpt, torch, args):
         "data": "synthetic training rows (uniform positions, random unit vectors, exponential contributions)",
         "config": {"workload": "guide_train: 42->3x64->40 vMF-mixture network, batch 2^18 rows, 2^20 rows cycled",
                    "batch": batch},
-        "roofline": {"bound": "mfma", "kernel": "k_guide_train + reduce + Adam + pack", "achieved": round(tflops, 2),
+        "roofline": {"bound": "mfma", "kernel": "k_guide_train + k_guide_finish", "achieved": round(tflops, 2),
                      "peak": MFMA_BF16_PEAK_TFLOPS, "unit": "TFLOP/s", "frac": round(tflops / MFMA_BF16_PEAK_TFLOPS, 5),
                      "traffic": None, "flop_per_row": TRAIN_FLOP_PER_ROW},
         "detail": {"last_loss": round(loss, 5)},
     }
+
+
+def timed_kernel(totals):
+    """The kernel that a profiled plain render spends its time in, from its
+    statistics: (name, milliseconds, launches).  Every plain render runs in path
+    launches; those of the scenes that the fused tail takes are counted in tail_*,
+    the others' in trace_*."""
+    assert totals["shade_launches"] == 0, "a plain render in bounce launches"
+    return "k_paths", totals["tail_ms"] + totals["trace_ms"], totals["tail_launches"] + totals["trace_launches"]
+
+
+def profile_of(scene, width, what, kernel):
+    """The committed counter profile of this kernel on this frame, or None."""
+    path = os.path.join(ROOT, "profiles", f"{scene}_{width}_plain_{what}.json")
+    if not os.path.exists(path):
+        return None
+    with open(path) as f:
+        return json.load(f)["kernels"].get(kernel)
+
+
+def roofline(scene, width, totals):
+    """What bounds the timed kernel is the issue of vector instructions: the rate is
+    the lane-operations it executes, from the counters of a committed profile times
+    this run's segments, over its time.  Beside it its HBM traffic."""
+    name, ms, launches = timed_kernel(totals)
+    per = max(launches, 1)
+    kbytes = PATH_BYTES * totals["paths"]
+    gbs = kbytes / (ms / 1e3) / 1e9 if ms > 0 else 0.0
+    vk, tk = profile_of(scene, width, "valu", name), profile_of(scene, width, "traffic", name)
+    ops = vk["executed_lane_ops_per_segment"] if vk else None
+    ach = ops * totals["segments"] / (ms / 1e3) / 1e12 if vk and ms > 0 else None
+    return {"bound": "valu", "kernel": name, "achieved": round(ach, 3) if ach is not None else None,
+            "peak": VALU_PEAK_TLANE_OPS, "unit": "Tlane-ops/s",
+            "frac": round(ach / VALU_PEAK_TLANE_OPS, 4) if ach is not None else None,
+            "traffic": round(tk["hbm_bytes_per_path"] * totals["paths"] / per) if tk else None,
+            "avg_launch_ms": round(ms / per, 4), "bytes_per_launch": round(kbytes / per),
+            "executed_lane_ops_per_segment": ops,
+            "hbm": {"achieved": round(gbs, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
+                    "frac": round(gbs / HBM_PEAK_GBS, 5)}}
 
 
 def guided(tpt, torch, args):
@@ -549,28 +582,6 @@ def main():
     value = samples / dt / 1e6
     segs = totals["segments"]
     paths = totals["paths"]
-    # the bounce-loop kernels' share: what the fused launches trace and shade is timed apart
-    loop_segs = segs - totals["tail_segments"]
-    trace_bytes = TRACE_BYTES_PER_SEGMENT * loop_segs
-    shade_bytes = SHADE_BYTES_PER_SEGMENT * loop_segs + ACCUM_BYTES_PER_PATH * paths
-    if totals["tail_ms"] >= max(totals["trace_ms"], totals["shade_ms"]):
-        # the whole render in fused path launches: 12 B written per sample, and
-        # read and summed once per pass
-        kname, kbytes, kms, nl = "k_paths", 12 * paths, totals["tail_ms"], totals["tail_launches"]
-    elif totals["trace_ms"] >= totals["shade_ms"]:
-        kname, kbytes, kms, nl = "k_trace", trace_bytes, totals["trace_ms"], totals["trace_launches"]
-    else:
-        kname, kbytes, kms, nl = "k_shade", shade_bytes, totals["shade_ms"], totals["shade_launches"]
-    achieved = kbytes / (kms / 1e3) / 1e9 if kms > 0 else 0.0
-    # measured HBM bytes per segment of this kernel (two rocprofv3 counter passes,
-    # scaled by a known-size copy): profiles/cornell555_1200_plain_traffic.md
-    traffic = None
-    tfile = os.path.join(ROOT, "profiles", f"{args.scene}_{W}_plain_traffic.json")
-    if os.path.exists(tfile):
-        with open(tfile) as f:
-            tk = json.load(f)["kernels"].get(kname)
-        if tk:
-            traffic = round(tk["hbm_bytes_per_segment"] * loop_segs / max(nl, 1))
     out = {
         "metric": ("Msamples/s (plain GPU tracer, Cornell 1200^2, 2048 spp, depth 50)" if args.scene == "cornell555"
                    else f"Msamples/s (plain GPU tracer, {args.scene} {W}x{H}, {spp} spp, depth {depth})"),
@@ -588,54 +599,27 @@ def main():
                  if args.scene == "cornell555" else f"synthetic (procedural scene {args.scene}, built through the scene API)"),
         "config": {"workload": f"{args.scene} {W}x{H}, {spp} spp, max depth {depth}, plain estimator",
                    "width": W, "height": H, "spp": spp, "max_depth": depth},
-        "roofline": {"bound": "hbm", "kernel": kname, "achieved": round(achieved, 2), "peak": HBM_PEAK_GBS,
-                     "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 5), "traffic": traffic,
-                     "avg_launch_ms": round(kms / max(nl, 1), 4),
-                     "bytes_per_launch": round(kbytes / max(nl, 1))},
+        "roofline": roofline(args.scene, W, totals),
         "detail": {"Mrays_per_s": round(segs / dt / 1e6, 2), "segments_per_path": round(segs / max(paths, 1), 3),
                    "light_queries": totals["light_queries"], "nodes_per_segment":
                        round(totals["nodes_visited"] / max(segs, 1), 2), "trace_ms": round(totals["trace_ms"], 1),
                    "shade_ms": round(totals["shade_ms"], 1), "nan_samples": totals["nan_samples"],
                    "tail_segments": totals["tail_segments"], "tail_ms": round(totals["tail_ms"], 1),
-                   "segments": segs, "tail_launches": totals["tail_launches"],
-                   # BVH / primitive bytes the walk requests: one 32-byte slot per visit (boxes and
-                   # leaves alike), served from L1/L2 (the Cornell box's slots are 576 bytes)
-                   "bvh_slot_bytes_per_segment": round(32 * totals["nodes_visited"] / max(segs, 1), 1),
-                   # (over the trace launches and the fused tail launches, which also walk)
-                   "bvh_requested_GBps": round(32 * totals["nodes_visited"] /
-                                               ((totals["trace_ms"] + totals["tail_ms"]) / 1e3) / 1e9, 1)
-                   if totals["trace_ms"] else None},
+                   "segments": segs, "tail_launches": totals["tail_launches"]},
     }
-    # counted VALU work of the walk: one untimed render of the same frame at
-    # COUNT_SPP samples per pixel with the counting trace kernel (every segment
-    # through k_trace), per segment, times the timed run's bounce-loop segments
+    # the reference's own walk, counted: one untimed render of the same frame at
+    # COUNT_SPP samples per pixel with the counting trace kernel of the bounce loop
     _, _, cst = sc.render(spp=COUNT_SPP, seed=4242, sum_buf=sum_buf, sumsq_buf=sq_buf, count_ops=True)
-    csegs = max(cst["segments"], 1)
-    per_seg = {k: cst[k] / csegs for k in LANE_OPS}
-    lane_ops_per_seg = sum(LANE_OPS[k] * v for k, v in per_seg.items())
-    valu = {"bound": "valu", "kernel": "k_trace", "unit": "Tlane-ops/s", "peak": VALU_PEAK_TLANE_OPS,
-            "counted_lane_ops_per_segment": round(lane_ops_per_seg, 2),
-            "ops_per_segment": {k: round(v, 4) for k, v in per_seg.items()},
-            "weights": LANE_OPS}
-    if totals["trace_ms"] > 0:
-        ach = lane_ops_per_seg * loop_segs / (totals["trace_ms"] / 1e3) / 1e12
-        valu.update(achieved=round(ach, 3), frac=round(ach / VALU_PEAK_TLANE_OPS, 4))
-    # executed VALU lane-operations per segment of the same kernel, from the
-    # gfx950 counters (SQ_INSTS_VALU x active lanes) of a committed profile
-    vfile = os.path.join(ROOT, "profiles", f"{args.scene}_{W}_plain_valu.json")
-    if os.path.exists(vfile) and totals["trace_ms"] > 0:
-        with open(vfile) as f:
-            vk = json.load(f)["kernels"].get("k_trace")
-        if vk:
-            ex = vk["executed_lane_ops_per_segment"] * loop_segs / (totals["trace_ms"] / 1e3) / 1e12
-            valu.update(executed_lane_ops_per_segment=vk["executed_lane_ops_per_segment"],
-                        executed=round(ex, 3), executed_frac=round(ex / VALU_PEAK_TLANE_OPS, 4),
-                        executed_source=f"profiles/{args.scene}_{W}_plain_valu.json")
-    out["roofline"]["valu"] = valu
+    per_seg = {k: cst[k] / max(cst["segments"], 1) for k in LANE_OPS}
+    out["detail"]["reference_walk"] = {
+        "ops_per_segment": {k: round(v, 4) for k, v in per_seg.items()}, "weights": LANE_OPS,
+        "lane_ops_per_segment": round(sum(LANE_OPS[k] * v for k, v in per_seg.items()), 2)}
     cpu_extra = None
     if not args.no_cpu:
         out["cpu_baseline"], cpu_extra = cpu_baseline(args.scene, W, H, args.cpu_spp, args.cpu_every, depth)
-        out["detail"]["x_host_cpu"] = round(value / out["cpu_baseline"]["value"], 1)
+        # (of the CPU port where the reference's own build is not here: cpu_baseline's kind)
+        port = out["cpu_baseline"]["kind"] == "port"
+        out["detail"]["x_host_cpu_port" if port else "x_host_cpu"] = round(value / out["cpu_baseline"]["value"], 1)
     if not args.no_rmse:
         del sum_buf, sq_buf
         out["time_to_rmse"] = time_to_rmse(tpt, torch, sc, args.ref_spp, cpu_extra)
