@@ -86,6 +86,9 @@ enum tpt_status {
  *          f[1] = entry count (as uint32 bits).  A leaf made of wrappers
  *          (translate / rotate_y / flip_normal), box and hitable_list around
  *          primitives; evaluated with the list's shrinking t_max.
+ * Where every box holds the boxes below it and the links describe one tree per
+ * segment (flattened hitables always do), faster walks with the same results
+ * are used; other arrays are walked box by box.
  * Leaf ids number primitive occurrences in depth-first order of the object
  * graph (bvh left before right, lists in order, an n==1 node's duplicate child
  * counted once); tpt_trace_closest reports them. */
@@ -365,8 +368,10 @@ typedef struct tpt_render_stats {
   uint64_t light_queries;  /* light-pdf intersections */
   uint64_t nan_samples;    /* samples with a NaN channel zeroed by de_nan */
   double kernel_ms;        /* GPU time of the whole pass (events around it) */
-  uint64_t nodes_visited;  /* pre-order slots visited by closest-hit queries (small scenes, which are traced
-                              without a walk: the primitives, a closed box of six rects counting once) */
+  uint64_t nodes_visited;  /* pre-order slots visited by closest-hit queries (sphere-only scenes: nodes of a tree of
+                              their own; scenes of at most 64 slots, which are traced without a walk: the primitives,
+                              a closed box of six rects counting once, but for path launches of many spheres in
+                              small boxes, which walk) */
   double trace_ms, shade_ms;          /* with TPT_RENDER_PROFILE */
   uint64_t trace_launches, shade_launches;
   /* the fused launches of the scenes that k_tail takes (k_tail and, for plain
