@@ -51,11 +51,12 @@ typedef const TPT_SCALAR flat_group *flat_group_ptr;
 
 // 1/d correctly rounded for 2^-100 <= |d| <= 2^100: the hardware reciprocal
 // (1 ulp) and one fused Newton step (Markstein 1990; checked against the IEEE
-// division for all 2^23 mantissas): 3 instructions instead of 11.
-__device__ __forceinline__ float recip_rn(float d) {
-  const float y = __builtin_amdgcn_rcpf(d);
+// division for all 2^23 mantissas): 3 instructions instead of 11.  (Not a number
+// where the hardware's y is infinite.)
+__device__ __forceinline__ float recip_step(float d, float y) {
   return __builtin_fmaf(__builtin_fmaf(-d, y, 1.0f), y, y);
 }
+__device__ __forceinline__ float recip_rn(float d) { return recip_step(d, __builtin_amdgcn_rcpf(d)); }
 
 __device__ __forceinline__ float max3f(float a, float b, float c) { return fmaxf(fmaxf(a, b), c); }
 
@@ -285,12 +286,14 @@ template <bool TIES, bool MEDIA>
 __device__ __forceinline__ bool flat_world(const scene_view &S, v3 o, v3 d, const ray_ctx &rc, float tmin, float tmax, bool live,
                                            hit_t *out, uint32_t *nodes, bool *slow, uint32_t *leaf, hit_geo *geo) {
   const bool zx = d.x == 0.0f, zy = d.y == 0.0f, zz = d.z == 0.0f;
-  const v3 inv{zx ? __builtin_amdgcn_rcpf(d.x) : recip_rn(d.x), zy ? __builtin_amdgcn_rcpf(d.y) : recip_rn(d.y),
-               zz ? __builtin_amdgcn_rcpf(d.z) : recip_rn(d.z)};
+  const v3 y{__builtin_amdgcn_rcpf(d.x), __builtin_amdgcn_rcpf(d.y), __builtin_amdgcn_rcpf(d.z)};
+  const v3 inv{zx ? y.x : recip_step(d.x, y.x), zy ? y.y : recip_step(d.y, y.y), zz ? y.z : recip_step(d.z, y.z)};
   const float mo = max3f(fabsf(o.x), fabsf(o.y), fabsf(o.z));
   const float m = (1.5f * mo + S.flat_mag) * 0x1p-19f;
-  const float my = zy ? 0.0f : fabsf(inv.y);
-  const float mi = max3f(zx ? 0.0f : fabsf(inv.x), my, zz ? 0.0f : fabsf(inv.z));
+  // (of the hardware's reciprocals, 1 ulp off: a denormal's is infinite, and what
+  // the step makes of it is no number, which a maximum would drop)
+  const float my = zy ? 0.0f : fabsf(y.y);
+  const float mi = max3f(zx ? 0.0f : fabsf(y.x), my, zz ? 0.0f : fabsf(y.z));
   const float big = fmaxf(max3f(fabsf(d.x), fabsf(d.y), fabsf(d.z)), fmaxf(mi, mo));
   // (fmaxf drops NaNs: they are looked for in the sum)
   const float sum = ((o.x + o.y) + o.z) + ((d.x + d.y) + d.z);
