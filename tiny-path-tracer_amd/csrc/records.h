@@ -25,7 +25,7 @@ struct flat_win {
   float f[5];                 // primitive parameters as in tpt_slot
   uint32_t slot, entry, mat;  // as in hit_t
   float box[6];               // the innermost box around it
-  uint32_t boxed;             // 0: there is none, or it is passed whenever the winner is certain
+  uint32_t boxed;             // 0: there is none; 1: it is passed whenever the winner is certain; 2: it is to be tested
   uint32_t xform, kind, leaf;  // wrapper chain or ~0u; TPT_SLOT_RECT, _SPHERE or _MEDIUM; leaf id
   uint32_t order, pad;         // its place in the order of segments, slots and entries
 };

@@ -566,6 +566,7 @@ flat_range flat_records(const tpt_flat_scene &f, uint32_t sb, uint32_t eb, uint3
                  uint32_t leaf, uint32_t parent) {
     flat_item it{};
     flat_win &q = it.win;
+    bool inside = false;
     const int nf = kind == TPT_SLOT_RECT ? 5 : (kind == TPT_SLOT_SPHERE ? 4 : 0);  // (a medium's hold indexes)
     for (int k = 0; k < nf; ++k) q.f[k] = w[k], ok = ok && std::fabs(w[k]) < 1e18f;
     flat_scan &p = it.scan;
@@ -577,11 +578,11 @@ flat_range flat_records(const tpt_flat_scene &f, uint32_t sb, uint32_t eb, uint3
       for (int k = 0; k < 5; ++k) mag = std::fmax(mag, std::fabs(w[k]));
       ok = ok && it.cls < 3;
       if (ok && parent != kNone && xform == 0xFFFFFFFFu) {
-        // inside its parent box: the box needs no test of its own
+        // inside its parent box: a certain hit needs no test of the box
         const float *b = f.slots[parent].f;
         const uint32_t a = it.cls, u = a == 0 ? 1 : 0, v = a == 2 ? 1 : 2;
         if (b[a] <= w[0] && w[0] <= b[3 + a] && b[u] <= w[1] && w[2] <= b[3 + u] && b[v] <= w[3] && w[4] <= b[3 + v])
-          parent = kNone;
+          inside = true;
       }
     } else if (kind == TPT_SLOT_SPHERE) {
       it.cls = FLAT_SPHERE;
@@ -599,7 +600,7 @@ flat_range flat_records(const tpt_flat_scene &f, uint32_t sb, uint32_t eb, uint3
     q.slot = slot + sb, q.entry = entry == kNone ? kNone : entry + eb, q.kind = kind;
     q.leaf = leaf;
     q.order = static_cast<uint32_t>(items.size());
-    q.boxed = parent != kNone;
+    q.boxed = parent == kNone ? 0u : (inside ? 1u : 2u);
     if (q.boxed) std::memcpy(q.box, f.slots[parent].f, sizeof(q.box));
     q.mat = rebase_word(word, mb);
     q.xform = xform == 0xFFFFFFFFu ? kNone : xform + xb;

@@ -180,11 +180,12 @@ __device__ __forceinline__ bool flat_in_plane(flat_scan_ptr p, uint32_t n, uint3
 }
 
 // Record `id` exactly: its leaf test with the reference's arithmetic (a
-// sphere's time t is exact already) and its parent's box.  *order: its place in
-// the reference's order.
+// sphere's time t is exact already) and its parent's box.  sure: it is inside its
+// bounds by the margin.  *order: its place in the reference's order.  False where
+// the leaf is missed, or its box is not certainly passed (entered after the hit).
 __device__ __forceinline__ bool flat_exact(const scene_view &S, uint32_t id, float t, v3 o, v3 d, v3 inv, float tmin,
-                                           float tmax, bool lost, hit_t *h, uint32_t *leaf, uint32_t *order,
-                                           bool *rect, hit_geo *geo) {
+                                           float tmax, bool lost, bool sure, hit_t *h, uint32_t *leaf,
+                                           uint32_t *order, bool *rect, hit_geo *geo) {
   const float4 *q = reinterpret_cast<const float4 *>(S.fwins + id);
   const float4 q0 = q[0], q1 = q[1], q2 = q[2], q3 = q[3], q4 = q[4];
   const uint32_t word = __float_as_uint(q1.w), xf = __float_as_uint(q3.w);
@@ -199,7 +200,8 @@ __device__ __forceinline__ bool flat_exact(const scene_view &S, uint32_t id, flo
     geo->kind = __float_as_uint(q4.x), geo->word = word, geo->xf = xf;
     geo->lo = lo, geo->ld = ld;
   }
-  if (__float_as_uint(q3.z) && !lost) {
+  const uint32_t boxed = __float_as_uint(q3.z);
+  if (boxed > (sure ? 1u : 0u) && !lost) {
     const slot_t b{{q2.x, q2.y, q2.z, q2.w, q3.x, q3.y}, 0u, 0u};
     got = got && slab_nn(b, o, inv, tmin, t + fabsf(t) * 0x1p-19f);
   }
@@ -279,9 +281,9 @@ __device__ __forceinline__ void flat_medium(const scene_view &S, flat_scan_ptr p
 // MEDIA: the scene holds constant_media (all bounded by closed boxes).
 //
 // TIES: two rects at the same time (the bottom of a box that stands on the
-// floor, seen from inside it) are both evaluated and the reference's rule
-// applied, the smaller t, at equal t the later one.  Paths do not get there;
-// for a caller's own rays it keeps such lanes off the exact walk.
+// floor, seen from inside it) are both evaluated, each with its box, and the
+// reference's rule applied, the smaller t, at equal t the later one.  Paths do
+// not get there; for a caller's own rays it keeps such lanes off the exact walk.
 template <bool TIES, bool MEDIA>
 __device__ __forceinline__ bool flat_world(const scene_view &S, v3 o, v3 d, const ray_ctx &rc, float tmin, float tmax, bool live,
                                            hit_t *out, uint32_t *nodes, bool *slow, uint32_t *leaf, hit_geo *geo) {
@@ -361,14 +363,16 @@ __device__ __forceinline__ bool flat_world(const scene_view &S, v3 o, v3 d, cons
   if (live && have && !amb) {
     uint32_t order, id;
     bool rect;
-    got = flat_exact(S, best.id, best.t1, o, d, inv, tmin, tmax, lost, out, &id, &order, &rect, geo);
+    got = flat_exact(S, best.id, best.t1, o, d, inv, tmin, tmax, lost, true, out, &id, &order, &rect, geo);
     if (TIES && !lost && !(best.t2 > best.t1 + fabsf(best.t1) * 0x1p-18f)) {
       hit_t h;
       uint32_t order2, id2;
       bool rect2;
-      const bool got2 = flat_exact(S, best.id2, best.t2, o, d, inv, tmin, tmax, false, &h, &id2, &order2, &rect2, nullptr);
+      // (nothing is known of how far inside its bounds the second is; if it is missed
+      // after all, the recursion decides)
+      got &= flat_exact(S, best.id2, best.t2, o, d, inv, tmin, tmax, false, false, &h, &id2, &order2, &rect2, nullptr);
       got = got && rect && rect2;
-      if (got && got2 && (h.t < out->t || (h.t == out->t && order2 > order))) *out = h, id = id2;
+      if (got && (h.t < out->t || (h.t == out->t && order2 > order))) *out = h, id = id2;
     }
     amb = !got;
     if (leaf) *leaf = id;
